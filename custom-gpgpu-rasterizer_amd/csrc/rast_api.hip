@@ -640,7 +640,7 @@ static int ensure_frame_storage(rast_renderer *r, uint32_t ntiles)
     HIP_TRY(grow(r, r->queue, (size_t)r->queue_cap * 4, &synced));
     HIP_TRY(grow(r, r->pool, (size_t)r->pool_cap * 4, &synced));
     HIP_TRY(grow(r, r->big, (size_t)r->big_cap * 4, &synced));
-    HIP_TRY(grow(r, r->bigp, (size_t)r->big_cap * 16, &synced));
+    HIP_TRY(grow(r, r->bigp, (size_t)r->big_cap * 32, &synced));
     return RAST_OK;
 }
 

@@ -128,7 +128,7 @@ struct alignas(16) JobDesc {  // 16-byte multiple: staged in 16-byte words
     uint32_t mesh0;              // first entry of the job in the mesh table
     uint32_t single;             // single-pass binning (capacities known before setup)
     uint32_t learned;            // capacities from the MLP (else previous count * margin + slack)
-    uint32_t small_limit;        // tile-clipped pixel count from which resolve goes pixel-parallel
+    uint32_t small_limit;        // tile-clipped pixel count from which resolve goes pixel-parallel (at least half a tile)
     float margin;
     uint32_t slack;
     uint32_t queue_cap, pool_cap, big_cap, ovf_cap;
@@ -159,8 +159,9 @@ struct alignas(16) JobDesc {  // 16-byte multiple: staged in 16-byte words
     uint2 *ovf;                  // single pass: (tile, id) entries beyond capacity
     uint32_t *survivors;
     uint32_t *big;
-    // per screen-list slot: the triangle's depth plane over its pixel range,
-    // formed once by the setup pass (screen_plane); read by every resolve tile
+    // per screen-list slot, formed once by the setup pass and read by every
+    // resolve tile: the triangle's depth plane over its pixel range
+    // (screen_plane), then bbox lo, bbox hi, ID
     float4 *big_plane;
     FrameCounters *counters;     // num_alive stays 0 here: see alive_part
     FrameCounters *host_counters;  // pinned host copy, written at the end of the launch

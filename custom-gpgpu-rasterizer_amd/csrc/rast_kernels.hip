@@ -69,6 +69,36 @@ __device__ __forceinline__ uint32_t wave_incl_sum(uint32_t v)
     return v;
 }
 
+// Largest / smallest of the lanes' values (all 64 active, no NaN; values at
+// least 0 for the maximum, at most 1 for the minimum), in every lane.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_f(float old, float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CTRL, ROWS, 0xf, false));
+}
+
+__device__ __forceinline__ float wave_max_f(float v)
+{
+    v = fmaxf(v, dpp_f<0x111, 0xf>(0.f, v));
+    v = fmaxf(v, dpp_f<0x112, 0xf>(0.f, v));
+    v = fmaxf(v, dpp_f<0x114, 0xf>(0.f, v));
+    v = fmaxf(v, dpp_f<0x118, 0xf>(0.f, v));
+    v = fmaxf(v, dpp_f<0x142, 0xa>(0.f, v));
+    v = fmaxf(v, dpp_f<0x143, 0xc>(0.f, v));
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
+__device__ __forceinline__ float wave_min_f(float v)
+{
+    v = fminf(v, dpp_f<0x111, 0xf>(1.f, v));
+    v = fminf(v, dpp_f<0x112, 0xf>(1.f, v));
+    v = fminf(v, dpp_f<0x114, 0xf>(1.f, v));
+    v = fminf(v, dpp_f<0x118, 0xf>(1.f, v));
+    v = fminf(v, dpp_f<0x142, 0xa>(1.f, v));
+    v = fminf(v, dpp_f<0x143, 0xc>(1.f, v));
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
 // Global-memory access through global-address-space pointers.  Pointers
 // read from the job and mesh tables are generic to the compiler, which would
 // emit flat loads, stores and atomics; those also count against the LDS /
@@ -353,7 +383,7 @@ __device__ __forceinline__ void edge_vectors(const MicroLds &t, float &ax, float
 
 // Item q of a triangle's pixel range [x0,x1) x [y0,y1), row-major, for
 // q < 1024 and a row width w = x1 - x0 <= 1024 (setup's micro triangles: q <
-// micro_limit; resolve's items: q < small_limit; both limits are at most
+// micro_limit; resolve's items: q < whole_limit; both limits are at most
 // 1024) with t.inv within 2^-23 of 1 / w, relative (the rounded quotient, or
 // the hardware reciprocal's 1 ulp).  (q + 0.5) / w lies at least 0.5 / w >=
 // 2^-11 from an integer, and fl(fl(q + 0.5) t.inv) is within 1.6 * 2^-23
@@ -1041,7 +1071,8 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
     if (is_big && bslot < J.big_cap) {
         TriLds bt;
         load_tri(trirec, gid, bt);
-        stg(J.big_plane + bslot, screen_plane(bt));
+        stg(J.big_plane + 2 * (size_t)bslot, screen_plane(bt));
+        stg(reinterpret_cast<uint4 *>(J.big_plane + 2 * (size_t)bslot + 1), make_uint4(bt.xr, bt.yr, gid, 0u));
     }
 }
 
@@ -1283,7 +1314,39 @@ __global__ __launch_bounds__(256) void k_fallback_fill(const JobDesc *__restrict
 // lo(p) > the pixel's depth and is out of range where lo(p) + w < 0.
 // x = +3e38: no pixel of the tile can take a fragment of t (outside an
 // edge, depth out of [0, 1], or behind every pixel).
-__device__ __forceinline__ float4 tile_bound(const TriLds &t, const float4 sp, int X0, int Y0, int T, float tmax)
+//
+// Two parts: plane_bound needs the list entry only (the stored plane and the
+// corner of the triangle's range); where it leaves the triangle standing,
+// coverage_bound reads the setup record.  Most tiles lie in front of all of a
+// scene's screen-list triangles and end with the first (with the record read
+// and all tests for every triangle in every tile, an 8K frame's resolve took
+// 311 us instead of 266, a 4K frame's 87 instead of 74, both with the tighter
+// item ranges).
+__device__ __forceinline__ float4 plane_bound(const float4 sp, uint32_t range_lo, int X0, int Y0, int T, float tmax)
+{
+    const float4 skip = make_float4(3.0e38f, 0.f, 0.f, 0.f);
+    const float4 none = make_float4(-1.0e30f, 0.f, 0.f, 1.0e30f);
+    if (!(sp.w < 0.2f)) return none;  // the triangle has no plane (+inf)
+    const float u = 1.0f / 16777216.0f;
+    const float dX = (float)(X0 - (int)(range_lo & 0xFFFFu)), dY = (float)(Y0 - (int)(range_lo >> 16));
+    const float px = sp.y * dX, py = sp.z * dY;
+    const float L0 = (sp.x + px) + py;
+    const float S = (fabsf(sp.x) + fabsf(px)) + fabsf(py);
+    const float Tm = (float)(T - 1);
+    const float span = (fabsf(sp.y) + fabsf(sp.z)) * Tm;
+    const float aL = fabsf(L0);
+    const float M = (sp.w + u * (4.02f * S + 12.0f * aL + 13.0f * span + 8.0f)) * 1.0001f + 1.0e-30f;
+    if (!(M < 0.25f)) return none;
+    // whole-tile tests at the tile's corners (L is affine)
+    const float Lmin = (L0 + fminf(sp.y, 0.f) * Tm) + fminf(sp.z, 0.f) * Tm;
+    const float Lmax = (L0 + fmaxf(sp.y, 0.f) * Tm) + fmaxf(sp.z, 0.f) * Tm;
+    if (Lmin - M > 1.0f || Lmax + M < 0.0f || Lmin - M > tmax) return skip;
+    return make_float4(L0 - M, sp.y, sp.z, 2.0f * M + 8.0f * u * (aL + span + 1.0f));
+}
+
+// plane_bound's bound pl of triangle t, with the tests of its setup record: skip where no
+// pixel of the tile is covered, and the constant bound where no plane applies.
+__device__ __forceinline__ float4 coverage_bound(const TriLds &t, const float4 pl, int X0, int Y0, int T, float tmax)
 {
     const float4 skip = make_float4(3.0e38f, 0.f, 0.f, 0.f);
     const float4 none = make_float4(-1.0e30f, 0.f, 0.f, 1.0e30f);
@@ -1302,24 +1365,7 @@ __device__ __forceinline__ float4 tile_bound(const TriLds &t, const float4 sp, i
         lo2 = fminf(lo2, w2); hi2 = fmaxf(hi2, w2);
     }
     if (hi0 < 0.f || hi1 < 0.f || hi2 < 0.f) return skip;
-    if (sp.w < 0.2f) {  // the triangle has a plane (+inf: none)
-        const float u = 1.0f / 16777216.0f;
-        const float dX = (float)(X0 - (int)(t.xr & 0xFFFFu)), dY = (float)(Y0 - (int)(t.xr >> 16));
-        const float px = sp.y * dX, py = sp.z * dY;
-        const float L0 = (sp.x + px) + py;
-        const float S = (fabsf(sp.x) + fabsf(px)) + fabsf(py);
-        const float Tm = (float)(T - 1);
-        const float span = (fabsf(sp.y) + fabsf(sp.z)) * Tm;
-        const float aL = fabsf(L0);
-        const float M = (sp.w + u * (4.02f * S + 12.0f * aL + 13.0f * span + 8.0f)) * 1.0001f + 1.0e-30f;
-        if (M < 0.25f) {
-            // whole-tile tests at the tile's corners (L is affine)
-            const float Lmin = (L0 + fminf(sp.y, 0.f) * Tm) + fminf(sp.z, 0.f) * Tm;
-            const float Lmax = (L0 + fmaxf(sp.y, 0.f) * Tm) + fmaxf(sp.z, 0.f) * Tm;
-            if (Lmin - M > 1.0f || Lmax + M < 0.0f || Lmin - M > tmax) return skip;
-            return make_float4(L0 - M, sp.y, sp.z, 2.0f * M + 8.0f * u * (aL + span + 1.0f));
-        }
-    }
+    if (pl.w < 1.0e29f) return pl;  // the plane's bound
     // no plane: the exact float depth range over the tile
     const float l0 = fmaxf(lo0, 0.f) / t.area, l1 = fmaxf(lo1, 0.f) / t.area, l2 = fmaxf(lo2, 0.f) / t.area;
     const float h0 = hi0 / t.area, h1 = hi1 / t.area, h2 = hi2 / t.area;
@@ -1331,7 +1377,7 @@ __device__ __forceinline__ float4 tile_bound(const TriLds &t, const float4 sp, i
     return zlo == zlo ? make_float4(fmaxf(zlo, -1.0e30f), 0.f, 0.f, 1.0e30f) : none;
 }
 
-// tile_bound's x for "no pixel of the tile": a plane's x stays below 5e5
+// A bound's x for "no pixel of the tile": a plane's x stays below 5e5
 // (its margin M < 0.25 bounds |x| by 0.25 / (8 u)), a constant bound below 1.
 constexpr float kSkipBound = 1.0e37f;
 
@@ -1349,7 +1395,7 @@ __device__ __forceinline__ float tile_max_depth(const uint64_t *best, uint32_t l
     float d = 0.f;
 #pragma unroll
     for (int q = 0; q < PPT; ++q) d = fmaxf(d, __uint_as_float((uint32_t)(best[q] >> 32)));
-    for (int o = 32; o > 0; o >>= 1) d = fmaxf(d, __shfl_xor(d, o));
+    d = wave_max_f(d);
     __syncthreads();  // the previous values are read
     if (lane == 0) wdmax[wave] = d;
     __syncthreads();
@@ -1380,7 +1426,7 @@ __device__ __forceinline__ void bitonic_sort(uint64_t *v, uint32_t P, uint32_t t
 // per tile, each lane owning PPT pixels.  The lane loads its pixels' keys
 // (micro triangles, already rasterized at setup) and resets them for the
 // next frame.  The tile's queued triangles (queue region + fallback pool
-// region) are rasterized in LDS: a triangle covering at least small_limit
+// region) are rasterized in LDS: a triangle covering at least whole_limit
 // pixels of the tile one pixel per lane, the others as one compacted item
 // list (prefix sum over their clipped pixel ranges, LDS atomic min).  The few
 // screen-list triangles are then tested by every lane on its own pixels, with
@@ -1406,7 +1452,6 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
     uint32_t *__restrict__ pool = J.pool;
     const uint32_t pool_cap = J.pool_cap;
     const uint2 *__restrict__ ovf = J.ovf;
-    const uint32_t *__restrict__ big = J.big;
     const float4 *__restrict__ big_plane = J.big_plane;
     const uint32_t big_cap = J.big_cap;
     FrameCounters *__restrict__ ctr = J.counters;
@@ -1415,8 +1460,14 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
     uint32_t *__restrict__ vis = J.vis;
     float *__restrict__ depth = J.depth;
     float *__restrict__ tile_min_depth = J.tile_min_depth;
-    const uint32_t small_limit = J.small_limit;
     constexpr int NPIX = T * T;
+    // A triangle tested at one pixel per lane costs the tile's 16 rounds of 64
+    // pixels, less the rows it misses (about 85 instructions each), whatever it
+    // covers; as items about 65 instructions per 64 pixels of its range plus
+    // 85 per 64 covered ones: the lines cross near half the tile, so smaller
+    // limits are raised to that (limit 16 on a 2561 x 1439 terrain: the kernel
+    // 128 us, its slowest tile's time; with this rule 46).
+    const uint32_t whole_limit = J.small_limit > (uint32_t)NPIX / 2u ? J.small_limit : (uint32_t)NPIX / 2u;
     constexpr int PPT = NPIX / NT;
     constexpr int NW = NT / 64;
     static_assert(NPIX % NT == 0, "tile pixels must be a multiple of the workgroup size");
@@ -1551,16 +1602,21 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
                 const uint32_t id = i < n_a ? ldg(list_a + i) : ldg(list_b + (i - n_a));
                 if (id < num_tris) {
                     load_tri(trirec, id, t);
+                    // the triangle's range, from the first pixel that can be
+                    // covered (as in the setup pass), within the tile
+                    const float mnx = fminf(fminf(t.sx0, t.sx1), t.sx2), mny = fminf(fminf(t.sy0, t.sy1), t.sy2);
+                    const float reach = edge_reach(fmaxf(fmaxf(t.sx0, t.sx1), t.sx2) - mnx,
+                                                   fmaxf(fmaxf(t.sy0, t.sy1), t.sy2) - mny, t.area);
                     const int bx0 = (int)(t.xr & 0xFFFFu), by0 = (int)(t.xr >> 16);
                     const int bx1 = (int)(t.yr & 0xFFFFu), by1 = (int)(t.yr >> 16);
-                    const int x0 = bx0 > X0 ? bx0 : X0, x1 = bx1 < X0 + T ? bx1 : X0 + T;
-                    const int y0 = by0 > Y0 ? by0 : Y0, y1 = by1 < Y0 + T ? by1 : Y0 + T;
+                    const int x0 = first_pixel(mnx, reach, bx0 > X0 ? bx0 : X0), x1 = bx1 < X0 + T ? bx1 : X0 + T;
+                    const int y0 = first_pixel(mny, reach, by0 > Y0 ? by0 : Y0), y1 = by1 < Y0 + T ? by1 : Y0 + T;
                     if (x0 < x1 && y0 < y1) {
                         t.xr = (uint32_t)x0 | ((uint32_t)x1 << 16);
                         t.yr = (uint32_t)y0 | ((uint32_t)y1 << 16);
                         area = (uint32_t)((x1 - x0) * (y1 - y0));
-                        if (area >= small_limit) { whole = true; area = 0; }
-                        t.inv = 1.0f / (float)(x1 - x0);
+                        if (area >= whole_limit) { whole = true; area = 0; }
+                        t.inv = __builtin_amdgcn_rcpf((float)(x1 - x0));
                     }
                 }
             }
@@ -1572,11 +1628,7 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
                 stage[tid] = m;
             }
             // block-wide exclusive scan of the item counts
-            uint32_t incl = area;
-            for (int o = 1; o < 64; o <<= 1) {
-                const uint32_t y = __shfl_up(incl, o);
-                if (lane >= (uint32_t)o) incl += y;
-            }
+            const uint32_t incl = wave_incl_sum(area);
             if (lane == 63) wred_u[wave] = incl;
             const uint64_t wm = __ballot(whole), hm = __ballot(area != 0);
             if (lane == 0) {
@@ -1636,11 +1688,7 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
                     __syncthreads();
                     if (wave == 0) {
                         const uint32_t c = lane < kOwnerWords ? (uint32_t)__popcll(omask[lane]) : 0u;
-                        uint32_t ci = c;
-                        for (int o = 1; o < 64; o <<= 1) {
-                            const uint32_t y = __shfl_up(ci, o);
-                            if (lane >= (uint32_t)o) ci += y;
-                        }
+                        const uint32_t ci = wave_incl_sum(c);
                         if (lane < kOwnerWords) ocum[lane] = rbase + ci - c;
                         if (lane == 63) otot = ci;
                     }
@@ -1675,16 +1723,16 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
                 __syncthreads();
 #pragma unroll
                 for (int q = 0; q < PPT; ++q) best[q] = key[(int)tid + q * NT];
-                // wave-uniform row range of this wave's pixels (PPT == 1)
-                const int wy0 = Y0 + (int)(wave * 64) / T;
-                const int wy1 = Y0 + ((int)(wave * 64) + 63) / T + 1;
                 for (uint32_t q2 = 0; q2 < nwhole; ++q2) {
                     const MicroLds &st = stage[wlist[q2]];
                     const int x0 = (int)(st.xr & 0xFFFFu), x1 = (int)(st.xr >> 16);
                     const int y0 = (int)(st.yr & 0xFFFFu), y1 = (int)(st.yr >> 16);
-                    if (PPT == 1 && (y1 <= wy0 || y0 >= wy1)) continue;
 #pragma unroll
                     for (int q = 0; q < PPT; ++q) {
+                        // the wave's pixels of this round are the rows [wy0, wy1)
+                        const int wy0 = Y0 + ((int)(wave * 64) + q * NT) / T;
+                        const int wy1 = Y0 + ((int)(wave * 64) + 63 + q * NT) / T + 1;
+                        if (y1 <= wy0 || y0 >= wy1) continue;
                         const int px = pxs[q], py = pys[q];
                         if (px >= x0 && px < x1 && py >= y0 && py < y1) {
                             float z;
@@ -1735,8 +1783,7 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
 #pragma unroll
             for (int q = 0; q < PPT; ++q)
                 if (inside[q]) d = fmaxf(d, __uint_as_float((uint32_t)(best[q] >> 32)));
-            for (int o = 32; o > 0; o >>= 1) d = fmaxf(d, __shfl_xor(d, o));
-            return d;
+            return wave_max_f(d);
         };
         auto wave_floor = [](const float4 &pl) {
             const float lmin = pl.x + fminf(pl.y, 0.f) * (float)(T - 1) + fminf(pl.z, 0.f) * (float)(T - 1);
@@ -1774,6 +1821,22 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
             wmax = wave_max_depth();
             return true;
         };
+        // entry i's bound over the tile against the depth dmax (x > kSkipBound: not run)
+        auto list_bound = [&](uint32_t i, float dmax, uint32_t &id) {
+            const float4 sp = ldg(big_plane + 2 * (size_t)i);
+            const uint4 e = ldg(reinterpret_cast<const uint4 *>(big_plane + 2 * (size_t)i + 1));
+            id = e.z;
+            float4 pl = make_float4(3.0e38f, 0.f, 0.f, 0.f);
+            const int x0 = (int)(e.x & 0xFFFFu), y0 = (int)(e.x >> 16), x1 = (int)(e.y & 0xFFFFu), y1 = (int)(e.y >> 16);
+            if (id < num_tris && x1 > X0 && x0 < X0 + T && y1 > Y0 && y0 < Y0 + T)
+                pl = plane_bound(sp, e.x, X0, Y0, T, dmax);
+            if (!(pl.x > kSkipBound)) {
+                TriLds t;
+                load_tri(trirec, id, t);
+                pl = coverage_bound(t, pl, X0, Y0, T, dmax);
+            }
+            return pl;
+        };
         // the short form: every wave bounds the whole list (at most 64) on
         // its own against its largest depth and keeps it in its own 64
         // entries of bplane / bid
@@ -1788,18 +1851,10 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
             bool keep = false;
             float lb = 0.f;
             if (i < n_big) {
-                const uint32_t id = ldg(big + i);
-                if (id < num_tris) {
-                    TriLds t;
-                    load_tri(trirec, id, t);
-                    const int x0 = (int)(t.xr & 0xFFFFu), y0 = (int)(t.xr >> 16);
-                    const int x1 = (int)(t.yr & 0xFFFFu), y1 = (int)(t.yr >> 16);
-                    if (x1 > X0 && x0 < X0 + T && y1 > Y0 && y0 < Y0 + T) {
-                        const float4 pl = tile_bound(t, ldg(big_plane + i), X0, Y0, T, tmax);
-                        keep = !(pl.x > kSkipBound);
-                        lb = pl.x + fminf(pl.y, 0.f) * (float)(T - 1) + fminf(pl.z, 0.f) * (float)(T - 1);
-                    }
-                }
+                uint32_t id;
+                const float4 pl = list_bound(i, tmax, id);
+                keep = !(pl.x > kSkipBound);
+                lb = pl.x + fminf(pl.y, 0.f) * (float)(T - 1) + fminf(pl.z, 0.f) * (float)(T - 1);
             }
             const uint64_t km = __ballot(keep);
             if (lane == 0) wred_u[wave] = (uint32_t)__popcll(km);
@@ -1835,18 +1890,8 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
             uint32_t id = 0xFFFFFFFFu;
             float4 pl = make_float4(3.0e38f, 0.f, 0.f, 0.f);
             if (i < n_list) {
-                const uint32_t li = sorted ? (uint32_t)cand[i] : i;
-                id = ldg(big + li);
-                if (id < num_tris) {
-                    TriLds t;
-                    load_tri(trirec, id, t);
-                    const int x0 = (int)(t.xr & 0xFFFFu), y0 = (int)(t.xr >> 16);
-                    const int x1 = (int)(t.yr & 0xFFFFu), y1 = (int)(t.yr >> 16);
-                    if (x1 > X0 && x0 < X0 + T && y1 > Y0 && y0 < Y0 + T) {
-                        pl = tile_bound(t, ldg(big_plane + li), X0, Y0, T, own ? wmax : tmax);
-                        keep = !(pl.x > kSkipBound);
-                    }
-                }
+                pl = list_bound(sorted ? (uint32_t)cand[i] : i, own ? wmax : tmax, id);
+                keep = !(pl.x > kSkipBound);
             }
             // the entries to run: the wave's own 64, or the block's compacted chunk
             uint32_t j0, nb;
@@ -1911,10 +1956,7 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
         }
     }
     if (tile_min_depth) {
-        for (int o = 32; o > 0; o >>= 1) {
-            const float y = __shfl_xor(dmin, o);
-            dmin = y < dmin ? y : dmin;
-        }
+        dmin = wave_min_f(dmin);
         // one block per tile: the block's minimum is the tile's, a plain store
         __syncthreads();  // wdmax may still be read by the screen-list bound
         if (lane == 0) wdmax[wave] = dmin;
