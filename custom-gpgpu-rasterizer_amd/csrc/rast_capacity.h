@@ -211,18 +211,14 @@ __device__ float learned_prediction(const JobDesc &J, uint32_t t, bool live, flo
     return own;
 }
 
-// Queue regions of a wave's 64 tiles: one atomic on the frame's 64-bit
-// allocation top per wave reserves the sum of the capacities, and each tile
-// takes its place in that block by the wave's prefix sum.  A region that
-// would end past the queue storage keeps only the room that is left (the
-// rest of its entries go to the exact fallback); the top keeps the full sum,
-// from which the host grows the storage for the next frame.  Regions are
-// ordered by wave, not by tile: a tile's queue is read through its own
-// offset only.
-__device__ __forceinline__ void place_queue_regions(const JobDesc &J, uint32_t t, bool live, uint32_t cap)
+// Start of this lane's queue region of c entries (the wave's 64 lanes call
+// it): one atomic on the frame's 64-bit allocation top reserves the sum of the
+// wave's regions, and each lane takes its place in that block by the wave's
+// prefix sum.  Regions are ordered by wave, not by tile: a tile's queue is read
+// through its own offset only, so no scan over the tiles is needed.
+__device__ __forceinline__ uint64_t reserve_regions(FrameCounters *ctr, uint64_t c)
 {
     const uint32_t lane = threadIdx.x & 63u;
-    const uint64_t c = live ? cap : 0u;
     uint64_t incl = c;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -232,11 +228,21 @@ __device__ __forceinline__ void place_queue_regions(const JobDesc &J, uint32_t t
     const uint64_t total = __shfl(incl, 63);
     uint64_t base = 0;
     if (total) {  // wave-uniform
-        if (lane == 63) base = atomicAdd(&J.counters->capacity_top, (unsigned long long)total);
+        if (lane == 63) base = atomicAdd(&ctr->capacity_top, (unsigned long long)total);
         base = __shfl(base, 63);
     }
+    return base + incl - c;
+}
+
+// Queue regions of a wave's 64 tiles.  A region that would end past the queue
+// storage keeps only the room that is left (the rest of its entries go to the
+// exact fallback); the top keeps the full sum, from which the host grows the
+// storage for the next frame.
+__device__ __forceinline__ void place_queue_regions(const JobDesc &J, uint32_t t, bool live, uint32_t cap)
+{
+    const uint64_t c = live ? cap : 0u;
+    const uint64_t start = reserve_regions(J.counters, c), limit = J.queue_cap;
     if (live) {
-        const uint64_t start = base + incl - c, limit = J.queue_cap;
         J.tile_off[t] = (uint32_t)(start < limit ? start : limit);
         J.tile_cap[t] = start >= limit ? 0u : (uint32_t)(c < limit - start ? c : limit - start);
     }

@@ -106,15 +106,15 @@ struct FrameCounters {
     uint32_t num_alive;       // survivors of culling
     uint32_t num_binned;      // survivors with a non-empty pixel range and span <= big_threshold
     uint32_t num_big;
-    uint32_t total_pairs;     // exact queue entries (sum of per-tile counts)
+    uint32_t total_pairs;     // exact queue entries (sum of per-tile counts; formed when published)
     uint32_t overflow_tiles;  // single pass: tiles whose count exceeded capacity
     uint32_t ovf_entries;     // single pass: queue entries beyond capacity (fallback input)
     uint32_t pool_used;       // fallback pool entries
     uint32_t storage_overflow;// queue / pool / big list storage exhausted -> frame invalid
     uint32_t capacity_total;  // single pass: capacities as used (their sum fits the queue storage)
     uint32_t capacity_wanted; // single pass: the capacities' sum before that bound (saturated)
-    unsigned long long capacity_top;  // single pass: queue allocation top (the capacities' full sum);
-                                      // the two fields above are derived from it when published
+    unsigned long long capacity_top;  // queue allocation top: the full sum of the capacities (single pass,
+                                      // the two fields above are derived from it when published) or counts
 };
 
 // One frame of a launch: its parameters and the device buffers of the
@@ -148,7 +148,7 @@ struct alignas(16) JobDesc {  // 16-byte multiple: staged in 16-byte words
     uint32_t *trirec;
     uint8_t *alive;
     uint32_t *tile_count;        // exact: counts; single pass: cursors (end = exact counts)
-    uint32_t *tile_off;          // num_tiles + 1
+    uint32_t *tile_off;          // start of each tile's queue region
     uint32_t *tile_cap;          // single pass capacities
     uint32_t *tile_pool;         // per tile: fallback pool offset, or ~0u (previous-frame policy)
     uint32_t *tile_cursor;       // exact fill cursors / fallback cursors
@@ -161,8 +161,9 @@ struct alignas(16) JobDesc {  // 16-byte multiple: staged in 16-byte words
     uint32_t *big;
     // per screen-list slot, formed once by the setup pass and read by every
     // resolve tile: the triangle's depth plane over its pixel range
-    // (screen_plane), then bbox lo, bbox hi, ID
+    // (screen_plane); its bbox lo, bbox hi and ID
     float4 *big_plane;
+    uint4 *big_entry;
     FrameCounters *counters;     // num_alive stays 0 here: see alive_part
     FrameCounters *host_counters;  // pinned host copy, written at the end of the launch
     // culling survivors per setup block (launch-wide, indexed by the setup

@@ -24,7 +24,7 @@ struct Launch {
     const uint16_t *table[ST_COUNT];  // device block -> job tables (null when njobs == 1)
     uint32_t grid[ST_COUNT];          // blocks of each stage over all jobs (0: stage skipped)
     uint32_t cap_jobs;                // jobs binning in a single pass (capacities placed by the vertex launch)
-    uint32_t exact_jobs;              // jobs binning in two passes (count scan)
+    uint32_t exact_jobs;              // jobs binning in two passes 
     int model_hidden;                 // hidden width of the learned jobs' MLP (16, 32 or 64; 0: none)
     uint32_t shade_modes;             // shading instances: bit 0 point, 1 linear; 2, 3 the same for jobs sharing a scene
     uint32_t unshaded_jobs;           // jobs without a shading stage (their counters go out with k_publish)
@@ -59,7 +59,7 @@ hipError_t launch_interleave_maps(const uint32_t *d, const uint32_t *n, const ui
 // Modes 0 and 1 also reset the jobs' per-tile counts and depths (the frame
 // counters start at zero with the staging upload).
 hipError_t launch_vertex(const Launch &L, int with_capacity, hipStream_t s);
-hipError_t launch_scan(const Launch &L, hipStream_t s);  // exact counts
+hipError_t launch_place(const Launch &L, hipStream_t s);  // queue regions from exact counts
 hipError_t launch_setup(const Launch &L, hipStream_t s);
 hipError_t launch_fill(const Launch &L, hipStream_t s);
 // One tile-size group (ST_RES8 / ST_RES16 / ST_RES32); the groups are independent.
