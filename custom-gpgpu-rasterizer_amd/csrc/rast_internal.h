@@ -126,7 +126,8 @@ struct alignas(16) JobDesc {  // 16-byte multiple: staged in 16-byte words
     uint32_t block0[ST_COUNT];   // first block of this job in each stage's grid
     uint32_t nblocks[ST_COUNT];  // its block count there (0: not part of that stage)
     uint32_t mesh0;              // first entry of the job in the mesh table
-    uint32_t single;             // single-pass binning (capacities known before setup)
+    uint32_t single;             // the tiles' queue regions are known before setup: it fills them directly
+    uint32_t stride;             // entries of every tile's region, at tile * stride (0: tile_off, tile_cap)
     uint32_t learned;            // capacities from the MLP (else previous count * margin + slack)
     uint32_t small_limit;        // tile-clipped pixel count from which resolve goes pixel-parallel (at least half a tile)
     float margin;

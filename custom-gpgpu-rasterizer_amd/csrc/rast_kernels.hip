@@ -21,11 +21,11 @@
 //   k_setup    per triangle: assembly, cull, screen setup record; triangles
 //              whose bounding box has at most micro_limit pixels are
 //              rasterized on the spot with 64-bit atomic min into the key
-//              buffer; larger ones are counted per tile (exact two-pass) or
-//              written straight into per-tile queues (single pass); triangles
+//              buffer; larger ones are written straight into per-tile queues
+//              (predicted or fixed regions) or counted per tile (two passes); triangles
 //              spanning more than big_threshold tiles go to one screen list
 //   k_place    queue regions from the exact counts
-//   k_fill     exact second pass over the binned triangles
+//   k_fill     second pass over the binned triangles (two-pass jobs)
 //   k_resolve  one workgroup per tile: keys -> LDS (and cleared for the next
 //              frame), queued triangles rasterized in LDS (single pass: a
 //              tile whose count exceeded its capacity first gathers its
@@ -552,7 +552,7 @@ __device__ __forceinline__ void frame_init_block(const JobDesc *__restrict__ job
     if (i < n) {
         J.tile_count[i] = 0;
         J.tile_min_depth[i] = 1.0f;
-        if (J.single && !J.learned) J.tile_pool[i] = 0xFFFFFFFFu;
+        if (J.single && !J.learned && !J.stride) J.tile_pool[i] = 0xFFFFFFFFu;
     }
 }
 
@@ -750,6 +750,51 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
     vertex_block(meshes, block_group, groups, entries, jobs, blk - init_blocks, lds);
 }
 
+// Smaller 16-bit halves of two words, and of the wave's lanes (all active).
+__device__ __forceinline__ uint32_t min_u16x2(uint32_t a, uint32_t b)
+{
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+
+__device__ __forceinline__ uint32_t wave_min_u16x2(uint32_t v)
+{
+    v = min_u16x2(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x111, 0xf, 0xf, false));
+    v = min_u16x2(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x112, 0xf, 0xf, false));
+    v = min_u16x2(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x114, 0xf, 0xf, false));
+    v = min_u16x2(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x118, 0xf, 0xf, false));
+    v = min_u16x2(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x142, 0xa, 0xf, false));
+    v = min_u16x2(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x143, 0xc, 0xf, false));
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// Queue region of tile tl where it is known before the setup pass: (start, capacity).
+__device__ __forceinline__ uint2 tile_region(const JobDesc &J, uint32_t tl)
+{
+    if (J.stride) return make_uint2(tl * J.stride, J.stride);
+    return make_uint2(ldg(J.tile_off + tl), ldg(J.tile_cap + tl));
+}
+
+// Writes entry `slot` of tile tl's queue; one past its capacity is kept for
+// the exact fallback (one atomic on the shared counter per wave).
+__device__ __forceinline__ void queue_entry(const JobDesc &J, uint32_t tl, uint32_t gid, uint32_t slot, uint32_t off,
+                                            uint32_t cap)
+{
+    const bool fits = slot < cap;
+    const uint64_t om = __ballot(!fits);
+    if (fits) {
+        const uint32_t pos = off + slot;
+        if (pos < J.queue_cap) stg(J.queue + pos, gid);
+    } else {
+        const int leader = __builtin_ctzll(om);
+        uint32_t base = 0;
+        if (lane_id() == (uint32_t)leader) base = gatomic_add(&J.counters->ovf_entries, (uint32_t)__popcll(om));
+        const uint32_t o = (uint32_t)__shfl((int)base, leader) + popc_below(om);
+        if (o < J.ovf_cap) stg(J.ovf + o, make_uint2(tl, gid));
+        else J.counters->storage_overflow = 1;
+    }
+}
+
 // Whether the face normal (fx, fy, fz), normalized as normalize3 does, makes a
 // dot product above 0 (sign = 1) or below 0 (sign = -1) with the camera's
 // forward c, decided as the binary32 evaluation decides it.  With s the dot
@@ -813,6 +858,10 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
     __shared__ uint32_t moff[256];
     __shared__ unsigned long long mmask[4 * kMaskChunks];
     __shared__ uint32_t mfrag[4 * kFragRing];
+    __shared__ uint32_t lrect[8];  // per wave: smallest tile x | y << 16, then the complement of the largest
+    // the block's tile rectangle once the micro triangles are done
+    uint32_t *const lcursor = reinterpret_cast<uint32_t *>(mstage), *const loff = lcursor + 256, *const lcap = loff + 256;
+    static_assert(sizeof(mstage) >= 3 * 256 * sizeof(uint32_t), "the tile cursors, offsets and capacities fit");
     // workgroups in launch order (consecutive blocks spread over the XCDs;
     // XCD-contiguous ranges measured slower)
     const uint32_t blk = blockIdx.x;
@@ -1038,7 +1087,19 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
         }
     }
 
-    // the survivor list feeds the exact binner's fill pass only
+    {  // the wave's tile rectangle; its slice of the block's tile counts
+        const uint32_t wave = threadIdx.x >> 6;
+        uint32_t lo = 0xFFFFFFFFu, hi = 0xFFFFFFFFu;
+        if (__ballot(binned)) {
+            lo = wave_min_u16x2(binned ? tx0 | ty0 << 16 : 0xFFFFFFFFu);
+            hi = wave_min_u16x2(binned ? ~(tx1 | ty1 << 16) : 0xFFFFFFFFu);
+        }
+        lrect[wave] = lo;
+        lrect[4 + wave] = hi;
+        __builtin_amdgcn_wave_barrier();  // the slice's items are done (one wave's LDS accesses stay in order)
+        moff[threadIdx.x] = 0u;
+    }
+    // the survivor list feeds the two-pass binner's fill pass only
     uint32_t bslot, sslot;
     block_append(J.alive_part, ok, &ctr->num_big, is_big, &ctr->num_binned, binned && !single_pass, lds_append, bslot,
                  sslot);
@@ -1046,29 +1107,70 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
         if (bslot < J.big_cap) stg(J.big + bslot, gid);
         else ctr->storage_overflow = 1;
     }
-    if (binned) {
-        if (!single_pass) stg(J.survivors + sslot, gid);
+    if (binned && !single_pass) stg(J.survivors + sslot, gid);
+    // The block's tile rectangle (the same in every thread).  Up to 256 tiles,
+    // the usual case, are counted in LDS: one atomic per tile and block on the
+    // frame's counters, where grouping each wave's lanes by tile cost a ballot
+    // loop over its distinct tiles and four times the atomics.
+    uint32_t rx0, ry0, rx1, ry1;
+    {
+        uint32_t lo = lrect[0], hi = lrect[4];
+        for (int w = 1; w < 4; ++w) {
+            lo = min_u16x2(lo, lrect[w]);
+            hi = min_u16x2(hi, lrect[4 + w]);
+        }
+        lo = __builtin_amdgcn_readfirstlane(lo);  // scalar: the barriers below are in uniform branches
+        hi = __builtin_amdgcn_readfirstlane(hi);
+        rx0 = lo & 0xFFFFu; ry0 = lo >> 16;
+        rx1 = 0xFFFFu - (hi & 0xFFFFu); ry1 = 0xFFFFu - (hi >> 16);
+    }
+    const uint32_t rw = rx1 - rx0 + 1u, rh = ry1 - ry0 + 1u;
+    if (rx0 == 0xFFFFu) {  // nothing binned in the block
+    } else if (rw * rh <= 256u) {
+        uint32_t *const cnt = moff;  // zeroed by each wave in its own slice
+        const uint32_t w = tx1 - tx0 + 1u, i0 = binned ? (ty0 - ry0) * rw + (tx0 - rx0) : 0u;
+        const uint32_t n = binned ? span : 0u;
+        uint32_t i = i0, c = w;
+        for (uint32_t k = 0; k < n; ++k) {
+            atomicAdd(cnt + i, 1u);
+            ++i;
+            if (--c == 0u) { c = w; i += rw - w; }
+        }
+        __syncthreads();
+        const uint32_t mine = cnt[threadIdx.x];
+        if (mine) {
+            const uint32_t r = (uint32_t)(((float)threadIdx.x + 0.5f) * __builtin_amdgcn_rcpf((float)rw));  // as item_pixel
+            const uint32_t tl = (ry0 + r) * fp.tiles_x + rx0 + threadIdx.x - r * rw;
+            if (single_pass) {
+                const uint2 g = tile_region(J, tl);
+                const uint32_t first = gatomic_add(tile_count + tl, mine);
+                lcursor[threadIdx.x] = first;
+                loff[threadIdx.x] = g.x;
+                lcap[threadIdx.x] = g.y;
+            } else {
+                gatomic_add(tile_count + tl, mine);
+            }
+        }
+        if (single_pass) {
+            __syncthreads();
+            i = i0;
+            c = w;
+            uint32_t tl = ty0 * fp.tiles_x + tx0;
+            for (uint32_t k = 0; k < n; ++k) {
+                queue_entry(J, tl, gid, atomicAdd(lcursor + i, 1u), loff[i], lcap[i]);
+                ++i;
+                ++tl;
+                if (--c == 0u) { c = w; i += rw - w; tl += fp.tiles_x - w; }
+            }
+        }
+    } else if (binned) {
         const uint32_t w = tx1 - tx0 + 1;
         uint32_t tx = tx0, ty = ty0;
-        for (uint32_t s = 0; s < span; ++s) {
+        for (uint32_t k = 0; k < span; ++k) {
             const uint32_t tl = ty * fp.tiles_x + tx;
             if (single_pass) {
-                const uint32_t slot = claim_slot(tile_count, tl);
-                const bool fits = slot < ldg(J.tile_cap + tl);
-                const uint64_t om = __ballot(!fits);
-                if (fits) {
-                    const uint32_t pos = ldg(J.tile_off + tl) + slot;
-                    if (pos < J.queue_cap) stg(J.queue + pos, gid);
-                } else {
-                    // capacity exceeded: keep the entry for the exact fallback
-                    // (one atomic on the shared counter per wave)
-                    const int leader = __builtin_ctzll(om);
-                    uint32_t base = 0;
-                    if (lane_id() == (uint32_t)leader) base = gatomic_add(&ctr->ovf_entries, (uint32_t)__popcll(om));
-                    const uint32_t o = (uint32_t)__shfl((int)base, leader) + popc_below(om);
-                    if (o < J.ovf_cap) stg(J.ovf + o, make_uint2(tl, gid));
-                    else ctr->storage_overflow = 1;
-                }
+                const uint2 g = tile_region(J, tl);
+                queue_entry(J, tl, gid, claim_slot(tile_count, tl), g.x, g.y);
             } else {
                 count_tile(tile_count, tl);
             }
@@ -1415,7 +1517,6 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
     const FrameParams &fp = J.fp;
     const uint32_t *__restrict__ tile_count = J.tile_count;
     const uint32_t *__restrict__ tile_off = J.tile_off;
-    const uint32_t *__restrict__ tile_cap = J.single ? J.tile_cap : nullptr;
     const uint32_t *__restrict__ tile_pool = J.tile_pool;
     const uint32_t *__restrict__ queue = J.queue;
     const uint32_t queue_cap = J.queue_cap;
@@ -1488,8 +1589,8 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
 
     // List A: the tile's queue region.  List B: for single-pass binning,
     // the tile's entries beyond its capacity, which setup appended to the
-    // overflow list as (tile, id) pairs.  Learned capacities: the tile's
-    // block gathers them itself into a pool region it allocates (one atomic
+    // overflow list as (tile, id) pairs.  Learned and fixed capacities: the
+    // tile's block gathers them itself into a pool region it allocates (one atomic
     // per overflowing tile; the list is read four entries per thread at a
     // time), so no placement pass runs.  Previous-frame capacities: the
     // fallback passes placed them in the tile's pool region.  The order of a
@@ -1497,12 +1598,18 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
     // fragments by depth, then ID).
     const uint32_t cnt = ldg(tile_count + tile);
     uint32_t n_a = cnt, n_b = 0;
-    const uint32_t qoff = ldg(tile_off + tile);
+    uint32_t qoff, cp = 0xFFFFFFFFu;
+    if (J.single) {
+        const uint2 g = tile_region(J, tile);
+        qoff = g.x;
+        cp = g.y;
+    } else {
+        qoff = ldg(tile_off + tile);
+    }
     const uint32_t *list_a = queue + qoff;
     const uint32_t *list_b = pool;
-    if (tile_cap) {
-        const uint32_t cp = ldg(tile_cap + tile);
-        if (cnt > cp && !J.learned) {
+    if (J.single) {
+        if (cnt > cp && !J.learned && !J.stride) {
             n_a = cp;
             const uint32_t po = ldg(tile_pool + tile);
             if (po != 0xFFFFFFFFu) {
@@ -2588,7 +2695,7 @@ hipError_t launch_setup(const Launch &L, hipStream_t s)
 
 hipError_t launch_place(const Launch &L, hipStream_t s)
 {
-    if (L.exact_jobs == 0) return hipSuccess;
+    if (L.two_pass_jobs == 0) return hipSuccess;
     hipLaunchKernelGGL(k_place, dim3(L.grid[ST_INIT]), dim3(256), 0, s, L.jobs, L.table[ST_INIT]);
     return hipGetLastError();
 }

@@ -24,7 +24,7 @@ struct Launch {
     const uint16_t *table[ST_COUNT];  // device block -> job tables (null when njobs == 1)
     uint32_t grid[ST_COUNT];          // blocks of each stage over all jobs (0: stage skipped)
     uint32_t cap_jobs;                // jobs binning in a single pass (capacities placed by the vertex launch)
-    uint32_t exact_jobs;              // jobs binning in two passes 
+    uint32_t two_pass_jobs;           // jobs binning in two passes
     int model_hidden;                 // hidden width of the learned jobs' MLP (16, 32 or 64; 0: none)
     uint32_t shade_modes;             // shading instances: bit 0 point, 1 linear; 2, 3 the same for jobs sharing a scene
     uint32_t unshaded_jobs;           // jobs without a shading stage (their counters go out with k_publish)

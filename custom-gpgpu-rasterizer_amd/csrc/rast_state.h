@@ -145,7 +145,9 @@ struct rast_renderer {
     rast_frame_opts last_opts{};
     bool frame_pending = false;
     bool frame_valid = false;
-    bool last_single = false;
+    bool last_single = false;              // capacities predicted (single-pass policies)
+    uint32_t last_stride = 0;              // exact binning into fixed regions of this many entries (0: two passes)
+    bool two_pass = false;                 // the scene overflowed its fixed regions: exact frames take two passes
     bool last_shared_attr = false;  // the last frame's attributes were split (views rendered together)
     bool prev_valid_before = false;
     bool frame_had_prev = false;  // the last frame had a previous frame (features valid)

@@ -61,10 +61,11 @@ enum { RAST_CULL_BACK = 0, RAST_CULL_FRONT = 1, RAST_CULL_NONE = 2 };
 enum { RAST_SAMPLE_POINT = 0, RAST_SAMPLE_LINEAR = 1 };
 /* CCR/VisualisationState.h:3-8 */
 enum { RAST_VIS_PBR = 0, RAST_VIS_DEPTH = 1, RAST_VIS_NORMAL = 2 };
-/* Bin-queue policy: exact two-pass (count, scan, fill); single pass with
- * capacities from the learned model; single pass with previous-frame
- * counts x margin.  The single-pass policies fall back to exact binning for
- * every tile whose capacity overflowed, so the frame output never changes. */
+/* Bin-queue policy: exact (nothing predicted: fixed queue regions, or two
+ * passes, count and fill, where the frame has too many tiles for them); single
+ * pass with capacities from the learned model; single pass with
+ * previous-frame counts x margin.  Entries beyond a tile's region are binned
+ * exactly under every policy, so the frame output never changes. */
 enum { RAST_BIN_EXACT = 0, RAST_BIN_LEARNED = 1, RAST_BIN_PREVFRAME = 2 };
 
 /* Camera of CCR/Camera.h:6-31 (position, m_Forward, FOV degrees, near, far).
