@@ -789,7 +789,7 @@ void plan_free(LaunchPlan &p)
         if (p.exec[i]) (void)hipGraphExecDestroy(p.exec[i]);
         p.exec[i] = nullptr;
     }
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < kSideStreams; ++i) {
         if (p.side[i]) (void)hipStreamDestroy(p.side[i]);
         if (p.joined[i]) (void)hipEventDestroy(p.joined[i]);
         p.side[i] = nullptr;
@@ -839,6 +839,13 @@ static int dev_alloc(DBuf &b, size_t bytes)
     return RAST_OK;
 }
 
+// Launches of at most this many 32x32 tiles in all (two per CU) are resolved in
+// quarters.  Resolve, quarters against whole tiles: 300 tiles (a sphere in 480p)
+// 8.3 and 14.0 us, 350 tiles of up to 1,191 triangles 17.8 and 25.9; 768 light
+// tiles 8.2 and 6.1; 2,040 tiles 32.2 and 32.6 (terrain), 17.0 and 14.0 (no
+// queues); 8,160 tiles 116 and 69.
+constexpr uint32_t kQuarterTiles = 512;
+
 // Grids, block -> job tables and block -> mesh tables of a launch structure.
 static int build_plan(LaunchPlan &P, rast_renderer *const *rs, uint32_t n, int hidden, uint64_t key)
 {
@@ -854,13 +861,6 @@ static int build_plan(LaunchPlan &P, rast_renderer *const *rs, uint32_t n, int h
         if (!P.done[i]) HIP_TRY(hipEventCreateWithFlags(&P.done[i], hipEventDisableTiming | hipEventDisableSystemFence));
     }
     P.built = false;
-    if (!P.fork) {
-        HIP_TRY(hipEventCreateWithFlags(&P.fork, hipEventDisableTiming | hipEventDisableSystemFence));
-        for (int i = 0; i < 2; ++i) {
-            HIP_TRY(hipStreamCreateWithFlags(&P.side[i], hipStreamNonBlocking));
-            HIP_TRY(hipEventCreateWithFlags(&P.joined[i], hipEventDisableTiming | hipEventDisableSystemFence));
-        }
-    }
     if (n > 65535) return rast_set_error(RAST_E_INVALID_ARG, "at most 65535 jobs per launch");
     Launch &L = P.L;
     L = Launch{};
@@ -878,9 +878,17 @@ static int build_plan(LaunchPlan &P, rast_renderer *const *rs, uint32_t n, int h
     P.tri_block0.clear();
     uint64_t grid[ST_COUNT] = {};
     uint32_t mesh_entry = 0;
+    std::vector<uint32_t> job_tiles(n);
+    uint64_t tiles32 = 0;
+    for (uint32_t j = 0; j < n; ++j) {
+        job_tiles[j] = ceil_div(rs[j]->W, rs[j]->tile) * ceil_div(rs[j]->H, rs[j]->tile);
+        if (rs[j]->tile == 32) tiles32 += job_tiles[j];
+    }
+    // (a persistent launch keeps whole tiles)
+    const bool few_tiles = tiles32 <= kQuarterTiles && rs[0]->resolve_mode == RAST_RESOLVE_PER_TILE;
     for (uint32_t j = 0; j < n; ++j) {
         rast_renderer *r = rs[j];
-        const uint32_t ntiles = ceil_div(r->W, r->tile) * ceil_div(r->H, r->tile);
+        const uint32_t ntiles = job_tiles[j];
         const uint32_t ntris = std::max<uint32_t>(r->total_tris, 1);
         const bool single = r->last_single, fixed = r->last_stride != 0;
         uint32_t nb[ST_COUNT] = {};
@@ -892,16 +900,12 @@ static int build_plan(LaunchPlan &P, rast_renderer *const *rs, uint32_t n, int h
         const bool placed = single && !job_learned(r);
         nb[ST_FBALLOC] = placed ? ceil_div(ntiles, 256) : 0;
         nb[ST_FBFILL] = placed ? std::min<uint32_t>(ceil_div(ntris, 256), 256) : 0;
-        const int res = r->tile == 8 ? ST_RES8 : (r->tile == 16 ? ST_RES16 : ST_RES32);
-        nb[res] = ntiles;
+        const bool quarters = r->tile == 32 && few_tiles;
+        const int res = r->tile == 8 ? ST_RES8 : r->tile == 16 ? ST_RES16 : quarters ? ST_RES32Q : ST_RES32;
+        nb[res] = quarters ? 4 * ntiles : ntiles;
         nb[ST_SHADE] = job_shades(r) ? ceil_div(r->W, 64) * ceil_div(r->H, (uint32_t)kShadeRows) : 0;
         if (!nb[ST_SHADE]) ++L.unshaded_jobs;
-        for (int st = 0; st < ST_COUNT; ++st) {
-            P.block0[(size_t)j * ST_COUNT + st] = (uint32_t)grid[st];
-            P.nblocks[(size_t)j * ST_COUNT + st] = nb[st];
-            grid[st] += nb[st];
-            if (n > 1) tables[st].insert(tables[st].end(), nb[st], (uint16_t)j);
-        }
+        for (int st = 0; st < ST_COUNT; ++st) P.nblocks[(size_t)j * ST_COUNT + st] = nb[st];
         if (single) ++L.cap_jobs;
         else if (!fixed) ++L.two_pass_jobs;
         for (rast_mesh *m : scene_meshes(r)) {
@@ -923,12 +927,38 @@ static int build_plan(LaunchPlan &P, rast_renderer *const *rs, uint32_t n, int h
             ++mesh_entry;
         }
     }
-    // a grid's threads must stay below 2^32 (256 threads per block in every stage but the scan)
+    // The jobs' blocks in each stage: in job order, but the resolve stages take
+    // the frames of fewest tiles first.  A tile's time is uneven in a small frame
+    // of a large scene (cube-map faces: up to 30 times the mean), so those start
+    // first and the even tiles of the large frames fill the launch's end.
+    std::vector<uint32_t> by_tiles(n);
+    for (uint32_t j = 0; j < n; ++j) by_tiles[j] = j;
+    std::stable_sort(by_tiles.begin(), by_tiles.end(), [&](uint32_t a, uint32_t b) { return job_tiles[a] < job_tiles[b]; });
+    for (int st = 0; st < ST_COUNT; ++st) {
+        const bool resolve = st == ST_RES8 || st == ST_RES16 || st == ST_RES32 || st == ST_RES32Q;
+        for (uint32_t k = 0; k < n; ++k) {
+            const size_t j = resolve ? by_tiles[k] : k;
+            const uint32_t nb = P.nblocks[j * ST_COUNT + st];
+            P.block0[j * ST_COUNT + st] = (uint32_t)grid[st];
+            grid[st] += nb;
+            if (n > 1) tables[st].insert(tables[st].end(), nb, (uint16_t)j);
+        }
+    }
+    // a grid's threads must stay below 2^32 (256 threads per block in every stage)
     for (int st = 0; st < ST_COUNT; ++st)
         if (grid[st] >= (1ull << 24)) return rast_set_error(RAST_E_INVALID_ARG, "launch too large (stage %d)", st);
     if (vs_group.size() >= (1ull << 24) || tri_mesh.size() >= (1ull << 24))
         return rast_set_error(RAST_E_INVALID_ARG, "launch too large (meshes)");
     for (int st = 0; st < ST_COUNT; ++st) L.grid[st] = (uint32_t)grid[st];
+    // side streams and their events, where the launch holds several tile-size groups
+    const int sides = !!grid[ST_RES8] + !!grid[ST_RES16] + !!grid[ST_RES32] + !!grid[ST_RES32Q] - 1;
+    if (sides > 0 && !P.fork)
+        HIP_TRY(hipEventCreateWithFlags(&P.fork, hipEventDisableTiming | hipEventDisableSystemFence));
+    for (int i = 0; i < sides; ++i) {
+        if (!P.side[i]) HIP_TRY(hipStreamCreateWithFlags(&P.side[i], hipStreamNonBlocking));
+        if (!P.joined[i])
+            HIP_TRY(hipEventCreateWithFlags(&P.joined[i], hipEventDisableTiming | hipEventDisableSystemFence));
+    }
     P.njobs = n;
     P.nmeshes = mesh_entry;
     L.vs_blocks = (uint32_t)vs_group.size();
@@ -1187,9 +1217,9 @@ static int enqueue_launch(LaunchPlan &P, hipStream_t s, rast_renderer *timed)
     HIP_TRY(launch_fallback(L, s));
     RAST_TRY(mark(timed, EV_FALLBACK, s));
     {
-        // tile-size groups are independent: the second and third run on side streams
-        int groups[3], ng = 0;
-        for (int st : { ST_RES16, ST_RES32, ST_RES8 })
+        // tile-size groups are independent: all but the first run on side streams
+        int groups[kSideStreams + 1], ng = 0;
+        for (int st : { ST_RES16, ST_RES32, ST_RES32Q, ST_RES8 })
             if (L.grid[st]) groups[ng++] = st;
         if (ng > 1) {
             HIP_TRY(hipEventRecord(P.fork, s));

@@ -97,6 +97,7 @@ enum Stage : int {
     ST_RES8,      // resolve, 8x8 tiles (one block per tile, in launch order)
     ST_RES16,     // resolve, 16x16 tiles
     ST_RES32,     // resolve, 32x32 tiles
+    ST_RES32Q,    // resolve, 32x32 tiles of small frames (one block per 16x16 quarter)
     ST_SHADE,     // 64 x kShadeRows-pixel blocks
     ST_COUNT
 };

@@ -179,6 +179,11 @@ __device__ __forceinline__ uint32_t gatomic_add(uint32_t *p, uint32_t v)
     return __hip_atomic_fetch_add(gptr(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+__device__ __forceinline__ void gatomic_min(uint32_t *p, uint32_t v)
+{
+    __hip_atomic_fetch_min(gptr(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 __device__ __forceinline__ void gatomic_min(unsigned long long *p, unsigned long long v)
 {
     __hip_atomic_fetch_min(gptr(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -442,12 +447,13 @@ __device__ __forceinline__ bool fragment(const Tri &t, float px, float py, float
 }
 
 // fragment() at a pixel whose current depth is dbest (<= 1), with a reject
-// that needs no division first.  With r = fl(1 / area) (t.inv) and
-// u = 2^-24, b_i = fl(w_i r) is within 3.0001 u of a_i = fl(w_i / area), and
-// both three-term sums are within 3.0001 u S of their exact values
-// (S = sum |a_i z_i|), so z' = fl(fl(b0 z0 + b1 z1) + b2 z2) is within
-// 9.0003 u S of the depth that depth_of() computes; S <= S' (1 + 6.01 u) for
-// the evaluated S' = sum |fl(b_i z_i)|.  m = 10 u S' + 1e-37 therefore covers
+// that needs no division first.  With r the hardware reciprocal of area
+// (t.inv, within 2 u: 1 ulp) and u = 2^-24, b_i = fl(w_i r) is within 4.0001 u
+// of a_i = fl(w_i / area), and both three-term sums are within 3.0001 u S of
+// their exact values (S = sum |a_i z_i|), so z' = fl(fl(b0 z0 + b1 z1) + b2
+// z2) is within 10.0004 u S of the depth that depth_of() computes; S <= S' (1
+// + 7.01 u) for the evaluated S' = sum |fl(b_i z_i)|.  m = 12 u S' + 1e-37
+// therefore covers
 // the difference (the constant covers gradual underflow): where
 // z' - m > dbest the fragment loses (or exceeds 1), where z' + m < 0 it is out
 // of range.  A NaN or infinite z' or m rejects nothing.
@@ -458,7 +464,7 @@ __device__ __forceinline__ bool fragment_closer(const TriLds &t, float px, float
     if (!(w0 >= 0.f && w1 >= 0.f && w2 >= 0.f)) return false;
     const float p0 = (w0 * t.inv) * t.z0, p1 = (w1 * t.inv) * t.z1, p2 = (w2 * t.inv) * t.z2;
     const float zq = (p0 + p1) + p2;
-    const float m = ((fabsf(p0) + fabsf(p1)) + fabsf(p2)) * (10.0f / 16777216.0f) + 1.0e-37f;
+    const float m = ((fabsf(p0) + fabsf(p1)) + fabsf(p2)) * (12.0f / 16777216.0f) + 1.0e-37f;
     if (zq - m > dbest || zq + m < 0.f) return false;
     return depth_of(t, w0, w1, w2, z);
 }
@@ -484,6 +490,25 @@ __device__ __forceinline__ void load_tri(const uint32_t *__restrict__ rec, uint3
     set_edges(t);
     t.id = id;
     t.inv = 0.f;
+}
+
+// The same for an ID that is the same in every lane: scalar loads, through the
+// constant address space (no kernel that reads a setup record writes one).
+__device__ __forceinline__ void load_tri_uniform(const uint32_t *__restrict__ rec, uint32_t id, TriLds &t)
+{
+    typedef const __attribute__((address_space(4))) u32x4_t *cptr;
+    const cptr r = (cptr)(uint64_t)(rec + (size_t)__builtin_amdgcn_readfirstlane(id) * kTriRecWords);
+    const u32x4_t q0 = r[0], q1 = r[1], q2 = r[2];
+    t.sx0 = __uint_as_float(q0.x); t.sy0 = __uint_as_float(q0.y);
+    t.sx1 = __uint_as_float(q0.z); t.sy1 = __uint_as_float(q0.w);
+    t.sx2 = __uint_as_float(q1.x); t.sy2 = __uint_as_float(q1.y);
+    t.z0 = __uint_as_float(q1.z); t.area = __uint_as_float(q1.w);
+    t.z2 = __uint_as_float(q2.x); t.z1 = __uint_as_float(q2.y);
+    t.xr = q2.z;
+    t.yr = q2.w;
+    set_edges(t);
+    t.id = id;
+    t.inv = __builtin_amdgcn_rcpf(t.area);
 }
 
 // The depth plane of a screen-list triangle over its pixel range (the
@@ -1355,8 +1380,9 @@ __global__ __launch_bounds__(256) void k_fallback_fill(const JobDesc *__restrict
     }
 }
 
-// Bounds of a screen-list triangle t over the tile at (X0, Y0), used to skip
-// the tile or single pixels before the exact fragment test.  tmax is the
+// Bounds of a screen-list triangle t over a tile, or a wave's rows of one: the
+// TX x TY pixels at (X0, Y0) ("the tile" below), used to skip them all or
+// single pixels before the exact fragment test.  tmax is the
 // largest depth the pixels in question hold; depths only decrease from there.
 // sp is the triangle's screen_plane.
 //
@@ -1394,7 +1420,8 @@ __global__ __launch_bounds__(256) void k_fallback_fill(const JobDesc *__restrict
 // and all tests for every triangle in every tile, an 8K frame's resolve took
 // 311 us instead of 266, a 4K frame's 87 instead of 74, both with the tighter
 // item ranges).
-__device__ __forceinline__ float4 plane_bound(const float4 sp, uint32_t range_lo, int X0, int Y0, int T, float tmax)
+__device__ __forceinline__ float4 plane_bound(const float4 sp, uint32_t range_lo, int X0, int Y0, int TX, int TY,
+                                               float tmax)
 {
     const float4 skip = make_float4(3.0e38f, 0.f, 0.f, 0.f);
     const float4 none = make_float4(-1.0e30f, 0.f, 0.f, 1.0e30f);
@@ -1404,21 +1431,22 @@ __device__ __forceinline__ float4 plane_bound(const float4 sp, uint32_t range_lo
     const float px = sp.y * dX, py = sp.z * dY;
     const float L0 = (sp.x + px) + py;
     const float S = (fabsf(sp.x) + fabsf(px)) + fabsf(py);
-    const float Tm = (float)(T - 1);
-    const float span = (fabsf(sp.y) + fabsf(sp.z)) * Tm;
+    const float Tx = (float)(TX - 1), Ty = (float)(TY - 1);
+    const float span = fabsf(sp.y) * Tx + fabsf(sp.z) * Ty;
     const float aL = fabsf(L0);
     const float M = (sp.w + u * (4.02f * S + 12.0f * aL + 13.0f * span + 8.0f)) * 1.0001f + 1.0e-30f;
     if (!(M < 0.25f)) return none;
     // whole-tile tests at the tile's corners (L is affine)
-    const float Lmin = (L0 + fminf(sp.y, 0.f) * Tm) + fminf(sp.z, 0.f) * Tm;
-    const float Lmax = (L0 + fmaxf(sp.y, 0.f) * Tm) + fmaxf(sp.z, 0.f) * Tm;
+    const float Lmin = (L0 + fminf(sp.y, 0.f) * Tx) + fminf(sp.z, 0.f) * Ty;
+    const float Lmax = (L0 + fmaxf(sp.y, 0.f) * Tx) + fmaxf(sp.z, 0.f) * Ty;
     if (Lmin - M > 1.0f || Lmax + M < 0.0f || Lmin - M > tmax) return skip;
     return make_float4(L0 - M, sp.y, sp.z, 2.0f * M + 8.0f * u * (aL + span + 1.0f));
 }
 
 // plane_bound's bound pl of triangle t, with the tests of its setup record: skip where no
 // pixel of the tile is covered, and the constant bound where no plane applies.
-__device__ __forceinline__ float4 coverage_bound(const TriLds &t, const float4 pl, int X0, int Y0, int T, float tmax)
+__device__ __forceinline__ float4 coverage_bound(const TriLds &t, const float4 pl, int X0, int Y0, int TX, int TY,
+                                                  float tmax)
 {
     const float4 skip = make_float4(3.0e38f, 0.f, 0.f, 0.f);
     const float4 none = make_float4(-1.0e30f, 0.f, 0.f, 1.0e30f);
@@ -1431,7 +1459,7 @@ __device__ __forceinline__ float4 coverage_bound(const TriLds &t, const float4 p
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         float w0, w1, w2;
-        edges(t, (float)(X0 + (c & 1) * (T - 1)), (float)(Y0 + (c >> 1) * (T - 1)), w0, w1, w2);
+        edges(t, (float)(X0 + (c & 1) * (TX - 1)), (float)(Y0 + (c >> 1) * (TY - 1)), w0, w1, w2);
         lo0 = fminf(lo0, w0); hi0 = fmaxf(hi0, w0);
         lo1 = fminf(lo1, w1); hi1 = fmaxf(hi1, w1);
         lo2 = fminf(lo2, w2); hi2 = fmaxf(hi2, w2);
@@ -1476,22 +1504,39 @@ __device__ __forceinline__ float tile_max_depth(const uint64_t *best, uint32_t l
     return m;
 }
 
-// Ascending bitonic sort of v[0, P) in LDS, P a power of two; ends with a barrier.
-template <int NT>
-__device__ __forceinline__ void bitonic_sort(uint64_t *v, uint32_t P, uint32_t tid)
+// Ascending sort of the n <= CAP distinct values v in LDS: an entry's place is
+// the count of smaller ones, so every thread reads the list once (all lanes the
+// same word) against the entries it holds.  For the 100 to 700 entries met
+// here that is 2 to 25 K cycles without a barrier inside, where a bitonic
+// network's 28 to 55 barrier-separated steps took 12 to 78 K.  Ends with a
+// barrier.
+template <int NT, int CAP>
+__device__ __forceinline__ void rank_sort(uint64_t *v, uint32_t n, uint32_t tid)
 {
-    for (uint32_t k = 2; k <= P; k <<= 1) {
-        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-            for (uint32_t i = tid; i < P; i += NT) {
-                const uint32_t l = i ^ j;
-                if (l > i) {
-                    const uint64_t a = v[i], b = v[l];
-                    if ((a > b) == ((i & k) == 0)) { v[i] = b; v[l] = a; }
-                }
+    constexpr int E = (CAP + NT - 1) / NT;
+    uint64_t own[E];
+    uint32_t rank[E];
+#pragma unroll
+    for (int k = 0; k < E; ++k) {
+        const uint32_t i = tid + (uint32_t)k * NT;
+        own[k] = i < n ? v[i] : 0ull;  // nothing is below 0: its rank is not used
+        rank[k] = 0;
+    }
+    for (uint32_t i = 0; i < n; ++i) {
+        const uint64_t x = v[i];
+        rank[0] += x < own[0];
+        if constexpr (E > 1) {
+            if (n > (uint32_t)NT) {  // the same for the whole block
+#pragma unroll
+                for (int k = 1; k < E; ++k) rank[k] += x < own[k];
             }
-            __syncthreads();
         }
     }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < E; ++k)
+        if (tid + (uint32_t)k * NT < n) v[rank[k]] = own[k];
+    __syncthreads();
 }
 
 // RA_PerTileKernel (CCR/CUDARenderer.cu:1039-1129) redesigned: one workgroup
@@ -1510,9 +1555,9 @@ template <bool kLinear, bool kSplit>
 __device__ __forceinline__ void shade_pixel(const DevMesh *__restrict__ meshes, const JobDesc &J, const float *unit,
                                             uint32_t x, uint32_t y, uint32_t id);
 
-template <int T, int NT, int STAGE, int SHADE>
-__device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, const DevMesh *__restrict__ meshes,
-                                             const float *unit)
+template <int T, int NT, int STAGE, int SHADE, int BIN = T>
+__device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, uint32_t part,
+                                             const DevMesh *__restrict__ meshes, const float *unit)
 {
     const FrameParams &fp = J.fp;
     const uint32_t *__restrict__ tile_count = J.tile_count;
@@ -1554,28 +1599,35 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
     float4 *const bplane = reinterpret_cast<float4 *>(stage);
     uint32_t *const bid = reinterpret_cast<uint32_t *>(bplane + NT);
     __shared__ uint32_t off[NT];
-    __shared__ uint32_t wlist[NT];
+    __shared__ uint8_t wlist[NT];  // staged triangles tested at one pixel per lane
     __shared__ uint32_t rring[NW * kFragRing];  // per wave: covered items waiting for their depth
     __shared__ unsigned long long omask[kOwnerWords];  // item window: bit k = a staged triangle's first item
     __shared__ uint32_t ocum[kOwnerWords];             // first items before each mask word
     __shared__ uint8_t olist[NT];                      // staged triangles with items, in item order
     __shared__ uint32_t wred_u[NW], wwhole[NW], wown[NW], otot;
     __shared__ float wdmax[NW];
-    __shared__ uint32_t ovf_base, ovf_fill;
+    __shared__ uint32_t ovf_base, ovf_fill, cand_n;
 
     const uint32_t ntiles = fp.tiles_x * fp.tiles_y;
     if (tile >= ntiles) return;  // the same for the whole block
     const uint32_t txi = tile % fp.tiles_x, tyi = tile / fp.tiles_x;
-    const int X0 = (int)(txi * T), Y0 = (int)(tyi * T);
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    constexpr uint32_t kParts = BIN / T;  // parts per tile edge
+    const int X0 = (int)(txi * BIN + part % kParts * T), Y0 = (int)(tyi * BIN + part / kParts * T);
+    if (BIN != T && (X0 >= (int)fp.width || Y0 >= (int)fp.height)) return;  // a part off the frame
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-    // the lane's pixels: p = tid + q * NT (rows of T pixels)
+    // the lane's pixels: p = p0 + q * 64 (rows of T pixels), so a wave's pixels
+    // are BH whole rows, which bound the screen-list triangles more tightly
+    // than rows spread over the tile
+    constexpr int BH = 64 * PPT / T;
+    const int p0 = (int)(wave * 64u * PPT + lane);
+    const int Y0w = Y0 + (int)wave * BH;
     uint64_t best[PPT];
     int pxs[PPT], pys[PPT];
     bool inside[PPT];
 #pragma unroll
     for (int q = 0; q < PPT; ++q) {
-        const int p = (int)tid + q * NT;
+        const int p = p0 + q * 64;
         pxs[q] = X0 + p % T;
         pys[q] = Y0 + p / T;
         inside[q] = pxs[q] < (int)fp.width && pys[q] < (int)fp.height;
@@ -1624,7 +1676,7 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
             if (tid == 0) {
                 const uint32_t b = gatomic_add(&ctr->pool_used, want);
                 if (b + want > pool_cap || b + want < b) ctr->storage_overflow = 1;
-                gatomic_add(&ctr->overflow_tiles, 1u);
+                if (part == 0) gatomic_add(&ctr->overflow_tiles, 1u);
                 ovf_base = b;
                 ovf_fill = 0;
             }
@@ -1669,7 +1721,7 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
 
     if (n_tile) {
 #pragma unroll
-        for (int q = 0; q < PPT; ++q) key[(int)tid + q * NT] = best[q];
+        for (int q = 0; q < PPT; ++q) key[p0 + q * 64] = best[q];
         for (uint32_t base = 0; base < n_tile; base += NT) {
             const uint32_t i = base + tid;
             uint32_t area = 0;
@@ -1722,7 +1774,7 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
             }
             const uint32_t first = before + incl - area;  // this triangle's first item
             off[tid] = first;
-            if (whole) wlist[pbefore + popc_below(wm)] = tid;
+            if (whole) wlist[pbefore + popc_below(wm)] = (uint8_t)tid;
             if (area) olist[obefore + popc_below(hm)] = (uint8_t)tid;
             __syncthreads();
             // compacted items, in windows of 64 kOwnerWords items: a mask bit
@@ -1800,7 +1852,7 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
             if (nwhole) {
                 __syncthreads();
 #pragma unroll
-                for (int q = 0; q < PPT; ++q) best[q] = key[(int)tid + q * NT];
+                for (int q = 0; q < PPT; ++q) best[q] = key[p0 + q * 64];
                 for (uint32_t q2 = 0; q2 < nwhole; ++q2) {
                     const MicroLds &st = stage[wlist[q2]];
                     const int x0 = (int)(st.xr & 0xFFFFu), x1 = (int)(st.xr >> 16);
@@ -1808,8 +1860,8 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
 #pragma unroll
                     for (int q = 0; q < PPT; ++q) {
                         // the wave's pixels of this round are the rows [wy0, wy1)
-                        const int wy0 = Y0 + ((int)(wave * 64) + q * NT) / T;
-                        const int wy1 = Y0 + ((int)(wave * 64) + 63 + q * NT) / T + 1;
+                        const int wy0 = Y0w + q * 64 / T;
+                        const int wy1 = Y0w + (q * 64 + 63) / T + 1;
                         if (y1 <= wy0 || y0 >= wy1) continue;
                         const int px = pxs[q], py = pys[q];
                         if (px >= x0 && px < x1 && py >= y0 && py < y1) {
@@ -1822,37 +1874,37 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
                     }
                 }
 #pragma unroll
-                for (int q = 0; q < PPT; ++q) key[(int)tid + q * NT] = best[q];
+                for (int q = 0; q < PPT; ++q) key[p0 + q * 64] = best[q];
             }
             __syncthreads();
         }
 #pragma unroll
-        for (int q = 0; q < PPT; ++q) best[q] = key[(int)tid + q * NT];
+        for (int q = 0; q < PPT; ++q) best[q] = key[p0 + q * 64];
     }
 
-    // Screen-list triangles.  A triangle's plane and pixel range are tested
-    // first, the whole triangle only where some lane passes them.  The
-    // wave's largest depth (pixels of the frame) skips a triangle for the
-    // whole wave where its plane lies above it over the entire tile: the
-    // plane's float value at its lowest corner, less 8 u S (S its term
+    // Screen-list triangles.  Every wave works on its own rows, with no barrier:
+    // it takes the list 64 entries at a time, one per lane, bounds each over
+    // its rows against its largest depth (pixels of the frame) and runs those
+    // left, one after the other, on its pixels.  LDS holds an entry's plane and
+    // ID; its record is read again, with scalar loads, where it is run.  There
+    // the plane and pixel range are tested first, the whole triangle only
+    // where some lane passes them.  The wave keeps a mask of the entries whose
+    // plane, at its lowest corner of the rows and less 8 u S (S its term
     // magnitudes; its float evaluation is within 3 u S of the exact affine
-    // plane, whose minimum over the tile is at that corner), bounds the
-    // triangle's depth at every pixel from below.  The wave keeps a mask of
-    // up to 64 triangles (one per lane) whose bound is not above its largest
-    // depth and narrows it each time that depth falls, so a skipped triangle
-    // costs no iteration.
+    // plane, whose minimum over the rows is at that corner), is not above its
+    // largest depth, and narrows it each time that depth falls, so a skipped
+    // triangle costs no iteration.
     //
-    // LDS holds a kept triangle's plane and ID; its record is read again at
-    // its (uniform) address where it is run.  A list of at most 64 is
-    // handled by every wave on its own: its lanes load and bound the whole
-    // list against the wave's largest depth, with no barrier.  A longer list is
-    // first bounded over the tile (pass 1), keeping the triangles that can
-    // still take a pixel, keyed by their depth lower bound (in the key
-    // array, free once the queue is resolved).  Sorted front to back, pass 2
-    // then stages them chunk by chunk and stops where the next lower bound
-    // lies behind every pixel of the tile.  More survivors than fit go to
-    // pass 2 in their stored order.  Each chunk is loaded and bounded in
-    // parallel and compacted into LDS.
+    // A list longer than NT is first bounded over the whole tile, keeping the
+    // triangles that can still take a pixel, keyed by their depth lower bound
+    // (in the key array, free once the queue is resolved) and sorted front to
+    // back; a wave then stops at the first group whose lower bound lies behind
+    // its pixels.  More survivors than fit are taken in their stored order.
+    //
+    // Faces of a cube map over terrain hold 900 to 1,800 triangles on the list,
+    // a tile 200 of them (up to 700), of which a wave runs 20 to 50 (up to 240):
+    // with these, the rows bounded per wave and the small frames' tiles first, the
+    // 7-view resolve went 298 -> 251 us.
     uint32_t n_big = ldg(&ctr->num_big);
     n_big = n_big < big_cap ? n_big : big_cap;
     if (n_big) {
@@ -1864,16 +1916,16 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
             return wave_max_f(d);
         };
         auto wave_floor = [](const float4 &pl) {
-            const float lmin = pl.x + fminf(pl.y, 0.f) * (float)(T - 1) + fminf(pl.z, 0.f) * (float)(T - 1);
-            const float mag = fabsf(pl.x) + (fabsf(pl.y) + fabsf(pl.z)) * (float)(T - 1);
+            const float lmin = pl.x + fminf(pl.y, 0.f) * (float)(T - 1) + fminf(pl.z, 0.f) * (float)(BH - 1);
+            const float mag = fabsf(pl.x) + fabsf(pl.y) * (float)(T - 1) + fabsf(pl.z) * (float)(BH - 1);
             return lmin - mag * (8.0f / 16777216.0f);
         };
         float wmax = wave_max_depth();
         // the exact tests of triangle st on the lanes' pixels; true when some
         // lane passed the per-pixel bounds (wmax is then current)
-        auto run = [&](const TriLds &st, const float4 &pl, const uint2 &bb) {
-            const int x0 = (int)(bb.x & 0xFFFFu), y0 = (int)(bb.x >> 16);
-            const int x1 = (int)(bb.y & 0xFFFFu), y1 = (int)(bb.y >> 16);
+        auto run = [&](const TriLds &st, const float4 &pl) {
+            const int x0 = (int)(st.xr & 0xFFFFu), y0 = (int)(st.xr >> 16);
+            const int x1 = (int)(st.yr & 0xFFFFu), y1 = (int)(st.yr >> 16);
             bool pass[PPT];
             bool any = false;
 #pragma unroll
@@ -1881,7 +1933,7 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
                 const int px = pxs[q], py = pys[q];
                 // lower bound of the triangle's depth here: above the current
                 // depth it loses, and with the band width below 0 it is out of range
-                const float zc = pl.x + pl.y * (float)(px - X0) + pl.z * (float)(py - Y0);
+                const float zc = pl.x + pl.y * (float)(px - X0) + pl.z * (float)(py - Y0w);
                 const float db = __uint_as_float((uint32_t)(best[q] >> 32));
                 pass[q] = px >= x0 && px < x1 && py >= y0 && py < y1 && !(zc > db) && !(zc + pl.w < 0.f);
                 any = any || pass[q];
@@ -1899,125 +1951,75 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
             wmax = wave_max_depth();
             return true;
         };
-        // entry i's bound over the tile against the depth dmax (x > kSkipBound: not run)
-        auto list_bound = [&](uint32_t i, float dmax, uint32_t &id) {
+        // entry i's bound over the TX x TY pixels at (X0, Yb) against the depth
+        // dmax (x > kSkipBound: not run)
+        auto list_bound = [&](uint32_t i, int Yb, int TY, float dmax, uint32_t &id) {
             const float4 sp = ldg(big_plane + i);
             const uint4 e = ldg(big_entry + i);
             id = e.z;
             float4 pl = make_float4(3.0e38f, 0.f, 0.f, 0.f);
             const int x0 = (int)(e.x & 0xFFFFu), y0 = (int)(e.x >> 16), x1 = (int)(e.y & 0xFFFFu), y1 = (int)(e.y >> 16);
-            if (id < num_tris && x1 > X0 && x0 < X0 + T && y1 > Y0 && y0 < Y0 + T)
-                pl = plane_bound(sp, e.x, X0, Y0, T, dmax);
+            if (id < num_tris && x1 > X0 && x0 < X0 + T && y1 > Yb && y0 < Yb + TY)
+                pl = plane_bound(sp, e.x, X0, Yb, T, TY, dmax);
             if (!(pl.x > kSkipBound)) {
                 TriLds t;
                 load_tri(trirec, id, t);
-                pl = coverage_bound(t, pl, X0, Y0, T, dmax);
+                pl = coverage_bound(t, pl, X0, Yb, T, TY, dmax);
             }
             return pl;
         };
-        // the short form: every wave bounds the whole list (at most 64) on
-        // its own against its largest depth and keeps it in its own 64
-        // entries of bplane / bid
-        const bool own = n_big <= 64u;  // the same for the whole block
-        float tmax = 1.0f;
         uint64_t *cand = key;  // NPIX entries: (ordered lower bound << 32) | list index
         uint32_t n_cand = 0;
         const bool presort = n_big > (uint32_t)NT;
-        if (!own) tmax = tile_max_depth<PPT, NW>(best, lane, wave, wdmax);
-        for (uint32_t base = 0; presort && base < n_big; base += NT) {
-            const uint32_t i = base + tid;
-            bool keep = false;
-            float lb = 0.f;
-            if (i < n_big) {
-                uint32_t id;
-                const float4 pl = list_bound(i, tmax, id);
-                keep = !(pl.x > kSkipBound);
-                lb = pl.x + fminf(pl.y, 0.f) * (float)(T - 1) + fminf(pl.z, 0.f) * (float)(T - 1);
+        if (presort) {
+            if (tid == 0) cand_n = 0;
+            const float tmax = tile_max_depth<PPT, NW>(best, lane, wave, wdmax);  // holds two barriers
+            for (uint32_t base = wave * 64u; base < n_big; base += NT) {
+                const uint32_t i = base + lane;
+                bool keep = false;
+                float lb = 0.f;
+                if (i < n_big) {
+                    uint32_t id;
+                    const float4 pl = list_bound(i, Y0, T, tmax, id);
+                    keep = !(pl.x > kSkipBound);
+                    lb = pl.x + fminf(pl.y, 0.f) * (float)(T - 1) + fminf(pl.z, 0.f) * (float)(T - 1);
+                }
+                const uint64_t km = __ballot(keep);
+                uint32_t slot = 0;
+                if (lane == 0 && km) slot = atomicAdd(&cand_n, (uint32_t)__popcll(km));
+                slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)slot) + popc_below(km);
+                if (keep && slot < (uint32_t)NPIX) cand[slot] = ((uint64_t)ordered_bits(lb) << 32) | i;
             }
-            const uint64_t km = __ballot(keep);
-            if (lane == 0) wred_u[wave] = (uint32_t)__popcll(km);
             __syncthreads();
-            uint32_t before = 0, nk = 0;
-            for (int w = 0; w < NW; ++w) {
-                if (w < (int)wave) before += wred_u[w];
-                nk += wred_u[w];
-            }
-            const uint32_t slot = n_cand + before + popc_below(km);
-            if (keep && slot < (uint32_t)NPIX) cand[slot] = ((uint64_t)ordered_bits(lb) << 32) | i;
-            n_cand += nk;
-            __syncthreads();
+            n_cand = cand_n;
         }
         const bool sorted = presort && n_cand <= (uint32_t)NPIX;
-        if (sorted) {
-            uint32_t P = 1;
-            while (P < n_cand) P <<= 1;
-            for (uint32_t q = n_cand + tid; q < P; q += NT) cand[q] = ~0ull;
-            __syncthreads();
-            bitonic_sort<NT>(cand, P, tid);
-        }
+        if (sorted) rank_sort<NT, NPIX>(cand, n_cand, tid);
         const uint32_t n_list = sorted ? n_cand : n_big;
-        const uint32_t step = own ? 64u : (uint32_t)NT;
-        for (uint32_t base = 0; base < n_list; base += step) {
-            if (!own) {
-                if (base) tmax = tile_max_depth<PPT, NW>(best, lane, wave, wdmax);
-                // sorted: every further triangle is bounded below by this one's bound
-                if (sorted && (uint32_t)(cand[base] >> 32) > ordered_bits(tmax)) break;
-            }
-            const uint32_t i = base + (own ? lane : tid);
-            bool keep = false;
+        const uint32_t j0 = wave * 64u;  // the wave's own entries of bplane / bid
+        for (uint32_t base = 0; base < n_list; base += 64u) {
+            // sorted: every further triangle is bounded below by this one's bound
+            if (sorted && (uint32_t)(cand[base] >> 32) > ordered_bits(wmax)) break;
+            const uint32_t i = base + lane;
             uint32_t id = 0xFFFFFFFFu;
             float4 pl = make_float4(3.0e38f, 0.f, 0.f, 0.f);
-            if (i < n_list) {
-                pl = list_bound(sorted ? (uint32_t)cand[i] : i, own ? wmax : tmax, id);
-                keep = !(pl.x > kSkipBound);
+            if (i < n_list) pl = list_bound(sorted ? (uint32_t)cand[i] : i, Y0w, BH, wmax, id);
+            const bool keep = !(pl.x > kSkipBound);
+            const float floor_l = wave_floor(pl);
+            bplane[j0 + lane] = pl;
+            bid[j0 + lane] = id;
+            // the wave's lanes read one another's entries below
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            uint64_t live = __ballot(keep && !(floor_l > wmax));
+            while (live) {
+                const uint32_t j = j0 + (uint32_t)__builtin_ctzll(live);
+                live &= live - 1u;
+                TriLds st;
+                load_tri_uniform(trirec, bid[j], st);
+                if (run(st, bplane[j])) live &= __ballot(!(floor_l > wmax));
             }
-            // the entries to run: the wave's own 64, or the block's compacted chunk
-            uint32_t j0, nb;
-            if (own) {
-                j0 = wave * 64u;
-                nb = n_list;
-                if (!keep) pl = make_float4(3.0e38f, 0.f, 0.f, 0.f);
-                bplane[j0 + lane] = pl;
-                bid[j0 + lane] = id;
-                // the wave's lanes read one another's entries below
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            } else {
-                const uint64_t km = __ballot(keep);
-                if (lane == 0) wred_u[wave] = (uint32_t)__popcll(km);
-                __syncthreads();
-                uint32_t before = 0;
-                nb = 0;
-                for (int w = 0; w < NW; ++w) {
-                    if (w < (int)wave) before += wred_u[w];
-                    nb += wred_u[w];
-                }
-                if (keep) {
-                    const uint32_t slot = before + popc_below(km);
-                    bplane[slot] = pl;
-                    bid[slot] = id;
-                }
-                __syncthreads();
-                j0 = 0;
-            }
-            // 64 entries at a time, one per lane
-            for (uint32_t g = 0; g < nb; g += 64u) {
-                const uint32_t jl = g + lane;
-                float floor_l = 3.0e38f;
-                if (jl < nb) floor_l = wave_floor(bplane[j0 + jl]);
-                uint64_t live = __ballot(jl < nb && !(floor_l > wmax));
-                while (live) {
-                    const uint32_t j = j0 + g + (uint32_t)__builtin_ctzll(live);
-                    live &= live - 1u;
-                    const float4 plj = bplane[j];
-                    TriLds st;
-                    load_tri(trirec, bid[j], st);
-                    st.inv = 1.0f / st.area;
-                    if (run(st, plj, make_uint2(st.xr, st.yr))) live &= __ballot(!(floor_l > wmax));
-                }
-            }
-            if (!own) __syncthreads();
         }
     }
 
@@ -2035,14 +2037,17 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, co
     }
     if (tile_min_depth) {
         dmin = wave_min_f(dmin);
-        // one block per tile: the block's minimum is the tile's, a plain store
+        // one block per tile: the block's minimum is the tile's, a plain store;
+        // parts of a tile: the smallest of theirs (depths are >= 0, so their
+        // bits order like the values; the vertex launch reset it to 1)
         __syncthreads();  // wdmax may still be read by the screen-list bound
         if (lane == 0) wdmax[wave] = dmin;
         __syncthreads();
         if (tid == 0) {
             float m = wdmax[0];
             for (int w = 1; w < NW; ++w) m = wdmax[w] < m ? wdmax[w] : m;
-            stg(tile_min_depth + tile, m);
+            if constexpr (BIN == T) stg(tile_min_depth + tile, m);
+            else if (m < 1.0f) gatomic_min(reinterpret_cast<uint32_t *>(tile_min_depth) + tile, __float_as_uint(m));
         }
     }
     if constexpr (SHADE != 0) {
@@ -2064,7 +2069,20 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_
 {
     uint32_t local;
     const JobDesc &J = jobs[job_of(table, jobs, STAGE, local)];
-    resolve_tile<T, NT, STAGE, 0>(J, local, nullptr, nullptr);
+    resolve_tile<T, NT, STAGE, 0>(J, local, 0u, nullptr, nullptr);
+}
+
+// Frames of few tiles: four workgroups per 32x32 tile, one per 16x16 quarter.
+// Such a frame's time is its slowest tile's, which a quarter's share of the
+// pixels, with bounds over 16x4 pixels per wave instead of 32x8, shortens; the
+// tile's queue is read four times for it (480p sphere, 300 tiles: 14.0 -> 8.3
+// us; on a full chip it is slower: the dispatch's rule has the figures).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_resolve_quarters(
+    const JobDesc *__restrict__ jobs, const uint16_t *__restrict__ table)
+{
+    uint32_t local;
+    const JobDesc &J = jobs[job_of(table, jobs, ST_RES32Q, local)];
+    resolve_tile<16, 256, ST_RES32Q, 0, 32>(J, local >> 2, local & 3u, nullptr, nullptr);
 }
 
 // ------------------------------------------------------------- shading
@@ -2565,7 +2583,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(SHADE ? 3 : 
             j = __builtin_amdgcn_readfirstlane((uint32_t)table[item]);
             local = item - jobs[j].block0[STAGE];
         }
-        resolve_tile<T, NT, STAGE, SHADE>(jobs[j], local, meshes, unit);
+        resolve_tile<T, NT, STAGE, SHADE>(jobs[j], local, 0u, meshes, unit);
     }
 }
 
@@ -2783,6 +2801,9 @@ hipError_t launch_resolve(const Launch &L, int stage, hipStream_t s)
         break;
     case ST_RES32:
         hipLaunchKernelGGL((k_resolve<32, 256, ST_RES32>), dim3(g), dim3(256), 0, s, L.jobs, L.table[ST_RES32]);
+        break;
+    case ST_RES32Q:
+        hipLaunchKernelGGL(k_resolve_quarters, dim3(g), dim3(256), 0, s, L.jobs, L.table[ST_RES32Q]);
         break;
     default: return hipErrorInvalidValue;
     }

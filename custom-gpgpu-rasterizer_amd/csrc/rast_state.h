@@ -45,6 +45,8 @@ inline void dfree(DBuf &b)
 // structure key (frame sizes, tile sizes, binning modes, mesh sizes); the
 // per-launch contents (cameras, options, buffer pointers) are restaged into
 // the pinned block and uploaded by the launch itself.
+constexpr int kSideStreams = 3;  // one less than the resolve stages
+
 struct LaunchPlan {
     uint64_t key = 0;
     bool built = false;
@@ -69,8 +71,8 @@ struct LaunchPlan {
     bool done_pending[2] = { false, false };
     int parity = 0;                                 // the block the next launch uses
     // side streams running the resolve passes of different tile sizes concurrently
-    hipStream_t side[2] = { nullptr, nullptr };
-    hipEvent_t fork = nullptr, joined[2] = { nullptr, nullptr };
+    hipStream_t side[kSideStreams] = {};
+    hipEvent_t fork = nullptr, joined[kSideStreams] = {};
 };
 void plan_free(LaunchPlan &p);
 // Waits until no queued GPU work uses r's buffers (its stream and, when its
