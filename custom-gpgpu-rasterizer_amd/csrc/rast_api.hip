@@ -309,6 +309,7 @@ static void orphan_mesh(rast_mesh *m)
     if (m->idx) (void)hipFree(m->idx);
     m->ivert14 = nullptr;
     m->idx = nullptr;
+    m->boxes = nullptr;
     for (auto &t : m->tex) t = nullptr;
     m->texq = nullptr;
     m->r = nullptr;
@@ -446,9 +447,15 @@ extern "C" int rast_mesh_create(rast_renderer *r, const rast_ivertex *verts, uin
     m->attr_max = attr_max;
     for (int i = 0; i < 16; ++i) m->world[i] = world ? world[i] : ((i % 5 == 0) ? 1.f : 0.f);
     hipError_t e = hipMalloc((void **)&m->ivert14, v14.size() * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void **)&m->idx, (size_t)num_indices * 4);
+    const size_t idx_bytes = ((size_t)num_indices * 4 + 15) & ~(size_t)15;
+    if (e == hipSuccess) e = hipMalloc((void **)&m->idx, idx_bytes + (size_t)ceil_div(ntri, 256) * 32);
     if (e == hipSuccess) e = hipMemcpy(m->ivert14, v14.data(), v14.size() * sizeof(float), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(m->idx, indices, (size_t)num_indices * 4, hipMemcpyHostToDevice);
+    if (e == hipSuccess) {  // on the copies' stream; done before any frame's stream can read them
+        m->boxes = reinterpret_cast<float4 *>(reinterpret_cast<char *>(m->idx) + idx_bytes);
+        e = launch_mesh_boxes(m->ivert14, m->idx, ntri, topology, m->boxes, nullptr);
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) {
         free_mesh(m);
         return rast_set_error(e == hipErrorOutOfMemory ? RAST_E_OUT_OF_MEMORY : RAST_E_HIP, "mesh upload: %s",
@@ -1147,6 +1154,7 @@ static int stage_launch(LaunchPlan &P, rast_renderer *const *rs, uint32_t n)
             DevMesh &d = dm[me];
             memset(&d, 0, sizeof d);
             d.ivert = m->ivert14;
+            d.boxes = m->boxes;
             d.idx = m->idx;
             d.num_verts = m->nv;
             d.num_tris = m->ntri;

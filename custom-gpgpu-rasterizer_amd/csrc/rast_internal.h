@@ -47,8 +47,9 @@ struct DevTexture {
 };
 
 // One mesh of the frame, rebuilt on the host each frame (matrices change).
-struct DevMesh {
+struct alignas(16) DevMesh {  // 16-byte multiple: staged in 16-byte words
     const float *ivert;       // 14 floats per vertex
+    const float4 *boxes;      // object-space box (lo, hi) of every 256 triangles
     const uint32_t *idx;
     uint32_t num_verts;
     uint32_t num_tris;

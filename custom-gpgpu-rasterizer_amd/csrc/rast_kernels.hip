@@ -15,7 +15,7 @@
 //
 // Pipeline (one launch per stage for all jobs and meshes of a launch):
 //   k_vertex   per vertex: clip/NDC position + shading attributes; beside
-//              it, single-pass jobs' tile capacities and queue regions, and
+//              it, the setup workgroups whose triangles' box is out of view, single-pass jobs' tile capacities and queue regions, and
 //              the reset of every job's per-tile counts (the frame counters
 //              start at zero with the launch's staging upload)
 //   k_setup    per triangle: assembly, cull, screen setup record; triangles
@@ -596,6 +596,111 @@ __global__ __launch_bounds__(256) void k_clear_keys(unsigned long long *__restri
     for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256u) keys[i] = kClearKey;
 }
 
+// Object-space box of every 256 consecutive triangles of a mesh (one setup
+// workgroup's), formed once when the mesh is created: (lo, -), (hi, -).  A corner
+// that is not finite, or huge, makes the box unbounded (never culled).
+__global__ __launch_bounds__(256) void k_mesh_boxes(const float *__restrict__ ivert, const uint32_t *__restrict__ idx,
+                                                    uint32_t ntri, int topology, float4 *__restrict__ boxes)
+{
+    __shared__ float red[4][6];
+    const uint32_t k = blockIdx.x * 256u + threadIdx.x;
+    const float inf = __int_as_float(0x7f800000);
+    float b[6] = { inf, inf, inf, inf, inf, inf };  // smallest x y z, smallest -x -y -z
+    if (k < ntri) {
+#pragma unroll
+        for (uint32_t c = 0; c < 3; ++c) {
+            const uint32_t v = ldg(idx + (topology == 0 ? 3 * (size_t)k + c : (size_t)k + c));
+            const float *p = ivert + (size_t)v * kIVertexFloats;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                const float x = ldg(p + a);
+                const bool fine = fabsf(x) < 1.0e18f;  // false for NaN
+                b[a] = fminf(b[a], fine ? x : -inf);
+                b[3 + a] = fminf(b[3 + a], fine ? -x : -inf);
+            }
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < 6; ++a) {
+        for (int o = 32; o > 0; o >>= 1) b[a] = fminf(b[a], __shfl_xor(b[a], o));
+        if (lane_id() == 0) red[threadIdx.x >> 6][a] = b[a];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float m[6];
+#pragma unroll
+        for (int a = 0; a < 6; ++a) m[a] = fminf(fminf(red[0][a], red[1][a]), fminf(red[2][a], red[3][a]));
+        stg(boxes + 2 * (size_t)blockIdx.x, make_float4(m[0], m[1], m[2], 0.f));
+        stg(boxes + 2 * (size_t)blockIdx.x + 1, make_float4(-m[3], -m[4], -m[5], 0.f));
+    }
+}
+
+// Whether every triangle with corners in the box [lo, hi] fails the evaluated
+// frustum test: all its corners outside one plane of the view volume.  An
+// evaluated clip coordinate is within 4.0003 u S of the exact affine value (S:
+// its row's term magnitudes, largest over the box; u = 2^-24), its quotient by
+// w within u more, and the values formed here, at the box's eight corners,
+// within 4.0003 u S too: with all corners' w on one side of zero by 16 u Sw
+// and, after multiplying by that sign, x + w, w - x and so on beyond 32 u (Sx
+// + Sw), each evaluated quotient of every point of the box is on the far side
+// of its plane.  A box reaching across w = 0, or with values that overflow or
+// are not finite, is not culled.
+__device__ __forceinline__ bool box_outside(const float *wvp, const float4 lo, const float4 hi)
+{
+    const float u = 1.0f / 16777216.0f;
+    const float ax = fmaxf(fabsf(lo.x), fabsf(hi.x)), ay = fmaxf(fabsf(lo.y), fabsf(hi.y));
+    const float az = fmaxf(fabsf(lo.z), fabsf(hi.z));
+    float m[16], S[4];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) m[k] = ldg(wvp + k);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[r] = fabsf(m[r]) * ax + fabsf(m[4 + r]) * ay + fabsf(m[8 + r]) * az + fabsf(m[12 + r]);
+    if (!(S[0] < 1.0e30f && S[1] < 1.0e30f && S[2] < 1.0e30f && S[3] < 1.0e30f)) return false;
+    const float ew = 16.0f * u * S[3] + 1.0e-30f;
+    const float ex = 32.0f * u * (S[0] + S[3]), ey = 32.0f * u * (S[1] + S[3]), ez = 32.0f * u * (S[2] + S[3]);
+    uint32_t out = 0xFFu;  // planes every corner so far is beyond; bits 6, 7: w > 0, w < 0
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const float x = c & 1 ? hi.x : lo.x, y = c & 2 ? hi.y : lo.y, z = c & 4 ? hi.z : lo.z;
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = m[r] * x + m[4 + r] * y + m[8 + r] * z + m[12 + r];
+        const float sg = v[3] < 0.f ? -1.f : 1.f, w = fabsf(v[3]);
+        const float X = v[0] * sg, Y = v[1] * sg, Z = v[2] * sg;
+        uint32_t b = 0;
+        b |= X + w < -ex ? 1u : 0u;
+        b |= X - w > ex ? 2u : 0u;
+        b |= Y + w < -ey ? 4u : 0u;
+        b |= Y - w > ey ? 8u : 0u;
+        b |= Z < -ez ? 16u : 0u;
+        b |= Z - w > ez ? 32u : 0u;
+        b |= v[3] > ew ? 64u : 0u;
+        b |= v[3] < -ew ? 128u : 0u;
+        out &= b;
+    }
+    return (out & 0xC0u) != 0u && (out & 0x3Fu) != 0u;
+}
+
+// The cull stage, workgroups of the vertex launch: one thread per setup
+// workgroup marks in its survivor count (alive_part) whether its triangles'
+// box lies outside the view, so that the workgroup ends at once.  In a
+// workgroup of its own per 256 boxes the test costs a few instructions per
+// setup wave and rides along with the vertex pass.  Six cube-map faces and a
+// main view of 4.0 M triangles: setup 338 -> 277 us; a frame that sees all of
+// its scene is unchanged.
+constexpr uint32_t kCulledBlock = 0x80000000u;
+
+__device__ __forceinline__ void cull_block(const DevMesh *__restrict__ meshes, const uint32_t *__restrict__ block_mesh,
+                                           const JobDesc *__restrict__ jobs, uint32_t tri_blocks, uint32_t blk)
+{
+    const uint32_t b = blk * 256u + threadIdx.x;
+    if (b >= tri_blocks) return;
+    const DevMesh *M = meshes + ldg(block_mesh + b);
+    const float4 *box = ldg(&M->boxes) + 2 * (size_t)(b - ldg(&M->tri_block0));
+    const bool out = box_outside(M->wvp, ldg(box), ldg(box + 1));
+    stg(ldg(&jobs[ldg(&M->job)].alive_part) + b, out ? kCulledBlock : 0u);
+}
+
 // VS_Kernel / GetNDCVertex (CCR/CUDARenderer.cu:673-700, CCR/CUDAROPs.cu:99-118).
 // A block's 256 vertices are 16 KB of input records and 16 KB of attribute
 // records per job, contiguous in HBM.  Both go through LDS so that global
@@ -755,7 +860,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
                                                 const uint32_t *__restrict__ entries,
                                                 const JobDesc *__restrict__ jobs,
                                                 const uint16_t *__restrict__ cap_table, uint32_t cap_blocks,
-                                                const uint16_t *__restrict__ init_table, uint32_t init_blocks)
+                                                const uint16_t *__restrict__ init_table, uint32_t init_blocks,
+                                                const uint32_t *__restrict__ tri_block_mesh, uint32_t tri_blocks,
+                                                uint32_t cull_blocks)
 {
     constexpr int kVertexF4 = 256 * 4, kCapF4 = (capacity_lds_floats<H>() + 3) / 4;
     __shared__ float4 lds[kVertexF4 > kCapF4 ? kVertexF4 : kCapF4];
@@ -772,7 +879,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
         frame_init_block(jobs, init_table, blk);
         return;
     }
-    vertex_block(meshes, block_group, groups, entries, jobs, blk - init_blocks, lds);
+    if (blk - init_blocks < cull_blocks) {
+        cull_block(meshes, tri_block_mesh, jobs, tri_blocks, blk - init_blocks);
+        return;
+    }
+    vertex_block(meshes, block_group, groups, entries, jobs, blk - init_blocks - cull_blocks, lds);
 }
 
 // Smaller 16-bit halves of two words, and of the wave's lanes (all active).
@@ -904,6 +1015,13 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
     const uint32_t k = (blk - M.tri_block0) * 256u + threadIdx.x;
     const bool valid = k < M.num_tris;
     const uint32_t gid = M.tri_base + k;
+    // the cull stage found the block's box outside the view: no triangle survives
+    if (__builtin_amdgcn_readfirstlane(ldg(J.alive_part + blk)) == kCulledBlock) {
+        if (valid) stg(J.alive + gid, (uint8_t)0);
+        __syncthreads();  // every wave has read the mark
+        if (threadIdx.x == 0) stg(J.alive_part + blk, 0u);
+        return;
+    }
     bool ok = false;
     int xmin = 0, ymin = 0, xmax = 0, ymax = 0;
     float mnx = 0.f, mny = 0.f, ext_x = 0.f, ext_y = 0.f;  // smallest corner, extent
@@ -2665,6 +2783,14 @@ hipError_t launch_interleave_maps(const uint32_t *d, const uint32_t *n, const ui
     return hipGetLastError();
 }
 
+hipError_t launch_mesh_boxes(const float *ivert, const uint32_t *idx, uint32_t ntri, int topology, float4 *boxes,
+                             hipStream_t s)
+{
+    if (ntri == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_mesh_boxes, dim3(ceil_div(ntri, 256u)), dim3(256), 0, s, ivert, idx, ntri, topology, boxes);
+    return hipGetLastError();
+}
+
 hipError_t launch_clear_keys(unsigned long long *keys, size_t n, hipStream_t s)
 {
     const size_t blocks = (n + 255) / 256;
@@ -2677,28 +2803,30 @@ hipError_t launch_vertex(const Launch &L, int with_capacity, hipStream_t s)
     const uint32_t cap_blocks = L.grid[ST_CAP];
     const uint32_t vs_blocks = with_capacity == 2 ? 0u : L.vs_blocks;  // 2: the capacity stage alone
     const uint32_t init_blocks = with_capacity == 2 ? 0u : L.grid[ST_INIT];
+    const uint32_t cull_blocks = with_capacity == 2 ? 0u : ceil_div(L.tri_blocks, 256u);
     const uint16_t *init_table = L.table[ST_INIT];
     if (!with_capacity || !cap_blocks) {
         if (vs_blocks + init_blocks == 0) return hipSuccess;
-        hipLaunchKernelGGL(k_vertex<0>, dim3(init_blocks + vs_blocks), dim3(256), 0, s, L.meshes, L.vs_block_group,
-                           L.vs_groups, L.vs_entries, L.jobs, (const uint16_t *)nullptr, 0u, init_table, init_blocks);
+        hipLaunchKernelGGL(k_vertex<0>, dim3(init_blocks + cull_blocks + vs_blocks), dim3(256), 0, s, L.meshes,
+                           L.vs_block_group, L.vs_groups, L.vs_entries, L.jobs, (const uint16_t *)nullptr, 0u, init_table,
+                           init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks);
         return hipGetLastError();
     }
-    const dim3 g(cap_blocks + init_blocks + vs_blocks), b(256);
+    const dim3 g(cap_blocks + init_blocks + cull_blocks + vs_blocks), b(256);
     // one instance per hidden width (a launch's learned jobs share one);
     // heuristic-only launches take the smallest
     switch (L.model_hidden) {
     case 32:
         hipLaunchKernelGGL(k_vertex<32>, g, b, 0, s, L.meshes, L.vs_block_group, L.vs_groups, L.vs_entries, L.jobs,
-                           L.table[ST_CAP], cap_blocks, init_table, init_blocks);
+                           L.table[ST_CAP], cap_blocks, init_table, init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks);
         break;
     case 64:
         hipLaunchKernelGGL(k_vertex<64>, g, b, 0, s, L.meshes, L.vs_block_group, L.vs_groups, L.vs_entries, L.jobs,
-                           L.table[ST_CAP], cap_blocks, init_table, init_blocks);
+                           L.table[ST_CAP], cap_blocks, init_table, init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks);
         break;
     default:
         hipLaunchKernelGGL(k_vertex<16>, g, b, 0, s, L.meshes, L.vs_block_group, L.vs_groups, L.vs_entries, L.jobs,
-                           L.table[ST_CAP], cap_blocks, init_table, init_blocks);
+                           L.table[ST_CAP], cap_blocks, init_table, init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks);
         break;
     }
     return hipGetLastError();

@@ -52,6 +52,9 @@ inline size_t stage_meshes_offset(uint32_t n)
 
 // Resets a key buffer to depth 1 / no triangle (before a renderer's first frame).
 hipError_t launch_clear_keys(unsigned long long *keys, size_t n, hipStream_t s);
+// Object-space boxes of a mesh's runs of 256 triangles (two float4 each).
+hipError_t launch_mesh_boxes(const float *ivert, const uint32_t *idx, uint32_t ntri, int topology, float4 *boxes,
+                             hipStream_t s);
 hipError_t launch_interleave_maps(const uint32_t *d, const uint32_t *n, const uint32_t *sp, const uint32_t *g,
                                   uint4 *out, size_t count, hipStream_t s);
 // with_capacity 0: the vertex pass; 1: the vertex pass with the single-pass

@@ -96,7 +96,8 @@ struct TexQuad {
 struct rast_mesh {
     rast_renderer *r = nullptr;
     float *ivert14 = nullptr;  // 14 floats per vertex (the 56-byte IVertex as given) + 16 bytes of padding
-    uint32_t *idx = nullptr;
+    uint32_t *idx = nullptr;   // the indices, then (16-byte aligned) the boxes
+    float4 *boxes = nullptr;   // object-space box (lo, hi) of every 256 triangles
     uint32_t nv = 0, ni = 0, ntri = 0;
     int topology = 0;
     float world[16];
