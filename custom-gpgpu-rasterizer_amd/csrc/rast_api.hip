@@ -1026,10 +1026,15 @@ static int build_plan(LaunchPlan &P, rast_renderer *const *rs, uint32_t n, int h
         }
         if (sbytes) RAST_TRY(dev_alloc(P.d_sattr, sbytes));
     }
-    // shading instances: bit (sampling mode + 2 for the shared-scene layout)
+    // shading instances: bit (sampling mode + 2 for the shared-scene layout + 4 for far records)
     for (uint32_t j = 0; j < n; ++j)
-        if (P.nblocks[(size_t)j * ST_COUNT + ST_SHADE])
-            L.shade_modes |= 1u << (rs[j]->last_opts.sample_state + (P.sattr_off[j] != SIZE_MAX ? 2 : 0));
+        if (P.nblocks[(size_t)j * ST_COUNT + ST_SHADE]) {
+            FrameParams fp{};
+            fp.num_verts = rs[j]->total_verts;
+            fp.num_tris = rs[j]->total_tris;
+            L.shade_modes |= 1u << (rs[j]->last_opts.sample_state + (P.sattr_off[j] != SIZE_MAX ? 2 : 0) +
+                                    (far_records(fp) ? 4 : 0));
+        }
     // resolve form: the persistent kernels are sized to what the device holds
     L.resolve_mode = n ? rs[0]->resolve_mode : 0;
     L.fused_shade = 0;

@@ -87,6 +87,14 @@ struct FrameParams {
     uint32_t num_meshes;
 };
 
+// Whether a frame's attribute records (48 bytes a vertex) or setup records (64
+// bytes a triangle) reach past a 32-bit byte offset: shaded by instances that
+// form 64-bit addresses.
+__host__ __device__ inline bool far_records(const FrameParams &fp)
+{
+    return fp.num_verts > 0xFFFFFFFFu / 48u || fp.num_tris > (1u << 26);
+}
+
 // Launch stages whose grids are shared by all jobs of a launch: block b of
 // stage s serves job table_s[b], as its block b - JobDesc::block0[s].
 enum Stage : int {

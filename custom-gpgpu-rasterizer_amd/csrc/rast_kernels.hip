@@ -145,6 +145,32 @@ __device__ __forceinline__ DevTexture ldg(const DevTexture *p)
     return t;
 }
 
+// Scalar loads of what no running kernel writes (the launch's tables), from an
+// address that is the same for the wave.
+template <typename T>
+__device__ __forceinline__ T ldc(const T *p)
+{
+    return *(const __attribute__((address_space(4))) T *)(uint64_t)p;
+}
+
+__device__ __forceinline__ DevTexture ldc(const DevTexture *p)
+{
+    const u32x4_t v = *(const __attribute__((address_space(4))) u32x4_t *)(uint64_t)p;
+    DevTexture t;
+    t.texels = reinterpret_cast<const uint32_t *>(((uint64_t)v.y << 32) | v.x);
+    t.w = v.z;
+    t.h = v.w;
+    return t;
+}
+
+// The element at a 32-bit byte offset from a base that is the same for the
+// wave: the base stays in scalar registers and no 64-bit address is formed.
+template <typename T>
+__device__ __forceinline__ T ldo(const T *base, uint32_t off)
+{
+    return ldg(reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + off));
+}
+
 template <typename T>
 __device__ __forceinline__ __attribute__((address_space(1))) T *gptr(T *p)
 {
@@ -1669,7 +1695,7 @@ __device__ __forceinline__ void rank_sort(uint64_t *v, uint32_t n, uint32_t tid)
 // (1 point, 2 linear sampling): the tile's pixels are shaded right after,
 // from the visibility the lanes hold (jobs with that sampling mode and a
 // shading stage).
-template <bool kLinear, bool kSplit>
+template <bool kLinear, bool kSplit, bool kFar>
 __device__ __forceinline__ void shade_pixel(const DevMesh *__restrict__ meshes, const JobDesc &J, const float *unit,
                                             uint32_t x, uint32_t y, uint32_t id);
 
@@ -2172,7 +2198,7 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, ui
         if (J.nblocks[ST_SHADE] && (fp.sample_state != 0) == (SHADE == 2)) {
 #pragma unroll
             for (int q = 0; q < PPT; ++q)
-                if (inside[q]) shade_pixel<SHADE == 2, false>(meshes, J, unit, (uint32_t)pxs[q], (uint32_t)pys[q],
+                if (inside[q]) shade_pixel<SHADE == 2, false, true>(meshes, J, unit, (uint32_t)pxs[q], (uint32_t)pys[q],
                                                        ~(uint32_t)best[q] - 1u);
         }
     }
@@ -2244,7 +2270,7 @@ __device__ __forceinline__ Taps texel_taps(const DevTexture &t, float u, float v
     const bool okx = texel_coord(u, t.w, x), oky = texel_coord(v, t.h, y);
     k.ok = okx && oky;
     const int w = (int)t.w, size = w * (int)t.h;
-    k.c = k.ok ? x + y * w : 0;
+    k.c = k.ok ? x + (int)__umul24((uint32_t)y, (uint32_t)w) : 0;  // both below 2^15
     k.n[0] = k.c - 1 < 0 ? k.c : k.c - 1;
     k.n[1] = k.c + 1 >= size ? k.c : k.c + 1;
     k.n[2] = k.c + w >= size ? k.c : k.c + w;
@@ -2464,6 +2490,13 @@ __device__ __forceinline__ uint32_t light_pixel_exact(const MapColours &c, float
     return pack_rgba(outr, outg, outb);
 }
 
+// Byte offset of vertex i's 48-byte attribute record, where 32 bits hold it
+// (kFar = false: far_records): a wave addresses the records from a scalar base,
+// without the quarter-rate 64-bit multiplies.  With the wave-uniform mesh's
+// fields read by scalar loads: 8K terrain 285 -> 279 us, 4K 78.4 -> 76.4, 7
+// views 165 -> 161.
+__device__ __forceinline__ uint32_t vertex_offset(uint32_t i) { return ((i << 1) + i) << 4; }
+
 // PS_Kernel + ShadePixelUnsafe (CCR/CUDARenderer.cu:833-897, CCR/CUDAROPs.cu:472-514)
 // with the attribute interpolation of RasterizePixelAtomic (CCR/CUDAROPs.cu:347-380)
 // for pixel (x, y) of the triangle whose setup record quads are q0, q1, q3.
@@ -2480,7 +2513,7 @@ __device__ __forceinline__ uint32_t light_pixel_exact(const MapColours &c, float
 // texture table is read with scalar loads, and when its four maps have one
 // size the texel indices are computed once and the texels come from the
 // maps' interleaved copy (one 16-byte load per tap).
-template <bool kLinear, bool kExact, bool kSplit>
+template <bool kLinear, bool kExact, bool kSplit, bool kFar>
 __device__ __forceinline__ void shade_body(const DevMesh *__restrict__ meshes, const JobDesc &J, const float *unit,
                                            uint32_t x, uint32_t y, const uint4 q0, const uint4 q1, const uint4 q3)
 {
@@ -2489,7 +2522,7 @@ __device__ __forceinline__ void shade_body(const DevMesh *__restrict__ meshes, c
     const float *__restrict__ depth = J.depth;
     const float4 *__restrict__ attr = J.attr;
     uint32_t *__restrict__ rgba = J.rgba;
-    const size_t pid = (size_t)y * fp.width + x;
+    const uint32_t pid = y * fp.width + x;  // below 2^28
     const float sx0 = __uint_as_float(q0.x), sy0 = __uint_as_float(q0.y);
     const float sx1 = __uint_as_float(q0.z), sy1 = __uint_as_float(q0.w);
     const float sx2 = __uint_as_float(q1.x), sy2 = __uint_as_float(q1.y);
@@ -2500,10 +2533,18 @@ __device__ __forceinline__ void shade_body(const DevMesh *__restrict__ meshes, c
     float4 a00, a10, a20, a01, a11, a21, a02, a12, a22;
     const float4 *__restrict__ sattr = J.sattr;
     if constexpr (kSplit) {
-        const float4 *S0 = sattr + (size_t)q3.x * 2, *S1 = sattr + (size_t)q3.y * 2, *S2 = sattr + (size_t)q3.z * 2;
-        const float4 s00 = ldg(S0), s10 = ldg(S1), s20 = ldg(S2);
-        const float4 s01 = ldg(S0 + 1), s11 = ldg(S1 + 1), s21 = ldg(S2 + 1);
-        const float4 v0 = ldg(attr + q3.x), v1 = ldg(attr + q3.y), v2 = ldg(attr + q3.z);
+        float4 s00, s10, s20, s01, s11, s21, v0, v1, v2;
+        if constexpr (kFar) {
+            const float4 *S0 = sattr + (size_t)q3.x * 2, *S1 = sattr + (size_t)q3.y * 2, *S2 = sattr + (size_t)q3.z * 2;
+            s00 = ldg(S0); s10 = ldg(S1); s20 = ldg(S2);
+            s01 = ldg(S0 + 1); s11 = ldg(S1 + 1); s21 = ldg(S2 + 1);
+            v0 = ldg(attr + q3.x); v1 = ldg(attr + q3.y); v2 = ldg(attr + q3.z);
+        } else {
+            const uint32_t o0 = q3.x * 32u, o1 = q3.y * 32u, o2 = q3.z * 32u;
+            s00 = ldo(sattr, o0); s10 = ldo(sattr, o1); s20 = ldo(sattr, o2);
+            s01 = ldo(sattr + 1, o0); s11 = ldo(sattr + 1, o1); s21 = ldo(sattr + 1, o2);
+            v0 = ldo(attr, q3.x * 16u); v1 = ldo(attr, q3.y * 16u); v2 = ldo(attr, q3.z * 16u);
+        }
         auto q0of = [](float4 a, float4 b, float4 vw) {
             return make_float4(a.x * vw.x, a.y * vw.x, vw.x, a.z * vw.x);
         };
@@ -2514,11 +2555,16 @@ __device__ __forceinline__ void shade_body(const DevMesh *__restrict__ meshes, c
         a00 = q0of(s00, s01, v0); a10 = q0of(s10, s11, v1); a20 = q0of(s20, s21, v2);
         a01 = q1of(s00, s01, v0); a11 = q1of(s10, s11, v1); a21 = q1of(s20, s21, v2);
         a02 = q2of(s00, s01, v0); a12 = q2of(s10, s11, v1); a22 = q2of(s20, s21, v2);
-    } else {
+    } else if constexpr (kFar) {
         const float4 *A0 = attr + (size_t)q3.x * 3, *A1 = attr + (size_t)q3.y * 3, *A2 = attr + (size_t)q3.z * 3;
         a00 = ldg(A0); a10 = ldg(A1); a20 = ldg(A2);
         a01 = ldg(A0 + 1); a11 = ldg(A1 + 1); a21 = ldg(A2 + 1);
         a02 = ldg(A0 + 2); a12 = ldg(A1 + 2); a22 = ldg(A2 + 2);
+    } else {
+        const uint32_t o0 = vertex_offset(q3.x), o1 = vertex_offset(q3.y), o2 = vertex_offset(q3.z);
+        a00 = ldo(attr, o0); a10 = ldo(attr, o1); a20 = ldo(attr, o2);
+        a01 = ldo(attr + 1, o0); a11 = ldo(attr + 1, o1); a21 = ldo(attr + 1, o2);
+        a02 = ldo(attr + 2, o0); a12 = ldo(attr + 2, o1); a22 = ldo(attr + 2, o2);
     }
     const uint32_t me = q3.w & 0x7FFFFFFFu;  // bit 31: the exact-shading mark
     const uint32_t mi = me - J.mesh0 < fp.num_meshes ? me : J.mesh0;  // entry in the launch's mesh table
@@ -2533,9 +2579,11 @@ __device__ __forceinline__ void shade_body(const DevMesh *__restrict__ meshes, c
     if (uniform) {
         const DevMesh &M = meshes[mi0];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) stex[k] = M.tex[k];
-        texq = M.texq;
-        has_diffuse = M.has_diffuse;
+        for (int k = 0; k < 4; ++k) stex[k] = ldc(M.tex + k);
+        texq = ldc(&M.texq);
+        // (as an ordinary load the compiler merges this one with the other
+        // branch's into one per-lane load, which every pixel then waits for)
+        has_diffuse = ldc(&M.has_diffuse);
     } else {
         has_diffuse = ldg(&meshes[mi].has_diffuse);
     }
@@ -2608,28 +2656,35 @@ __device__ __forceinline__ void shade_body(const DevMesh *__restrict__ meshes, c
 // triangle's setup record and runs the fused or the exact shading body as
 // setup marked the triangle (two separate code paths, so the rare exact one
 // does not raise the register count of the fused one).
-template <bool kLinear, bool kSplit>
+template <bool kLinear, bool kSplit, bool kFar>
 __device__ __forceinline__ void shade_pixel(const DevMesh *__restrict__ meshes, const JobDesc &J, const float *unit,
                                             uint32_t x, uint32_t y, uint32_t id)
 {
     const FrameParams &fp = J.fp;
     if (id >= fp.num_tris) {
-        stg(J.rgba + (size_t)y * fp.width + x, (uint32_t)(fp.visualisation == 0 ? fp.clear_rgba : 0xFF000000u));
+        stg(J.rgba + (y * fp.width + x), (uint32_t)(fp.visualisation == 0 ? fp.clear_rgba : 0xFF000000u));
         return;
     }
-    const uint4 *rp = reinterpret_cast<const uint4 *>(J.trirec + (size_t)id * kTriRecWords);
-    const uint4 q0 = ldg(rp), q1 = ldg(rp + 1), q3 = ldg(rp + 3);  // q2 holds z2, z1 and the bbox
-    if (q3.w >> 31) shade_body<kLinear, true, kSplit>(meshes, J, unit, x, y, q0, q1, q3);
-    else shade_body<kLinear, false, kSplit>(meshes, J, unit, x, y, q0, q1, q3);
+    // quads 0, 1 and 3 of the record (q2 holds z2, z1 and the bbox)
+    const uint4 *rec = reinterpret_cast<const uint4 *>(J.trirec);
+    uint4 q0, q1, q3;
+    if constexpr (kFar) {
+        const uint4 *rp = rec + (size_t)id * (kTriRecWords / 4);
+        q0 = ldg(rp); q1 = ldg(rp + 1); q3 = ldg(rp + 3);
+    } else {
+        q0 = ldo(rec, id << 6); q1 = ldo(rec + 1, id << 6); q3 = ldo(rec + 3, id << 6);
+    }
+    if (q3.w >> 31) shade_body<kLinear, true, kSplit, kFar>(meshes, J, unit, x, y, q0, q1, q3);
+    else shade_body<kLinear, false, kSplit, kFar>(meshes, J, unit, x, y, q0, q1, q3);
 }
 
 
 // A block shades 64 x kShadeRows pixels: lane x of wave w takes the pixels
 // (x, w), (x, w + 4), ...  The vis reads of all of them go out first, so each
 // further pixel of a lane waits for three dependent gathers instead of four.
-template <bool kLinear, bool kSplit>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kSplit && !kLinear ? 8 : 1))) void k_shade(const DevMesh *__restrict__ meshes, const JobDesc *__restrict__ jobs,
-                                               const uint16_t *__restrict__ table)
+template <bool kLinear, bool kSplit, bool kFar>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kSplit && !kLinear && !kFar ? 8 : 1))) void k_shade(
+    const DevMesh *__restrict__ meshes, const JobDesc *__restrict__ jobs, const uint16_t *__restrict__ table)
 {
     __shared__ float unit[256];
     unit[threadIdx.x] = byte_unit(threadIdx.x);
@@ -2637,9 +2692,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kSplit && !
     uint32_t local;
     const JobDesc &J = jobs[job_of(table, jobs, ST_SHADE, local)];
     const FrameParams &fp = J.fp;
-    // another instance shades this frame: the other sampling mode's, or the
-    // one for the other attribute layout
-    if ((fp.sample_state != 0) != kLinear || (J.sattr != nullptr) != kSplit) return;
+    // another instance shades this frame: the other sampling mode's, or one
+    // for the other attribute layout or the other reach
+    if ((fp.sample_state != 0) != kLinear || (J.sattr != nullptr) != kSplit || far_records(fp) != kFar) return;
     // the frame's counters are final once resolve has run: the job's first
     // block copies them to the renderer's pinned host block (k_publish does
     // this for jobs that are not shaded)
@@ -2656,11 +2711,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kSplit && !
 #pragma unroll
     for (int k = 0; k < P; ++k) {
         const uint32_t y = y0 + 4u * k;
-        ids[k] = y < fp.height ? ldg(J.vis + (size_t)y * fp.width + x) : 0u;
+        ids[k] = y < fp.height ? ldo(J.vis, (y * fp.width + x) * 4u) : 0u;
     }
 #pragma unroll
     for (int k = 0; k < P; ++k)
-        if (y0 + 4u * k < fp.height) shade_pixel<kLinear, kSplit>(meshes, J, unit, x, y0 + 4u * k, ids[k]);
+        if (y0 + 4u * k < fp.height) shade_pixel<kLinear, kSplit, kFar>(meshes, J, unit, x, y0 + 4u * k, ids[k]);
 }
 
 // The persistent form of the resolve stage (the reference's TODO at
@@ -2960,21 +3015,19 @@ hipError_t launch_upload(void *dst, const void *src, size_t bytes, hipStream_t s
 hipError_t launch_shade(const Launch &L, hipStream_t s)
 {
     if (!L.grid[ST_SHADE] || L.fused_shade) return hipSuccess;
-    // one instance per sampling mode and attribute layout present: a mode's
-    // code alone keeps the register count (and so the waves per SIMD) of that
-    // instance
-    if (L.shade_modes & 1u)
-        hipLaunchKernelGGL((k_shade<false, false>), dim3(L.grid[ST_SHADE]), dim3(256), 0, s, L.meshes, L.jobs,
-                           L.table[ST_SHADE]);
-    if (L.shade_modes & 2u)
-        hipLaunchKernelGGL((k_shade<true, false>), dim3(L.grid[ST_SHADE]), dim3(256), 0, s, L.meshes, L.jobs,
-                           L.table[ST_SHADE]);
-    if (L.shade_modes & 4u)
-        hipLaunchKernelGGL((k_shade<false, true>), dim3(L.grid[ST_SHADE]), dim3(256), 0, s, L.meshes, L.jobs,
-                           L.table[ST_SHADE]);
-    if (L.shade_modes & 8u)
-        hipLaunchKernelGGL((k_shade<true, true>), dim3(L.grid[ST_SHADE]), dim3(256), 0, s, L.meshes, L.jobs,
-                           L.table[ST_SHADE]);
+    // one instance per sampling mode, attribute layout and reach present: a
+    // mode's code alone keeps the register count (and so the waves per SIMD) of
+    // that instance
+    const dim3 g(L.grid[ST_SHADE]), b(256);
+    const uint16_t *t = L.table[ST_SHADE];
+    if (L.shade_modes & 0x01u) hipLaunchKernelGGL((k_shade<false, false, false>), g, b, 0, s, L.meshes, L.jobs, t);
+    if (L.shade_modes & 0x02u) hipLaunchKernelGGL((k_shade<true, false, false>), g, b, 0, s, L.meshes, L.jobs, t);
+    if (L.shade_modes & 0x04u) hipLaunchKernelGGL((k_shade<false, true, false>), g, b, 0, s, L.meshes, L.jobs, t);
+    if (L.shade_modes & 0x08u) hipLaunchKernelGGL((k_shade<true, true, false>), g, b, 0, s, L.meshes, L.jobs, t);
+    if (L.shade_modes & 0x10u) hipLaunchKernelGGL((k_shade<false, false, true>), g, b, 0, s, L.meshes, L.jobs, t);
+    if (L.shade_modes & 0x20u) hipLaunchKernelGGL((k_shade<true, false, true>), g, b, 0, s, L.meshes, L.jobs, t);
+    if (L.shade_modes & 0x40u) hipLaunchKernelGGL((k_shade<false, true, true>), g, b, 0, s, L.meshes, L.jobs, t);
+    if (L.shade_modes & 0x80u) hipLaunchKernelGGL((k_shade<true, true, true>), g, b, 0, s, L.meshes, L.jobs, t);
     return hipGetLastError();
 }
 
