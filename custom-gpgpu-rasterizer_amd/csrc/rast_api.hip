@@ -343,7 +343,7 @@ extern "C" int rast_renderer_destroy(rast_renderer *r)
     }
     DBuf *bufs[] = { &r->pos4, &r->attr, &r->trirec,
                      &r->alive, &r->survivors, &r->tile_count[0], &r->tile_count[1], &r->tile_off, &r->tile_cap,
-                     &r->tile_pool, &r->tile_cursor, &r->tile_min_depth[0], &r->tile_min_depth[1], &r->keys,
+                     &r->tile_pool, &r->tile_cursor, &r->tile_keys, &r->tile_min_depth[0], &r->tile_min_depth[1], &r->keys,
                      &r->queue, &r->pool, &r->big, &r->bigp, &r->bige, &r->ovf, &r->vis, &r->depth,
                      &r->rgba };
     for (DBuf *b : bufs) dfree(*b);
@@ -661,6 +661,7 @@ static int ensure_frame_storage(rast_renderer *r, uint32_t ntiles)
     HIP_TRY(grow(r, r->tile_cap, tb, &synced));
     HIP_TRY(grow(r, r->tile_pool, tb, &synced));
     HIP_TRY(grow(r, r->tile_cursor, tb, &synced));
+    HIP_TRY(grow(r, r->tile_keys, tb, &synced));
     if (r->queue_cap == 0) r->queue_cap = std::max<uint32_t>(1u << 20, std::min<uint64_t>(4ull * nt, 0x7FFFFFFFull));
     // room for fixed regions (fixed_stride) in frames of many tiles: 4 KB a tile, up to 256 MB
     r->queue_cap = std::max<uint32_t>(r->queue_cap, std::min<uint64_t>((uint64_t)ntiles * kFixedRegion, 1u << 26));
@@ -1124,6 +1125,7 @@ static int stage_launch(LaunchPlan &P, rast_renderer *const *rs, uint32_t n)
         J.tile_cap = (uint32_t *)r->tile_cap.p;
         J.tile_pool = (uint32_t *)r->tile_pool.p;
         J.tile_cursor = (uint32_t *)r->tile_cursor.p;
+        J.tile_keys = (uint32_t *)r->tile_keys.p;
         J.prev_count = (const uint32_t *)r->tile_count[r->cur ^ 1].p;
         J.prev_depth = (const float *)r->tile_min_depth[r->cur ^ 1].p;
         J.queue = (uint32_t *)r->queue.p;

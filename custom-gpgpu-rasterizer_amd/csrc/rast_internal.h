@@ -183,6 +183,7 @@ struct alignas(16) JobDesc {  // 16-byte multiple: staged in 16-byte words
     // every block serializes those updates at its cache line.
     uint32_t *alive_part;
     uint32_t alive_part0, alive_parts;
+    uint32_t *tile_keys;         // per tile: 1 where micro triangles may have written keys
     float *tile_min_depth;       // per tile min depth written by the resolve pass
     unsigned long long *keys;    // per pixel (z << 32 | ~(id + 1)), reset to depth 1 / none after each resolve
     uint32_t *vis;

@@ -602,6 +602,7 @@ __device__ __forceinline__ void frame_init_block(const JobDesc *__restrict__ job
     const uint32_t i = local * 256u + threadIdx.x;
     if (i < n) {
         J.tile_count[i] = 0;
+        J.tile_keys[i] = 0;
         J.tile_min_depth[i] = 1.0f;
         if (J.single && !J.learned && !J.stride) J.tile_pool[i] = 0xFFFFFFFFu;
     }
@@ -1182,6 +1183,15 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
             uint32_t *wo = moff + wave * 64;
             unsigned long long *wm = mmask + wave * kMaskChunks;
             if (items) {
+                // the tiles whose keys this triangle can touch: mostly one
+                const uint32_t sh = (uint32_t)__builtin_ctz(fp.tile);
+                const uint32_t kx0 = (uint32_t)mx0 >> sh, ky0 = (uint32_t)my0 >> sh;
+                stg(J.tile_keys + (__umul24(ky0, fp.tiles_x) + kx0), 1u);
+                if ((uint32_t)((mx0 ^ (xmax - 1)) | (my0 ^ (ymax - 1))) >> sh) {
+                    const uint32_t kx1 = (uint32_t)(xmax - 1) >> sh, ky1 = (uint32_t)(ymax - 1) >> sh;
+                    for (uint32_t ky = ky0; ky <= ky1; ++ky)
+                        for (uint32_t kx = kx0; kx <= kx1; ++kx) stg(J.tile_keys + ky * fp.tiles_x + kx, 1u);
+                }
                 MicroLds m;
                 m.sx0 = t.sx0; m.sy0 = t.sy0; m.sx1 = t.sx1; m.sy1 = t.sy1; m.sx2 = t.sx2; m.sy2 = t.sy2;
                 m.z0 = t.z0; m.z1 = t.z1; m.z2 = t.z2; m.area = t.area;
@@ -1766,6 +1776,19 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, ui
     constexpr int BH = 64 * PPT / T;
     const int p0 = (int)(wave * 64u * PPT + lane);
     const int Y0w = Y0 + (int)wave * BH;
+    // the tile's words, all written by earlier launches: scalar loads, in flight
+    // together
+    const uint32_t cnt = ldc(tile_count + tile);
+    const bool micro = ldc(J.tile_keys + tile) != 0u;
+    uint32_t n_big = ldc(&ctr->num_big);
+    uint32_t qoff, cp = 0xFFFFFFFFu;
+    if (J.single && J.stride) {
+        qoff = tile * J.stride;
+        cp = J.stride;
+    } else {
+        qoff = ldc(tile_off + tile);
+        if (J.single) cp = ldc(J.tile_cap + tile);
+    }
     uint64_t best[PPT];
     int pxs[PPT], pys[PPT];
     bool inside[PPT];
@@ -1776,7 +1799,10 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, ui
         pys[q] = Y0 + p / T;
         inside[q] = pxs[q] < (int)fp.width && pys[q] < (int)fp.height;
         best[q] = kClearKey;
-        if (inside[q]) {
+        // keys that no micro triangle can have touched are clear: neither read
+        // nor reset (8K terrain: resolve 259 -> 226 us; where most tiles hold
+        // micro triangles the saving pays for the marks, 2 us each way at 4K)
+        if (micro && inside[q]) {
             const size_t o = (size_t)pys[q] * fp.width + pxs[q];
             best[q] = ldg(keys + o);
             stg(keys + o, (unsigned long long)kClearKey);
@@ -1792,16 +1818,7 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, ui
     // fallback passes placed them in the tile's pool region.  The order of a
     // tile's entries does not change the frame (the depth keys order
     // fragments by depth, then ID).
-    const uint32_t cnt = ldg(tile_count + tile);
     uint32_t n_a = cnt, n_b = 0;
-    uint32_t qoff, cp = 0xFFFFFFFFu;
-    if (J.single) {
-        const uint2 g = tile_region(J, tile);
-        qoff = g.x;
-        cp = g.y;
-    } else {
-        qoff = ldg(tile_off + tile);
-    }
     const uint32_t *list_a = queue + qoff;
     const uint32_t *list_b = pool;
     if (J.single) {
@@ -2049,7 +2066,6 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, ui
     // a tile 200 of them (up to 700), of which a wave runs 20 to 50 (up to 240):
     // with these, the rows bounded per wave and the small frames' tiles first, the
     // 7-view resolve went 298 -> 251 us.
-    uint32_t n_big = ldg(&ctr->num_big);
     n_big = n_big < big_cap ? n_big : big_cap;
     if (n_big) {
         auto wave_max_depth = [&]() {
