@@ -73,6 +73,15 @@ int resolve_resident_blocks(int stage, int fused_shade);
 hipError_t launch_shade(const Launch &L, hipStream_t s);
 // Copies a staging block (a multiple of 16 bytes) from pinned host memory.
 hipError_t launch_upload(void *dst, const void *src, size_t bytes, hipStream_t s);
+// Copies of device memory to the host in pieces of up to kReadPiece bytes (a
+// multiple of 4; both ends 16-byte aligned), through kReadSlots pinned slots:
+// flags[i], in coherent host memory, becomes epoch once chunk i (kReadChunk
+// bytes) of the piece is there.  count: kReadChunks words of device memory, zero
+// before and after.
+constexpr size_t kReadChunk = 256u << 10, kReadPiece = 8u << 20;
+constexpr uint32_t kReadChunks = (uint32_t)(kReadPiece / kReadChunk), kReadSlots = 2;
+hipError_t launch_read_out(const void *src, void *dst, size_t bytes, uint32_t *count, uint32_t *flags, uint32_t epoch,
+                           hipStream_t s);
 hipError_t launch_publish(const Launch &L, hipStream_t s);
 // Placement of the previous-frame policy's entries beyond capacity.
 hipError_t launch_fallback(const Launch &L, hipStream_t s);
