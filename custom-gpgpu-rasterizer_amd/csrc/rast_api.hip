@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstring>
 #include <atomic>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <string>
@@ -311,6 +312,7 @@ static void orphan_mesh(rast_mesh *m)
     m->ivert14 = nullptr;
     m->idx = nullptr;
     m->boxes = nullptr;
+    m->reach = nullptr;
     for (auto &t : m->tex) t = nullptr;
     m->texq = nullptr;
     m->r = nullptr;
@@ -450,12 +452,15 @@ extern "C" int rast_mesh_create(rast_renderer *r, const rast_ivertex *verts, uin
     for (int i = 0; i < 16; ++i) m->world[i] = world ? world[i] : ((i % 5 == 0) ? 1.f : 0.f);
     hipError_t e = hipMalloc((void **)&m->ivert14, v14.size() * sizeof(float));
     const size_t idx_bytes = ((size_t)num_indices * 4 + 15) & ~(size_t)15;
-    if (e == hipSuccess) e = hipMalloc((void **)&m->idx, idx_bytes + (size_t)ceil_div(ntri, 256) * 32);
+    const size_t box_bytes = (size_t)ceil_div(ntri, 256) * 32, reach_bytes = (size_t)ceil_div(num_verts, kVertexChunk) * 32;
+    if (e == hipSuccess) e = hipMalloc((void **)&m->idx, idx_bytes + box_bytes + reach_bytes);
     if (e == hipSuccess) e = hipMemcpy(m->ivert14, v14.data(), v14.size() * sizeof(float), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(m->idx, indices, (size_t)num_indices * 4, hipMemcpyHostToDevice);
     if (e == hipSuccess) {  // on the copies' stream; done before any frame's stream can read them
         m->boxes = reinterpret_cast<float4 *>(reinterpret_cast<char *>(m->idx) + idx_bytes);
-        e = launch_mesh_boxes(m->ivert14, m->idx, ntri, topology, m->boxes, nullptr);
+        m->reach = reinterpret_cast<uint4 *>(reinterpret_cast<char *>(m->boxes) + box_bytes);
+        e = launch_mesh_boxes(m->ivert14, m->idx, ntri, topology, m->boxes, m->reach, ceil_div(num_verts, kVertexChunk),
+                              nullptr);
     }
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) {
@@ -469,6 +474,8 @@ extern "C" int rast_mesh_create(rast_renderer *r, const rast_ivertex *verts, uin
     *out = m;
     return RAST_OK;
 }
+
+static int complete_debug(rast_renderer *r);
 
 extern "C" int rast_mesh_destroy(rast_mesh *m)
 {
@@ -484,6 +491,13 @@ extern "C" int rast_mesh_destroy(rast_mesh *m)
         HIP_TRY(renderer_wait(v));
         v->have_prev = false;
     }
+    // the last frames' debug buffers are completed while the mesh is there (as
+    // far as there is memory for it)
+    (void)complete_debug(r);
+    for (rast_renderer *v : r->views) (void)complete_debug(v);
+    r->frame_scene.reset();
+    for (rast_renderer *v : r->views) v->frame_scene.reset();
+    r->drawn.reset();
     r->meshes.erase(std::remove(r->meshes.begin(), r->meshes.end(), m), r->meshes.end());
     free_mesh(m);
     ++r->scene_version;
@@ -496,6 +510,7 @@ extern "C" int rast_mesh_set_world(rast_mesh *m, const float world[16])
 {
     if (!m || !world) return rast_set_error(RAST_E_INVALID_ARG, "rast_mesh_set_world: null argument");
     memcpy(m->world, world, sizeof m->world);
+    if (m->r) ++m->r->world_version;
     return RAST_OK;
 }
 
@@ -744,10 +759,37 @@ static int ensure_tex_quads(rast_renderer *r)
     return RAST_OK;
 }
 
+// Notes the scene as the next frame draws it (made again only when it has
+// changed; the views of a scene share it).
+static std::mutex g_drawn_mutex;
+
+static int note_scene(rast_renderer *r)
+{
+    rast_renderer *o = scene_owner(r);
+    std::lock_guard<std::mutex> lock(g_drawn_mutex);
+    if (!o->drawn || o->drawn_scene != o->scene_version || o->drawn_world != o->world_version) {
+        try {
+            auto v = std::make_shared<std::vector<FrameMesh>>(o->meshes.size());
+            for (size_t i = 0; i < v->size(); ++i) {
+                (*v)[i].m = o->meshes[i];
+                memcpy((*v)[i].world, o->meshes[i]->world, sizeof (*v)[i].world);
+            }
+            o->drawn = std::move(v);
+        } catch (const std::bad_alloc &) {
+            return rast_set_error(RAST_E_OUT_OF_MEMORY, "host allocation failed");
+        }
+        o->drawn_scene = o->scene_version;
+        o->drawn_world = o->world_version;
+    }
+    r->next_scene = o->drawn;
+    return RAST_OK;
+}
+
 static int prepare_job(rast_renderer *r)
 {
     HIP_TRY(hipSetDevice(r->device));
     if (scene_meshes(r).empty()) return rast_set_error(RAST_E_STATE, "rast_render: no meshes loaded");
+    RAST_TRY(note_scene(r));
     if (r->layout_version != scene_owner(r)->scene_version) refresh_layout(r);
     RAST_TRY(ensure_tex_quads(r));
     const uint32_t ntiles = ceil_div(r->W, r->tile) * ceil_div(r->H, r->tile);
@@ -816,6 +858,7 @@ void plan_free(LaunchPlan &p)
     }
     dfree(p.d_block_mesh);
     dfree(p.d_alive_part);
+    dfree(p.d_chunk_views);
     dfree(p.d_tables);
     dfree(p.d_stage);
     dfree(p.d_sattr);
@@ -839,6 +882,8 @@ static int plan_wait(LaunchPlan &P)
     RAST_TRY(plan_wait_block(P, 0));
     return plan_wait_block(P, 1);
 }
+
+constexpr uint64_t kViewChunks = 16384;
 
 static int dev_alloc(DBuf &b, size_t bytes)
 {
@@ -992,6 +1037,18 @@ static int build_plan(LaunchPlan &P, rast_renderer *const *rs, uint32_t n, int h
     RAST_TRY(dev_alloc(P.d_alive_part, ((size_t)L.tri_blocks + 1) * 4));
     uint32_t *bm = (uint32_t *)P.d_block_mesh.p;
     if (!tab.empty()) HIP_TRY(hipMemcpy(bm, tab.data(), tab.size() * 4, hipMemcpyHostToDevice));
+    // Views of large scenes: a vertex chunk is transformed for the views it may be
+    // in only.  The test is a launch of its own, 5 to 9 us, so it takes a vertex
+    // pass that is several times that (7 views of 1.35 M vertices, 74 K chunks to
+    // transform: 110 -> 9 + 64 us; 12 views of a small object, 3.8 K chunks: 15 us
+    // in all).  A frame of one view mostly sees its scene.
+    uint64_t view_chunks = 0;
+    for (uint32_t g : vs_group)
+        if (members[g].size() > 1) view_chunks += members[g].size();
+    if (view_chunks >= kViewChunks) {
+        RAST_TRY(dev_alloc(P.d_chunk_views, vs_group.size() * 8));
+        L.chunk_views = (uint64_t *)P.d_chunk_views.p;
+    }
     L.vs_block_group = bm;
     L.tri_block_mesh = bm + vs_group.size();
     L.vs_groups = reinterpret_cast<const uint2 *>(bm + groups_at);
@@ -1065,6 +1122,38 @@ static int build_plan(LaunchPlan &P, rast_renderer *const *rs, uint32_t n, int h
     return RAST_OK;
 }
 
+// A mesh's entry: its geometry and matrices (not its textures).
+static void fill_mesh(DevMesh &d, const rast_mesh *m, const float *world, const rast_frame_consts &fc, uint32_t vert_base,
+                      uint32_t tri_base, uint32_t vs_block0, uint32_t tri_block0)
+{
+    memset(&d, 0, sizeof d);
+    d.ivert = m->ivert14;
+    d.boxes = m->boxes;
+    d.reach = m->reach;
+    d.idx = m->idx;
+    d.num_verts = m->nv;
+    d.num_tris = m->ntri;
+    d.vert_base = vert_base;
+    d.tri_base = tri_base;
+    d.vs_block0 = vs_block0;
+    d.tri_block0 = tri_block0;
+    d.topology = m->topology;
+    d.has_diffuse = m->tex[0] != nullptr;
+    // the rotated normal / tangent stays below attr_max times the
+    // largest row sum of the world matrix's 3x3 part
+    float rowsum = 0.f;
+    for (int row = 0; row < 3; ++row)
+        rowsum = std::max(rowsum, std::fabs(M4c(world, row, 0)) + std::fabs(M4c(world, row, 1)) +
+                                      std::fabs(M4c(world, row, 2)));
+    d.shade_exact = !(m->attr_max * rowsum <= 4.f);
+    mat4_mul(fc.viewproj, world, d.wvp);  // CCR/CUDARenderer.cu:241
+    memcpy(d.world, world, sizeof d.world);
+    for (int q = 0; q < 3; ++q) {
+        d.cam_pos[q] = fc.cam_pos[q];
+        d.cam_fwd[q] = fc.cam_fwd[q];
+    }
+}
+
 // Writes every job's descriptor and mesh entries (this frame's cameras,
 // options and buffer parities) into the staging block of the next launch,
 // once the launch before last, which used it, is done.
@@ -1119,7 +1208,7 @@ static int stage_launch(LaunchPlan &P, rast_renderer *const *rs, uint32_t n)
         J.defaults[3] = o.default_gloss;
         J.model = J.learned ? rast_model_params(r->model) : nullptr;
         J.pos4 = (float4 *)r->pos4.p;
-        J.attr = (float4 *)r->attr.p;
+        J.attr = job_shades(r) || P.sattr_off[j] != SIZE_MAX ? (float4 *)r->attr.p : nullptr;
         J.trirec = (uint32_t *)r->trirec.p;
         J.alive = (uint8_t *)r->alive.p;
         J.tile_count = (uint32_t *)r->tile_count[r->cur].p;
@@ -1161,32 +1250,8 @@ static int stage_launch(LaunchPlan &P, rast_renderer *const *rs, uint32_t n)
         for (size_t i = 0; i < meshes.size(); ++i, ++me) {
             const rast_mesh *m = meshes[i];
             DevMesh &d = dm[me];
-            memset(&d, 0, sizeof d);
-            d.ivert = m->ivert14;
-            d.boxes = m->boxes;
-            d.idx = m->idx;
-            d.num_verts = m->nv;
-            d.num_tris = m->ntri;
-            d.vert_base = vb;
-            d.tri_base = (uint32_t)m->tri_base;
-            d.vs_block0 = P.vs_block0[me];
-            d.tri_block0 = P.tri_block0[me];
-            d.topology = m->topology;
-            d.has_diffuse = m->tex[0] != nullptr;
+            fill_mesh(d, m, m->world, fc, vb, (uint32_t)m->tri_base, P.vs_block0[me], P.tri_block0[me]);
             d.job = j;
-            // the rotated normal / tangent stays below attr_max times the
-            // largest row sum of the world matrix's 3x3 part
-            float rowsum = 0.f;
-            for (int row = 0; row < 3; ++row)
-                rowsum = std::max(rowsum, std::fabs(M4c(m->world, row, 0)) + std::fabs(M4c(m->world, row, 1)) +
-                                              std::fabs(M4c(m->world, row, 2)));
-            d.shade_exact = !(m->attr_max * rowsum <= 4.f);
-            mat4_mul(fc.viewproj, m->world, d.wvp);  // CCR/CUDARenderer.cu:241
-            memcpy(d.world, m->world, sizeof d.world);
-            for (int q = 0; q < 3; ++q) {
-                d.cam_pos[q] = fc.cam_pos[q];
-                d.cam_fwd[q] = fc.cam_fwd[q];
-            }
             for (int q = 0; q < 4; ++q) {
                 if (m->tex[q]) d.tex[q] = { m->tex[q]->texels, m->tex[q]->w, m->tex[q]->h };
                 else d.tex[q] = { dflt + q, 1u, 1u };
@@ -1298,6 +1363,91 @@ static void finish_enqueue(rast_renderer *r)
     r->frame_valid = false;
     r->have_prev = true;
     r->cur ^= 1;
+    r->frame_scene = std::move(r->next_scene);
+    r->frame_cam = r->last_cam;
+    r->frame_w = r->W;
+    r->frame_h = r->H;
+    r->frame_cull = r->last_opts.cull_mode;
+}
+
+// Completes the last frame's debug buffers: positions and attributes of the
+// vertices out of view, the records of the survivors that nothing of the frame
+// reads (launch_debug_fill).  r's GPU work is done.
+static int complete_debug_of(rast_renderer *r, const std::vector<FrameMesh> &ms)
+{
+    // one job, a vertex group per mesh: [job][meshes][vertex block -> group]
+    // [triangle block -> mesh][groups][entries]
+    std::vector<DevMesh> rows(ms.size());
+    std::vector<uint32_t> vs_group, tri_mesh, groups, entries;
+    rast_frame_consts fc;
+    camera_frame(r->frame_cam, r->frame_w, r->frame_h, fc);
+    JobDesc J;
+    memset(&J, 0, sizeof J);
+    uint32_t vb = 0, tb = 0;
+    for (uint32_t i = 0; i < ms.size(); ++i) {
+        const rast_mesh *m = ms[i].m;
+        fill_mesh(rows[i], m, ms[i].world, fc, vb, tb, (uint32_t)vs_group.size(), (uint32_t)tri_mesh.size());
+        vs_group.insert(vs_group.end(), ceil_div(m->nv, kVertexChunk), i);
+        tri_mesh.insert(tri_mesh.end(), ceil_div(m->ntri, 256), i);
+        groups.push_back(i);
+        groups.push_back(1u);
+        entries.push_back(i);
+        vb += m->nv;
+        tb += m->ntri;
+    }
+    // (a later frame that failed may have lost them)
+    if (r->pos4.n < (size_t)vb * 16 || r->attr.n < (size_t)vb * 48 || r->trirec.n < (size_t)tb * kTriRecWords * 4)
+        return RAST_OK;
+    J.fp.width = r->frame_w;
+    J.fp.height = r->frame_h;
+    J.fp.cull_mode = r->frame_cull;
+    J.fp.tile = 32;
+    J.fp.num_verts = vb;
+    J.fp.num_tris = tb;
+    J.pos4 = (float4 *)r->pos4.p;
+    J.attr = r->last_shared_attr ? nullptr : (float4 *)r->attr.p;  // where the frame's are in this layout
+    J.trirec = (uint32_t *)r->trirec.p;
+    std::vector<char> block;
+    auto put = [&block](const void *p, size_t n) {
+        block.resize((block.size() + 15) & ~(size_t)15);
+        const size_t at = block.size();
+        block.insert(block.end(), (const char *)p, (const char *)p + n);
+        return at;
+    };
+    const size_t at_job = put(&J, sizeof J), at_mesh = put(rows.data(), rows.size() * sizeof(DevMesh));
+    const size_t at_vs = put(vs_group.data(), vs_group.size() * 4), at_tri = put(tri_mesh.data(), tri_mesh.size() * 4);
+    const size_t at_gr = put(groups.data(), groups.size() * 4), at_en = put(entries.data(), entries.size() * 4);
+    char *d = nullptr;
+    HIP_TRY(hipMalloc((void **)&d, block.size()));
+    Launch L{};
+    L.njobs = 1;
+    L.jobs = (const JobDesc *)(d + at_job);
+    L.meshes = (const DevMesh *)(d + at_mesh);
+    L.vs_block_group = (const uint32_t *)(d + at_vs);
+    L.tri_block_mesh = (const uint32_t *)(d + at_tri);
+    L.vs_groups = (const uint2 *)(d + at_gr);
+    L.vs_entries = (const uint32_t *)(d + at_en);
+    L.vs_blocks = (uint32_t)vs_group.size();
+    L.tri_blocks = (uint32_t)tri_mesh.size();
+    hipError_t e = hipMemcpyAsync(d, block.data(), block.size(), hipMemcpyHostToDevice, r->stream);
+    if (e == hipSuccess) e = launch_debug_fill(L, r->stream);
+    const hipError_t w = hipStreamSynchronize(r->stream);
+    (void)hipFree(d);
+    HIP_TRY(e);
+    HIP_TRY(w);
+    return RAST_OK;
+}
+
+static int complete_debug(rast_renderer *r)
+{
+    if (!r->frame_scene) return RAST_OK;
+    try {
+        RAST_TRY(complete_debug_of(r, *r->frame_scene));
+    } catch (const std::bad_alloc &) {
+        return rast_set_error(RAST_E_OUT_OF_MEMORY, "host allocation failed");
+    }
+    r->frame_scene.reset();
+    return RAST_OK;
 }
 
 static int clear_keys_if_dirty(rast_renderer *r, hipStream_t s)
@@ -1584,6 +1734,8 @@ extern "C" int rast_debug_read(rast_renderer *r, int which, void *dst, size_t by
     size_t size = 0;
     const void *src = nullptr;
     std::vector<uint32_t> tmp;
+    if (dst && (which == RAST_DEBUG_VERTEX_POS || which == RAST_DEBUG_VERTEX_ATTR || which == RAST_DEBUG_TRI_RECORDS))
+        RAST_TRY(complete_debug(r));
     switch (which) {
     case RAST_DEBUG_VERTEX_POS: size = (size_t)r->total_verts * 16; src = r->pos4.p; break;
     case RAST_DEBUG_VERTEX_ATTR:

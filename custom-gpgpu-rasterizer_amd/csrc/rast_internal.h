@@ -7,7 +7,8 @@
 //   attr     4 x float4 / global vertex, each attribute times 1/w:
 //            u v 1/w n'.x | n'.yz tan'.xy | tan'.z vd | c.rgb 0
 //            (64 B; PBR shading reads the first 48 B)
-//   trirec   16 words / global triangle ID (written for survivors):
+//   trirec   16 words / global triangle ID (written for the survivors that
+//            are binned or cover a pixel; k_setup<true> writes the others'):
 //            [0..5] screen x0,y0,x1,y1,x2,y2  [6..8] z0,z1,z2  [9] |area|
 //            [10] xmin | ymin << 16  [11] xmax | ymax << 16 (pixel range
 //            [min, max)), [12..14] global vertex indices, [15] mesh index,
@@ -50,6 +51,9 @@ struct DevTexture {
 struct alignas(16) DevMesh {  // 16-byte multiple: staged in 16-byte words
     const float *ivert;       // 14 floats per vertex
     const float4 *boxes;      // object-space box (lo, hi) of every 256 triangles
+    // per kVertexChunk vertices, the box of all boxes whose triangles use one of
+    // them, as k_vertex_boxes leaves it (8 words)
+    const uint4 *reach;
     const uint32_t *idx;
     uint32_t num_verts;
     uint32_t num_tris;
@@ -153,7 +157,8 @@ struct alignas(16) JobDesc {  // 16-byte multiple: staged in 16-byte words
     // n.y | n.z t.xyz, not times 1/w), and attr one float4 per vertex per job
     // (1/w, vd.xyz times 1/w); shading forms the same products.  The vertex
     // colour (read only where a mesh has no diffuse map) is taken from the
-    // mesh's input vertices at shading, times the stored 1/w.
+    // mesh's input vertices at shading, times the stored 1/w.  A frame of its own
+    // that is not shaded: attr null.
     float4 *attr;
     float4 *sattr;
     uint32_t *trirec;

@@ -627,10 +627,12 @@ __global__ __launch_bounds__(256) void k_clear_keys(unsigned long long *__restri
 // workgroup's), formed once when the mesh is created: (lo, -), (hi, -).  A corner
 // that is not finite, or huge, makes the box unbounded (never culled).
 __global__ __launch_bounds__(256) void k_mesh_boxes(const float *__restrict__ ivert, const uint32_t *__restrict__ idx,
-                                                    uint32_t ntri, int topology, float4 *__restrict__ boxes)
+                                                    uint32_t ntri, int topology, float4 *__restrict__ boxes,
+                                                    uint32_t *__restrict__ reach, uint32_t reach_words)
 {
     __shared__ float red[4][6];
     const uint32_t k = blockIdx.x * 256u + threadIdx.x;
+    for (uint32_t i = k; i < reach_words; i += gridDim.x * 256u) stg(reach + i, 0xFFFFFFFFu);  // for k_vertex_boxes
     const float inf = __int_as_float(0x7f800000);
     float b[6] = { inf, inf, inf, inf, inf, inf };  // smallest x y z, smallest -x -y -z
     if (k < ntri) {
@@ -659,6 +661,49 @@ __global__ __launch_bounds__(256) void k_mesh_boxes(const float *__restrict__ iv
         for (int a = 0; a < 6; ++a) m[a] = fminf(fminf(red[0][a], red[1][a]), fminf(red[2][a], red[3][a]));
         stg(boxes + 2 * (size_t)blockIdx.x, make_float4(m[0], m[1], m[2], 0.f));
         stg(boxes + 2 * (size_t)blockIdx.x + 1, make_float4(-m[3], -m[4], -m[5], 0.f));
+    }
+}
+
+// Float bits that order like the values (negative values reversed), and back.
+__device__ __forceinline__ uint32_t ordered_bits(float v)
+{
+    const uint32_t b = __float_as_uint(v);
+    return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+}
+
+__device__ __forceinline__ float from_ordered(uint32_t o)
+{
+    return __uint_as_float((o & 0x80000000u) ? (o ^ 0x80000000u) : ~o);
+}
+
+// Reach of every kVertexChunk vertices, formed once after the mesh's boxes: the
+// box of all the boxes (of 256 triangles) that hold a triangle with one of the
+// vertices.  reach (8 words a chunk): the ordered bits of the smallest x y z, -x
+// -y -z, all ones at first, as they stay where no triangle uses the chunk.
+// A block's triangles share their box, so a chunk is widened about once per
+// block: LDS remembers the chunks it has met (by their low bits; one that is
+// forgotten is only widened again, to no effect).
+__global__ __launch_bounds__(256) void k_vertex_boxes(const uint32_t *__restrict__ idx, uint32_t ntri, int topology,
+                                                      const float4 *__restrict__ boxes, uint32_t *reach)
+{
+    constexpr uint32_t kMet = 1024;
+    __shared__ uint32_t met[kMet];
+    for (uint32_t i = threadIdx.x; i < kMet; i += 256u) met[i] = 0xFFFFFFFFu;
+    __syncthreads();
+    const uint32_t k = blockIdx.x * 256u + threadIdx.x;
+    if (k >= ntri) return;
+    const float4 lo = ldg(boxes + 2 * (size_t)blockIdx.x), hi = ldg(boxes + 2 * (size_t)blockIdx.x + 1);
+    const uint32_t o[6] = { ordered_bits(lo.x),  ordered_bits(lo.y),  ordered_bits(lo.z),
+                            ordered_bits(-hi.x), ordered_bits(-hi.y), ordered_bits(-hi.z) };
+#pragma unroll
+    for (uint32_t c = 0; c < 3; ++c) {
+        const uint32_t chunk = ldg(idx + (topology == 0 ? 3 * (size_t)k + c : (size_t)k + c)) / kVertexChunk;
+        if (atomicExch(&met[chunk % kMet], chunk) == chunk) continue;
+#pragma unroll
+        for (int a = 0; a < 6; ++a) {
+            uint32_t *p = reach + (size_t)chunk * 8u + a;
+            if (o[a] < ldg(p)) gatomic_min(p, o[a]);  // (an older value read here only costs an update)
+        }
     }
 }
 
@@ -728,6 +773,81 @@ __device__ __forceinline__ void cull_block(const DevMesh *__restrict__ meshes, c
     stg(ldg(&jobs[ldg(&M->job)].alive_part) + b, out ? kCulledBlock : 0u);
 }
 
+// The entries [0, min(n, 64)) of a vertex group whose view the reach [lo, hi] of a
+// chunk of its vertices may be in, as bits; a chunk out of a view is not
+// transformed for it.  Eight entries at a time, one box corner per lane, with
+// the tests of box_outside at twice its margins: then the exact values at every
+// point of the reach, within 4.0003 u S of the ones formed here, clear
+// box_outside's margins by more than its own error, so that every box inside
+// this one is culled too, and the setup pass reads no position that was not
+// written.  (box_outside's S are no larger, the boxes lying inside this one.)
+__device__ __forceinline__ uint64_t entries_in_view(const DevMesh *__restrict__ meshes,
+                                                    const uint32_t *__restrict__ entries, uint32_t n, float3 lo, float3 hi)
+{
+    const float u = 1.0f / 16777216.0f;
+    const float ax = fmaxf(fabsf(lo.x), fabsf(hi.x)), ay = fmaxf(fabsf(lo.y), fabsf(hi.y));
+    const float az = fmaxf(fabsf(lo.z), fabsf(hi.z));
+    const uint32_t lane = lane_id();
+    const float x = lane & 1u ? hi.x : lo.x, y = lane & 2u ? hi.y : lo.y, z = lane & 4u ? hi.z : lo.z;
+    n = n < 64u ? n : 64u;
+    uint64_t keep = 0;
+    for (uint32_t e0 = 0; e0 < n; e0 += 8u) {
+        const uint32_t e = e0 + (lane >> 3);
+        const float *wvp = meshes[ldg(entries + (e < n ? e : e0))].wvp;
+        float v[4], S[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float mx = ldg(wvp + r), my = ldg(wvp + 4 + r), mz = ldg(wvp + 8 + r), mw = ldg(wvp + 12 + r);
+            S[r] = fabsf(mx) * ax + fabsf(my) * ay + fabsf(mz) * az + fabsf(mw);
+            v[r] = mx * x + my * y + mz * z + mw;
+        }
+        const bool fine = S[0] < 1.0e30f && S[1] < 1.0e30f && S[2] < 1.0e30f && S[3] < 1.0e30f;
+        const float ew = 32.0f * u * S[3] + 2.0e-30f;
+        const float ex = 64.0f * u * (S[0] + S[3]), ey = 64.0f * u * (S[1] + S[3]), ez = 64.0f * u * (S[2] + S[3]);
+        const float sg = v[3] < 0.f ? -1.f : 1.f, w = fabsf(v[3]);
+        const float X = v[0] * sg, Y = v[1] * sg, Z = v[2] * sg;
+        uint32_t b = 0;  // planes this corner is beyond; bits 6, 7: w > 0, w < 0
+        b |= X + w < -ex ? 1u : 0u;
+        b |= X - w > ex ? 2u : 0u;
+        b |= Y + w < -ey ? 4u : 0u;
+        b |= Y - w > ey ? 8u : 0u;
+        b |= Z < -ez ? 16u : 0u;
+        b |= Z - w > ez ? 32u : 0u;
+        b |= v[3] > ew ? 64u : 0u;
+        b |= v[3] < -ew ? 128u : 0u;
+        // over the entry's eight corners: pairs, quads, then the quad beside
+        b &= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b, 0xB1, 0xF, 0xF, false);
+        b &= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b, 0x4E, 0xF, 0xF, false);
+        b &= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b, 0x141, 0xF, 0xF, false);
+        const uint64_t in = __ballot(e < n && !(fine && (b & 0xC0u) != 0u && (b & 0x3Fu) != 0u));
+#pragma unroll
+        for (uint32_t g = 0; g < 8; ++g) keep |= (in >> (8u * g) & 1ull) << (e0 + g);
+    }
+    return keep;
+}
+
+// The views each vertex chunk may be in, one wave per chunk, ahead of the vertex
+// launch (where the vertex workgroups tested their own chunk, the wait for the
+// matrices before the vertices were read cost more than it saved: 4K terrain
+// 26 -> 36 us, 7 views 110 -> 76).
+__global__ __launch_bounds__(256) void k_chunk_views(const DevMesh *__restrict__ meshes,
+                                                     const uint32_t *__restrict__ block_group,
+                                                     const uint2 *__restrict__ groups,
+                                                     const uint32_t *__restrict__ entries,
+                                                     uint64_t *__restrict__ chunk_views, uint32_t vs_blocks)
+{
+    const uint32_t blk = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (blk >= vs_blocks) return;
+    const uint2 gr = groups[block_group[blk]];
+    const DevMesh &M0 = meshes[entries[gr.x]];
+    const uint4 *reach = M0.reach + 2 * (size_t)(blk - M0.vs_block0);
+    const uint4 a = ldg(reach), b = ldg(reach + 1);
+    const uint64_t keep = entries_in_view(meshes, entries + gr.x, gr.y,
+                                          make_float3(from_ordered(a.x), from_ordered(a.y), from_ordered(a.z)),
+                                          make_float3(-from_ordered(a.w), -from_ordered(b.x), -from_ordered(b.y)));
+    if (lane_id() == 0) chunk_views[blk] = keep;
+}
+
 // VS_Kernel / GetNDCVertex (CCR/CUDARenderer.cu:673-700, CCR/CUDAROPs.cu:99-118).
 // A block's 256 vertices are 16 KB of input records and 16 KB of attribute
 // records per job, contiguous in HBM.  Both go through LDS so that global
@@ -740,7 +860,8 @@ __device__ __forceinline__ void vertex_block(const DevMesh *__restrict__ meshes,
                                              const uint32_t *__restrict__ block_group,
                                              const uint2 *__restrict__ groups,
                                              const uint32_t *__restrict__ entries,
-                                             const JobDesc *__restrict__ jobs, uint32_t blk, float4 *rows)
+                                             const JobDesc *__restrict__ jobs,
+                                             const uint64_t *__restrict__ chunk_views, uint32_t blk, float4 *rows)
 {
     auto at = [](uint32_t r, uint32_t q) { return r * 4u + (q ^ ((r >> 2) & 3u)); };
     // a group is one source mesh drawn by one or more jobs (views of one
@@ -752,6 +873,9 @@ __device__ __forceinline__ void vertex_block(const DevMesh *__restrict__ meshes,
     const uint32_t vbase = (blk - M0.vs_block0) * kVertexChunk;
     const uint32_t nv = M0.num_verts - vbase < kVertexChunk ? M0.num_verts - vbase : kVertexChunk;  // vertices of this block
     const uint32_t tid = threadIdx.x;
+    // the group's entries whose view the chunk may be in, where that was worked out
+    const uint64_t keep = chunk_views ? ldc(chunk_views + blk) : ~0ull;
+    if (keep == 0 && gr.y <= 64u) return;
     // the block's 56-byte input vertices are one contiguous run of 16-byte
     // words (its start is a multiple of 4 vertices; the last word may reach
     // into the mesh buffer's 16 bytes of padding), copied to LDS as they are
@@ -803,6 +927,7 @@ __device__ __forceinline__ void vertex_block(const DevMesh *__restrict__ meshes,
             if (w < nv * 2u) stg(sdst + w, rows[at(w >> 1, w & 1u)]);
         }
         for (uint32_t e = 0; e < gr.y; ++e) {
+            if (e < 64u && !(keep >> e & 1ull)) continue;
             const DevMesh &M = meshes[entries[gr.x + e]];
             const JobDesc &J = jobs[M.job];
             const float *W = M.wvp;
@@ -839,6 +964,7 @@ __device__ __forceinline__ void vertex_block(const DevMesh *__restrict__ meshes,
         o2 /= o3;
         const uint32_t g = M.vert_base + v;
         if (live) stg(pos4 + g, make_float4(o0, o1, o2, o3));
+        if (!attr) continue;  // the frame is not shaded: nothing reads them
         const float n0 = m4(Wd, 0, 0) * nx + m4(Wd, 0, 1) * ny + m4(Wd, 0, 2) * nz;
         const float n1 = m4(Wd, 1, 0) * nx + m4(Wd, 1, 1) * ny + m4(Wd, 1, 2) * nz;
         const float n2 = m4(Wd, 2, 0) * nx + m4(Wd, 2, 1) * ny + m4(Wd, 2, 2) * nz;
@@ -889,7 +1015,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
                                                 const uint16_t *__restrict__ cap_table, uint32_t cap_blocks,
                                                 const uint16_t *__restrict__ init_table, uint32_t init_blocks,
                                                 const uint32_t *__restrict__ tri_block_mesh, uint32_t tri_blocks,
-                                                uint32_t cull_blocks)
+                                                uint32_t cull_blocks, const uint64_t *__restrict__ chunk_views)
 {
     constexpr int kVertexF4 = 256 * 4, kCapF4 = (capacity_lds_floats<H>() + 3) / 4;
     __shared__ float4 lds[kVertexF4 > kCapF4 ? kVertexF4 : kCapF4];
@@ -910,7 +1036,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
         cull_block(meshes, tri_block_mesh, jobs, tri_blocks, blk - init_blocks);
         return;
     }
-    vertex_block(meshes, block_group, groups, entries, jobs, blk - init_blocks - cull_blocks, lds);
+    vertex_block(meshes, block_group, groups, entries, jobs, chunk_views, blk - init_blocks - cull_blocks, lds);
 }
 
 // Smaller 16-bit halves of two words, and of the wave's lanes (all active).
@@ -1012,6 +1138,7 @@ __device__ __forceinline__ int first_pixel(float mn, float reach, int lo)
 // path's rules (CCR/ERenderer.cpp:73-157, 603-624) with D4/D5, plus the
 // micro-triangle raster (RasterizeTriangle, CCR/CUDAROPs.cu:394-407, over the
 // whole bbox with the order-free key).
+template <bool kRecords>
 __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshes,
                                                const uint32_t *__restrict__ block_mesh,
                                                const JobDesc *__restrict__ jobs, uint32_t nblocks)
@@ -1021,6 +1148,7 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
     __shared__ uint32_t moff[256];
     __shared__ unsigned long long mmask[4 * kMaskChunks];
     __shared__ uint32_t mfrag[4 * kFragRing];
+    __shared__ uint8_t mhit[256];  // staged triangles that cover a pixel
     __shared__ uint32_t lrect[8];  // per wave: smallest tile x | y << 16, then the complement of the largest
     // the block's tile rectangle once the micro triangles are done
     uint32_t *const lcursor = reinterpret_cast<uint32_t *>(mstage), *const loff = lcursor + 256, *const lcap = loff + 256;
@@ -1043,7 +1171,7 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
     const bool valid = k < M.num_tris;
     const uint32_t gid = M.tri_base + k;
     // the cull stage found the block's box outside the view: no triangle survives
-    if (__builtin_amdgcn_readfirstlane(ldg(J.alive_part + blk)) == kCulledBlock) {
+    if (!kRecords && __builtin_amdgcn_readfirstlane(ldg(J.alive_part + blk)) == kCulledBlock) {
         if (valid) stg(J.alive + gid, (uint8_t)0);
         __syncthreads();  // every wave has read the mark
         if (threadIdx.x == 0) stg(J.alive_part + blk, 0u);
@@ -1053,6 +1181,7 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
     int xmin = 0, ymin = 0, xmax = 0, ymax = 0;
     float mnx = 0.f, mny = 0.f, ext_x = 0.f, ext_y = 0.f;  // smallest corner, extent
     TriLds t;
+    uint4 last = make_uint4(0u, 0u, 0u, 0u);  // the record's last quad
     if (valid) {
         uint32_t i0, i1, i2;
         if (M.topology == 0) {
@@ -1112,23 +1241,16 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
                 ymin = ymin < 0 ? 0 : ymin;
                 xmax = xmax > (int)fp.width ? (int)fp.width : xmax;
                 ymax = ymax > (int)fp.height ? (int)fp.height : ymax;
-                uint4 *r = reinterpret_cast<uint4 *>(trirec + (size_t)gid * kTriRecWords);
-                stg(r, make_uint4(__float_as_uint(t.sx0), __float_as_uint(t.sy0), __float_as_uint(t.sx1),
-                                  __float_as_uint(t.sy1)));
-                stg(r + 1, make_uint4(__float_as_uint(t.sx2), __float_as_uint(t.sy2), __float_as_uint(t.z0),
-                                      __float_as_uint(t.area)));
-                stg(r + 2, make_uint4(__float_as_uint(t.z2), __float_as_uint(t.z1),
-                                      (uint32_t)xmin | ((uint32_t)ymin << 16), (uint32_t)xmax | ((uint32_t)ymax << 16)));
                 // shading follows the reference's operation order where the
                 // interpolated attributes can be ill-conditioned: a vertex with
                 // clip w below 0.75 (at or behind the camera plane, 1/w above
                 // 4/3: its premultiplied attributes dominate and cancel), or a
                 // mesh whose attributes may exceed 4 in magnitude
                 const bool exact = M.shade_exact || !(P0.w >= 0.75f && P1.w >= 0.75f && P2.w >= 0.75f);
-                stg(r + 3, make_uint4(i0, i1, i2, mi | (exact ? 0x80000000u : 0u)));
+                last = make_uint4(i0, i1, i2, mi | (exact ? 0x80000000u : 0u));
             }
         }
-        stg(J.alive + gid, (uint8_t)(ok ? 1 : 0));
+        if (!kRecords) stg(J.alive + gid, (uint8_t)(ok ? 1 : 0));
     }
 
     // classification by the pixel range [xmin,xmax) x [ymin,ymax)
@@ -1144,6 +1266,24 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
     }
     const bool is_big = nonempty && !micro && span > fp.big_threshold;
     const bool binned = nonempty && !micro && !is_big;
+    const uint32_t range_lo = (uint32_t)xmin | ((uint32_t)ymin << 16), range_hi = (uint32_t)xmax | ((uint32_t)ymax << 16);
+    auto write_record = [&](const auto &v) {
+        uint4 *r = reinterpret_cast<uint4 *>(trirec + (size_t)gid * kTriRecWords);
+        stg(r, make_uint4(__float_as_uint(v.sx0), __float_as_uint(v.sy0), __float_as_uint(v.sx1), __float_as_uint(v.sy1)));
+        stg(r + 1, make_uint4(__float_as_uint(v.sx2), __float_as_uint(v.sy2), __float_as_uint(v.z0),
+                              __float_as_uint(v.area)));
+        stg(r + 2, make_uint4(__float_as_uint(v.z2), __float_as_uint(v.z1), range_lo, range_hi));
+        stg(r + 3, last);
+    };
+    if constexpr (kRecords) {
+        if (ok) write_record(t);
+        return;
+    }
+    // Only the records of triangles that something reads: the binned ones, and
+    // the micro triangles that cover a pixel (below), a third of the survivors
+    // where those are sub-pixel (2.4 M survivors at 1080p: 95 -> 73 us; 7 views
+    // of 4.0 M triangles: 277 -> 236; where nearly all are binned it is even).
+    if (binned || is_big) write_record(t);
 
     // Micro triangles: the wave rasterizes the union of their pixel ranges as
     // one item list (prefix sum over the ranges), so a lane's work does not
@@ -1201,6 +1341,7 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
                 m.inv = __builtin_amdgcn_rcpf((float)(xmax - mx0));
                 mstage[wsb + rank] = m;
                 wo[rank] = start;
+                mhit[wsb + rank] = 0;
             }
             uint32_t before = 0;  // triangles starting before the current chunk (wave-uniform)
             uint32_t *ring = mfrag + wave * kFragRing;
@@ -1256,13 +1397,20 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
                                 ((uint32_t)(py - (int)(mt.yr & 0xFFFFu)) << 16);
                     }
                     const uint64_t cm = __ballot(covered);
-                    if (covered) ring[(head + queued + popc_below(cm)) & (kFragRing - 1u)] = entry;
+                    if (covered) {
+                        ring[(head + queued + popc_below(cm)) & (kFragRing - 1u)] = entry;
+                        mhit[wsb + (entry & 63u)] = 1;
+                    }
                     queued += (uint32_t)__popcll(cm);
                     if (queued >= 64u) drain(64u);
                     before += (uint32_t)__popcll(m);
                 }
             }
             if (queued) drain(queued);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (items && mhit[wsb + rank]) write_record(mstage[wsb + rank]);
         }
     }
 
@@ -1634,13 +1782,6 @@ __device__ __forceinline__ float4 coverage_bound(const TriLds &t, const float4 p
 // A bound's x for "no pixel of the tile": a plane's x stays below 5e5
 // (its margin M < 0.25 bounds |x| by 0.25 / (8 u)), a constant bound below 1.
 constexpr float kSkipBound = 1.0e37f;
-
-// Float bits that order like the values (negative values reversed).
-__device__ __forceinline__ uint32_t ordered_bits(float v)
-{
-    const uint32_t b = __float_as_uint(v);
-    return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-}
 
 // The largest depth a tile's pixels hold (block-wide; one barrier).
 template <int PPT, int NW>
@@ -2855,10 +2996,13 @@ hipError_t launch_interleave_maps(const uint32_t *d, const uint32_t *n, const ui
 }
 
 hipError_t launch_mesh_boxes(const float *ivert, const uint32_t *idx, uint32_t ntri, int topology, float4 *boxes,
-                             hipStream_t s)
+                             uint4 *reach, uint32_t chunks, hipStream_t s)
 {
     if (ntri == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_mesh_boxes, dim3(ceil_div(ntri, 256u)), dim3(256), 0, s, ivert, idx, ntri, topology, boxes);
+    const dim3 g(ceil_div(ntri, 256u)), b(256);
+    hipLaunchKernelGGL(k_mesh_boxes, g, b, 0, s, ivert, idx, ntri, topology, boxes, (uint32_t *)reach,
+                       chunks * 8u);
+    hipLaunchKernelGGL(k_vertex_boxes, g, b, 0, s, idx, ntri, topology, (const float4 *)boxes, (uint32_t *)reach);
     return hipGetLastError();
 }
 
@@ -2876,11 +3020,14 @@ hipError_t launch_vertex(const Launch &L, int with_capacity, hipStream_t s)
     const uint32_t init_blocks = with_capacity == 2 ? 0u : L.grid[ST_INIT];
     const uint32_t cull_blocks = with_capacity == 2 ? 0u : ceil_div(L.tri_blocks, 256u);
     const uint16_t *init_table = L.table[ST_INIT];
+    if (L.chunk_views && vs_blocks)
+        hipLaunchKernelGGL(k_chunk_views, dim3(ceil_div(vs_blocks, 4u)), dim3(256), 0, s, L.meshes, L.vs_block_group,
+                           L.vs_groups, L.vs_entries, L.chunk_views, vs_blocks);
     if (!with_capacity || !cap_blocks) {
         if (vs_blocks + init_blocks == 0) return hipSuccess;
         hipLaunchKernelGGL(k_vertex<0>, dim3(init_blocks + cull_blocks + vs_blocks), dim3(256), 0, s, L.meshes,
                            L.vs_block_group, L.vs_groups, L.vs_entries, L.jobs, (const uint16_t *)nullptr, 0u, init_table,
-                           init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks);
+                           init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks, L.chunk_views);
         return hipGetLastError();
     }
     const dim3 g(cap_blocks + init_blocks + cull_blocks + vs_blocks), b(256);
@@ -2889,15 +3036,15 @@ hipError_t launch_vertex(const Launch &L, int with_capacity, hipStream_t s)
     switch (L.model_hidden) {
     case 32:
         hipLaunchKernelGGL(k_vertex<32>, g, b, 0, s, L.meshes, L.vs_block_group, L.vs_groups, L.vs_entries, L.jobs,
-                           L.table[ST_CAP], cap_blocks, init_table, init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks);
+                           L.table[ST_CAP], cap_blocks, init_table, init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks, L.chunk_views);
         break;
     case 64:
         hipLaunchKernelGGL(k_vertex<64>, g, b, 0, s, L.meshes, L.vs_block_group, L.vs_groups, L.vs_entries, L.jobs,
-                           L.table[ST_CAP], cap_blocks, init_table, init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks);
+                           L.table[ST_CAP], cap_blocks, init_table, init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks, L.chunk_views);
         break;
     default:
         hipLaunchKernelGGL(k_vertex<16>, g, b, 0, s, L.meshes, L.vs_block_group, L.vs_groups, L.vs_entries, L.jobs,
-                           L.table[ST_CAP], cap_blocks, init_table, init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks);
+                           L.table[ST_CAP], cap_blocks, init_table, init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks, L.chunk_views);
         break;
     }
     return hipGetLastError();
@@ -2906,7 +3053,21 @@ hipError_t launch_vertex(const Launch &L, int with_capacity, hipStream_t s)
 hipError_t launch_setup(const Launch &L, hipStream_t s)
 {
     if (L.tri_blocks == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_setup, dim3(L.tri_blocks), dim3(256), 0, s, L.meshes, L.tri_block_mesh, L.jobs, L.tri_blocks);
+    hipLaunchKernelGGL(k_setup<false>, dim3(L.tri_blocks), dim3(256), 0, s, L.meshes, L.tri_block_mesh, L.jobs, L.tri_blocks);
+    return hipGetLastError();
+}
+
+// Every position and attribute, and every survivor's record, of a launch whose
+// frame is done (job 0's buffers hold the rest of it).
+hipError_t launch_debug_fill(const Launch &L, hipStream_t s)
+{
+    if (L.vs_blocks)
+        hipLaunchKernelGGL(k_vertex<0>, dim3(L.vs_blocks), dim3(256), 0, s, L.meshes, L.vs_block_group, L.vs_groups,
+                           L.vs_entries, L.jobs, (const uint16_t *)nullptr, 0u, (const uint16_t *)nullptr, 0u,
+                           L.tri_block_mesh, 0u, 0u, (const uint64_t *)nullptr);
+    if (L.tri_blocks)
+        hipLaunchKernelGGL(k_setup<true>, dim3(L.tri_blocks), dim3(256), 0, s, L.meshes, L.tri_block_mesh, L.jobs,
+                           L.tri_blocks);
     return hipGetLastError();
 }
 

@@ -21,6 +21,7 @@ struct Launch {
     const uint32_t *vs_entries;       // the mesh entries of each group (one source mesh, one entry per job)
     const uint32_t *tri_block_mesh;   // triangle block -> mesh entry
     uint32_t vs_blocks, tri_blocks;
+    uint64_t *chunk_views;            // per vertex block: the entries of its group whose view it may be in (null: all)
     const uint16_t *table[ST_COUNT];  // device block -> job tables (null when njobs == 1)
     uint32_t grid[ST_COUNT];          // blocks of each stage over all jobs (0: stage skipped)
     uint32_t cap_jobs;                // jobs binning in a single pass (capacities placed by the vertex launch)
@@ -52,9 +53,13 @@ inline size_t stage_meshes_offset(uint32_t n)
 
 // Resets a key buffer to depth 1 / no triangle (before a renderer's first frame).
 hipError_t launch_clear_keys(unsigned long long *keys, size_t n, hipStream_t s);
-// Object-space boxes of a mesh's runs of 256 triangles (two float4 each).
+// Object-space boxes of a mesh's runs of 256 triangles (two float4 each), and its
+// vertex chunks' reach (two uint4 each).
 hipError_t launch_mesh_boxes(const float *ivert, const uint32_t *idx, uint32_t ntri, int topology, float4 *boxes,
-                             hipStream_t s);
+                             uint4 *reach, uint32_t chunks, hipStream_t s);
+// What a frame left out because nothing of its own reads it: the positions and
+// attributes of vertices out of view, and the other survivors' records.
+hipError_t launch_debug_fill(const Launch &L, hipStream_t s);
 hipError_t launch_interleave_maps(const uint32_t *d, const uint32_t *n, const uint32_t *sp, const uint32_t *g,
                                   uint4 *out, size_t count, hipStream_t s);
 // with_capacity 0: the vertex pass; 1: the vertex pass with the single-pass

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <memory>
 #include <vector>
 
 #include "rast.h"
@@ -56,6 +57,7 @@ struct LaunchPlan {
     std::vector<uint32_t> vs_block0, tri_block0;  // per mesh entry
     DBuf d_block_mesh, d_tables, d_stage;
     DBuf d_alive_part;  // culling survivors per setup block
+    DBuf d_chunk_views; // Launch::chunk_views
     // view-independent attributes of the scenes two or more jobs draw (views):
     // 32 bytes per vertex of each such scene, at sattr_off[job] (SIZE_MAX: none)
     DBuf d_sattr;
@@ -96,8 +98,9 @@ struct TexQuad {
 struct rast_mesh {
     rast_renderer *r = nullptr;
     float *ivert14 = nullptr;  // 14 floats per vertex (the 56-byte IVertex as given) + 16 bytes of padding
-    uint32_t *idx = nullptr;   // the indices, then (16-byte aligned) the boxes
+    uint32_t *idx = nullptr;   // the indices, then (16-byte aligned) the boxes and reaches
     float4 *boxes = nullptr;   // object-space box (lo, hi) of every 256 triangles
+    uint4 *reach = nullptr;    // behind them: the boxes the triangles of every kVertexChunk vertices lie in
     uint32_t nv = 0, ni = 0, ntri = 0;
     int topology = 0;
     float world[16];
@@ -105,6 +108,13 @@ struct rast_mesh {
     const uint4 *texq = nullptr;  // interleaved maps for tex[0..3], set by prepare_job
     float attr_max = 0.f;         // largest |component| of the input normals and tangents
     uint64_t tri_base = 0;
+};
+
+// The meshes of a frame and their world matrices, for data of the frame that is
+// formed only when it is asked for.
+struct FrameMesh {
+    const rast_mesh *m;
+    float world[16];
 };
 
 struct rast_renderer {
@@ -120,6 +130,10 @@ struct rast_renderer {
     std::vector<rast_renderer *> views;    // views drawing this renderer's meshes
     uint64_t scene_version = 1;            // bumped when the mesh list changes
     uint64_t layout_version = 0;           // scene version the block tables were built for
+    uint64_t world_version = 1;            // bumped when a mesh's world matrix changes
+    // the scene as of these versions, shared by the frames that drew it
+    std::shared_ptr<const std::vector<FrameMesh>> drawn;
+    uint64_t drawn_scene = 0, drawn_world = 0;
     hipEvent_t join = nullptr;             // orders a batch after this renderer's earlier work
     uint64_t batch_seq = 0;                // batch that rendered the last frame (0: none pending)
     bool stream_busy = false;              // work queued on `stream` since its last synchronization
@@ -154,6 +168,11 @@ struct rast_renderer {
     rast_frame_opts last_opts{};
     bool frame_pending = false;
     bool frame_valid = false;
+    // what the last frame was drawn from, until its debug buffers are whole
+    std::shared_ptr<const std::vector<FrameMesh>> frame_scene, next_scene;
+    rast_camera frame_cam{};
+    uint32_t frame_w = 0, frame_h = 0;
+    int32_t frame_cull = 0;
     bool last_single = false;              // capacities predicted (single-pass policies)
     uint32_t last_stride = 0;              // exact binning into fixed regions of this many entries (0: two passes)
     bool two_pass = false;                 // the scene overflowed its fixed regions: exact frames take two passes
