@@ -859,6 +859,7 @@ void plan_free(LaunchPlan &p)
     dfree(p.d_block_mesh);
     dfree(p.d_alive_part);
     dfree(p.d_chunk_views);
+    dfree(p.d_live);
     dfree(p.d_tables);
     dfree(p.d_stage);
     dfree(p.d_sattr);
@@ -1035,6 +1036,8 @@ static int build_plan(LaunchPlan &P, rast_renderer *const *rs, uint32_t n, int h
     for (const auto &mm : members) tab.insert(tab.end(), mm.begin(), mm.end());
     RAST_TRY(dev_alloc(P.d_block_mesh, (tab.size() + 2) * 4));
     RAST_TRY(dev_alloc(P.d_alive_part, ((size_t)L.tri_blocks + 1) * 4));
+    RAST_TRY(dev_alloc(P.d_live, ((size_t)L.tri_blocks + 1) * 8));
+    L.live = (uint2 *)P.d_live.p;
     uint32_t *bm = (uint32_t *)P.d_block_mesh.p;
     if (!tab.empty()) HIP_TRY(hipMemcpy(bm, tab.data(), tab.size() * 4, hipMemcpyHostToDevice));
     // Views of large scenes: a vertex chunk is transformed for the views it may be
@@ -1371,14 +1374,14 @@ static void finish_enqueue(rast_renderer *r)
 }
 
 // Completes the last frame's debug buffers: positions and attributes of the
-// vertices out of view, the records of the survivors that nothing of the frame
-// reads (launch_debug_fill).  r's GPU work is done.
+// vertices out of view, survivor flags, the records of the survivors that
+// nothing of the frame reads (launch_debug_fill).  r's GPU work is done.
 static int complete_debug_of(rast_renderer *r, const std::vector<FrameMesh> &ms)
 {
     // one job, a vertex group per mesh: [job][meshes][vertex block -> group]
-    // [triangle block -> mesh][groups][entries]
+    // [triangle blocks][groups][entries][work counters]
     std::vector<DevMesh> rows(ms.size());
-    std::vector<uint32_t> vs_group, tri_mesh, groups, entries;
+    std::vector<uint32_t> vs_group, live, groups, entries;
     rast_frame_consts fc;
     camera_frame(r->frame_cam, r->frame_w, r->frame_h, fc);
     JobDesc J;
@@ -1386,9 +1389,12 @@ static int complete_debug_of(rast_renderer *r, const std::vector<FrameMesh> &ms)
     uint32_t vb = 0, tb = 0;
     for (uint32_t i = 0; i < ms.size(); ++i) {
         const rast_mesh *m = ms[i].m;
-        fill_mesh(rows[i], m, ms[i].world, fc, vb, tb, (uint32_t)vs_group.size(), (uint32_t)tri_mesh.size());
+        fill_mesh(rows[i], m, ms[i].world, fc, vb, tb, (uint32_t)vs_group.size(), (uint32_t)live.size() / 2);
         vs_group.insert(vs_group.end(), ceil_div(m->nv, kVertexChunk), i);
-        tri_mesh.insert(tri_mesh.end(), ceil_div(m->ntri, 256), i);
+        for (uint32_t b = 0; b < ceil_div(m->ntri, 256); ++b) {
+            live.push_back((uint32_t)live.size() / 2);
+            live.push_back(i);
+        }
         groups.push_back(i);
         groups.push_back(1u);
         entries.push_back(i);
@@ -1396,7 +1402,8 @@ static int complete_debug_of(rast_renderer *r, const std::vector<FrameMesh> &ms)
         tb += m->ntri;
     }
     // (a later frame that failed may have lost them)
-    if (r->pos4.n < (size_t)vb * 16 || r->attr.n < (size_t)vb * 48 || r->trirec.n < (size_t)tb * kTriRecWords * 4)
+    if (r->pos4.n < (size_t)vb * 16 || r->attr.n < (size_t)vb * 48 || r->trirec.n < (size_t)tb * kTriRecWords * 4 ||
+        r->alive.n < tb)
         return RAST_OK;
     J.fp.width = r->frame_w;
     J.fp.height = r->frame_h;
@@ -1407,6 +1414,7 @@ static int complete_debug_of(rast_renderer *r, const std::vector<FrameMesh> &ms)
     J.pos4 = (float4 *)r->pos4.p;
     J.attr = r->last_shared_attr ? nullptr : (float4 *)r->attr.p;  // where the frame's are in this layout
     J.trirec = (uint32_t *)r->trirec.p;
+    J.alive = (uint8_t *)r->alive.p;
     std::vector<char> block;
     auto put = [&block](const void *p, size_t n) {
         block.resize((block.size() + 15) & ~(size_t)15);
@@ -1415,8 +1423,11 @@ static int complete_debug_of(rast_renderer *r, const std::vector<FrameMesh> &ms)
         return at;
     };
     const size_t at_job = put(&J, sizeof J), at_mesh = put(rows.data(), rows.size() * sizeof(DevMesh));
-    const size_t at_vs = put(vs_group.data(), vs_group.size() * 4), at_tri = put(tri_mesh.data(), tri_mesh.size() * 4);
+    const size_t at_vs = put(vs_group.data(), vs_group.size() * 4), at_live = put(live.data(), live.size() * 4);
     const size_t at_gr = put(groups.data(), groups.size() * 4), at_en = put(entries.data(), entries.size() * 4);
+    uint32_t work[kStageCounterBytes / 4] = {};
+    work[kLiveWord] = (uint32_t)live.size() / 2;
+    const size_t at_work = put(work, sizeof work);
     char *d = nullptr;
     HIP_TRY(hipMalloc((void **)&d, block.size()));
     Launch L{};
@@ -1424,11 +1435,12 @@ static int complete_debug_of(rast_renderer *r, const std::vector<FrameMesh> &ms)
     L.jobs = (const JobDesc *)(d + at_job);
     L.meshes = (const DevMesh *)(d + at_mesh);
     L.vs_block_group = (const uint32_t *)(d + at_vs);
-    L.tri_block_mesh = (const uint32_t *)(d + at_tri);
+    L.live = (uint2 *)(d + at_live);
+    L.work = (uint32_t *)(d + at_work);
     L.vs_groups = (const uint2 *)(d + at_gr);
     L.vs_entries = (const uint32_t *)(d + at_en);
     L.vs_blocks = (uint32_t)vs_group.size();
-    L.tri_blocks = (uint32_t)tri_mesh.size();
+    L.tri_blocks = (uint32_t)live.size() / 2;
     hipError_t e = hipMemcpyAsync(d, block.data(), block.size(), hipMemcpyHostToDevice, r->stream);
     if (e == hipSuccess) e = launch_debug_fill(L, r->stream);
     const hipError_t w = hipStreamSynchronize(r->stream);
@@ -1734,7 +1746,8 @@ extern "C" int rast_debug_read(rast_renderer *r, int which, void *dst, size_t by
     size_t size = 0;
     const void *src = nullptr;
     std::vector<uint32_t> tmp;
-    if (dst && (which == RAST_DEBUG_VERTEX_POS || which == RAST_DEBUG_VERTEX_ATTR || which == RAST_DEBUG_TRI_RECORDS))
+    if (dst && (which == RAST_DEBUG_VERTEX_POS || which == RAST_DEBUG_VERTEX_ATTR || which == RAST_DEBUG_TRI_RECORDS ||
+                which == RAST_DEBUG_TRI_ALIVE))
         RAST_TRY(complete_debug(r));
     switch (which) {
     case RAST_DEBUG_VERTEX_POS: size = (size_t)r->total_verts * 16; src = r->pos4.p; break;

@@ -236,7 +236,7 @@ __device__ __forceinline__ uint64_t match_tile(uint32_t t)
 // p0: every thread with p1 / p2 set gets a slot of its counter, one atomic
 // per counter per 256-thread block and only where the predicate holds
 // somewhere in the block (two barriers; every thread of the block must call
-// it).  The p0 count is stored to part[blockIdx.x], with no atomic: a counter
+// it).  The p0 count is stored to part, with no atomic: a counter
 // that every block updates serializes those updates at its cache line, and
 // every block waiting for the returned value paid for that.
 __device__ __forceinline__ void block_append(uint32_t *part, bool p0, uint32_t *c1, bool p1, uint32_t *c2, bool p2,
@@ -255,7 +255,7 @@ __device__ __forceinline__ void block_append(uint32_t *part, bool p0, uint32_t *
         const uint32_t a = l[0], b = l[1], c = l[2], d = l[3];
         const uint32_t tot = a + b + c + d;
         if (threadIdx.x == 0) {
-            stg(part + blockIdx.x, tot);
+            stg(part, tot);
         } else {
             const uint32_t base = tot ? gatomic_add(threadIdx.x == 1 ? c1 : c2, tot) : 0u;
             l[0] = base;
@@ -753,24 +753,39 @@ __device__ __forceinline__ bool box_outside(const float *wvp, const float4 lo, c
     return (out & 0xC0u) != 0u && (out & 0x3Fu) != 0u;
 }
 
-// The cull stage, workgroups of the vertex launch: one thread per setup
-// workgroup marks in its survivor count (alive_part) whether its triangles'
-// box lies outside the view, so that the workgroup ends at once.  In a
+// The cull stage, workgroups of the vertex launch: one thread per block of 256
+// triangles tests its box and puts a block that may be in view on the setup
+// pass's list (block, mesh entry); the others have no survivors.  In a
 // workgroup of its own per 256 boxes the test costs a few instructions per
 // setup wave and rides along with the vertex pass.  Six cube-map faces and a
-// main view of 4.0 M triangles: setup 338 -> 277 us; a frame that sees all of
-// its scene is unchanged.
-constexpr uint32_t kCulledBlock = 0x80000000u;
-
+// main view of 4.0 M triangles: setup 338 -> 277 us where blocks out of view
+// ended at once, and 230 -> 184 with the list, as workgroups past its end need one
+// load only (2.1 M triangles at 4K: 66 -> 59).
 __device__ __forceinline__ void cull_block(const DevMesh *__restrict__ meshes, const uint32_t *__restrict__ block_mesh,
-                                           const JobDesc *__restrict__ jobs, uint32_t tri_blocks, uint32_t blk)
+                                           const JobDesc *__restrict__ jobs, uint32_t tri_blocks, uint2 *live,
+                                           uint32_t *live_n, uint32_t blk, uint32_t *lds)
 {
     const uint32_t b = blk * 256u + threadIdx.x;
-    if (b >= tri_blocks) return;
-    const DevMesh *M = meshes + ldg(block_mesh + b);
-    const float4 *box = ldg(&M->boxes) + 2 * (size_t)(b - ldg(&M->tri_block0));
-    const bool out = box_outside(M->wvp, ldg(box), ldg(box + 1));
-    stg(ldg(&jobs[ldg(&M->job)].alive_part) + b, out ? kCulledBlock : 0u);
+    bool in = false;
+    uint32_t mi = 0;
+    if (b < tri_blocks) {
+        mi = ldg(block_mesh + b);
+        const DevMesh *M = meshes + mi;
+        const float4 *box = ldg(&M->boxes) + 2 * (size_t)(b - ldg(&M->tri_block0));
+        in = !box_outside(M->wvp, ldg(box), ldg(box + 1));
+        if (!in) stg(ldg(&jobs[ldg(&M->job)].alive_part) + b, 0u);
+    }
+    // places on the list: one atomic per workgroup (per wave, 7 views' 1,700
+    // updates of the one counter took the vertex pass 10 us longer)
+    const uint64_t m = __ballot(in);
+    const uint32_t wave = threadIdx.x >> 6;
+    if (lane_id() == 0) lds[wave] = (uint32_t)__popcll(m);
+    __syncthreads();
+    if (threadIdx.x == 0) lds[4] = gatomic_add(live_n, lds[0] + lds[1] + lds[2] + lds[3]);
+    __syncthreads();
+    uint32_t at = lds[4] + popc_below(m);
+    for (uint32_t w = 0; w < wave; ++w) at += lds[w];
+    if (in) stg(live + at, make_uint2(b, mi));
 }
 
 // The entries [0, min(n, 64)) of a vertex group whose view the reach [lo, hi] of a
@@ -1015,7 +1030,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
                                                 const uint16_t *__restrict__ cap_table, uint32_t cap_blocks,
                                                 const uint16_t *__restrict__ init_table, uint32_t init_blocks,
                                                 const uint32_t *__restrict__ tri_block_mesh, uint32_t tri_blocks,
-                                                uint32_t cull_blocks, const uint64_t *__restrict__ chunk_views)
+                                                uint32_t cull_blocks, const uint64_t *__restrict__ chunk_views,
+                                                uint2 *__restrict__ live, uint32_t *__restrict__ live_n)
 {
     constexpr int kVertexF4 = 256 * 4, kCapF4 = (capacity_lds_floats<H>() + 3) / 4;
     __shared__ float4 lds[kVertexF4 > kCapF4 ? kVertexF4 : kCapF4];
@@ -1033,7 +1049,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
         return;
     }
     if (blk - init_blocks < cull_blocks) {
-        cull_block(meshes, tri_block_mesh, jobs, tri_blocks, blk - init_blocks);
+        cull_block(meshes, tri_block_mesh, jobs, tri_blocks, live, live_n, blk - init_blocks,
+                   reinterpret_cast<uint32_t *>(lds));
         return;
     }
     vertex_block(meshes, block_group, groups, entries, jobs, chunk_views, blk - init_blocks - cull_blocks, lds);
@@ -1140,8 +1157,8 @@ __device__ __forceinline__ int first_pixel(float mn, float reach, int lo)
 // whole bbox with the order-free key).
 template <bool kRecords>
 __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshes,
-                                               const uint32_t *__restrict__ block_mesh,
-                                               const JobDesc *__restrict__ jobs, uint32_t nblocks)
+                                               const uint2 *__restrict__ live, const uint32_t *__restrict__ live_n,
+                                               const JobDesc *__restrict__ jobs)
 {
     __shared__ uint32_t lds_append[12];
     __shared__ MicroLds mstage[256];
@@ -1155,9 +1172,9 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
     static_assert(sizeof(mstage) >= 3 * 256 * sizeof(uint32_t), "the tile cursors, offsets and capacities fit");
     // workgroups in launch order (consecutive blocks spread over the XCDs;
     // XCD-contiguous ranges measured slower)
-    const uint32_t blk = blockIdx.x;
-    if (blk >= nblocks) return;
-    const uint32_t mi = block_mesh[blk];
+    if (blockIdx.x >= ldc(live_n)) return;
+    const uint64_t entry = ldc(reinterpret_cast<const uint64_t *>(live) + blockIdx.x);
+    const uint32_t blk = (uint32_t)entry, mi = (uint32_t)(entry >> 32);
     const DevMesh &M = meshes[mi];
     const JobDesc &J = jobs[M.job];
     const FrameParams &fp = J.fp;
@@ -1170,13 +1187,6 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
     const uint32_t k = (blk - M.tri_block0) * 256u + threadIdx.x;
     const bool valid = k < M.num_tris;
     const uint32_t gid = M.tri_base + k;
-    // the cull stage found the block's box outside the view: no triangle survives
-    if (!kRecords && __builtin_amdgcn_readfirstlane(ldg(J.alive_part + blk)) == kCulledBlock) {
-        if (valid) stg(J.alive + gid, (uint8_t)0);
-        __syncthreads();  // every wave has read the mark
-        if (threadIdx.x == 0) stg(J.alive_part + blk, 0u);
-        return;
-    }
     bool ok = false;
     int xmin = 0, ymin = 0, xmax = 0, ymax = 0;
     float mnx = 0.f, mny = 0.f, ext_x = 0.f, ext_y = 0.f;  // smallest corner, extent
@@ -1250,7 +1260,7 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
                 last = make_uint4(i0, i1, i2, mi | (exact ? 0x80000000u : 0u));
             }
         }
-        if (!kRecords) stg(J.alive + gid, (uint8_t)(ok ? 1 : 0));
+        if constexpr (kRecords) stg(J.alive + gid, (uint8_t)(ok ? 1 : 0));
     }
 
     // classification by the pixel range [xmin,xmax) x [ymin,ymax)
@@ -1428,7 +1438,7 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
     }
     // the survivor list feeds the two-pass binner's fill pass only
     uint32_t bslot, sslot;
-    block_append(J.alive_part, ok, &ctr->num_big, is_big, &ctr->num_binned, binned && !single_pass, lds_append, bslot,
+    block_append(J.alive_part + blk, ok, &ctr->num_big, is_big, &ctr->num_binned, binned && !single_pass, lds_append, bslot,
                  sslot);
     if (is_big) {
         if (bslot < J.big_cap) stg(J.big + bslot, gid);
@@ -3053,7 +3063,7 @@ hipError_t launch_vertex(const Launch &L, int with_capacity, hipStream_t s)
         if (vs_blocks + init_blocks == 0) return hipSuccess;
         hipLaunchKernelGGL(k_vertex<0>, dim3(init_blocks + cull_blocks + vs_blocks), dim3(256), 0, s, L.meshes,
                            L.vs_block_group, L.vs_groups, L.vs_entries, L.jobs, (const uint16_t *)nullptr, 0u, init_table,
-                           init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks, L.chunk_views);
+                           init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks, L.chunk_views, L.live, L.work + kLiveWord);
         return hipGetLastError();
     }
     const dim3 g(cap_blocks + init_blocks + cull_blocks + vs_blocks), b(256);
@@ -3062,15 +3072,15 @@ hipError_t launch_vertex(const Launch &L, int with_capacity, hipStream_t s)
     switch (L.model_hidden) {
     case 32:
         hipLaunchKernelGGL(k_vertex<32>, g, b, 0, s, L.meshes, L.vs_block_group, L.vs_groups, L.vs_entries, L.jobs,
-                           L.table[ST_CAP], cap_blocks, init_table, init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks, L.chunk_views);
+                           L.table[ST_CAP], cap_blocks, init_table, init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks, L.chunk_views, L.live, L.work + kLiveWord);
         break;
     case 64:
         hipLaunchKernelGGL(k_vertex<64>, g, b, 0, s, L.meshes, L.vs_block_group, L.vs_groups, L.vs_entries, L.jobs,
-                           L.table[ST_CAP], cap_blocks, init_table, init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks, L.chunk_views);
+                           L.table[ST_CAP], cap_blocks, init_table, init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks, L.chunk_views, L.live, L.work + kLiveWord);
         break;
     default:
         hipLaunchKernelGGL(k_vertex<16>, g, b, 0, s, L.meshes, L.vs_block_group, L.vs_groups, L.vs_entries, L.jobs,
-                           L.table[ST_CAP], cap_blocks, init_table, init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks, L.chunk_views);
+                           L.table[ST_CAP], cap_blocks, init_table, init_blocks, L.tri_block_mesh, L.tri_blocks, cull_blocks, L.chunk_views, L.live, L.work + kLiveWord);
         break;
     }
     return hipGetLastError();
@@ -3079,21 +3089,22 @@ hipError_t launch_vertex(const Launch &L, int with_capacity, hipStream_t s)
 hipError_t launch_setup(const Launch &L, hipStream_t s)
 {
     if (L.tri_blocks == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_setup<false>, dim3(L.tri_blocks), dim3(256), 0, s, L.meshes, L.tri_block_mesh, L.jobs, L.tri_blocks);
+    hipLaunchKernelGGL(k_setup<false>, dim3(L.tri_blocks), dim3(256), 0, s, L.meshes, (const uint2 *)L.live,
+                       (const uint32_t *)(L.work + kLiveWord), L.jobs);
     return hipGetLastError();
 }
 
-// Every position and attribute, and every survivor's record, of a launch whose
-// frame is done (job 0's buffers hold the rest of it).
+// Every position and attribute, every survivor's record and the survivor flags
+// of a launch whose frame is done; L.live lists every triangle block.
 hipError_t launch_debug_fill(const Launch &L, hipStream_t s)
 {
     if (L.vs_blocks)
         hipLaunchKernelGGL(k_vertex<0>, dim3(L.vs_blocks), dim3(256), 0, s, L.meshes, L.vs_block_group, L.vs_groups,
                            L.vs_entries, L.jobs, (const uint16_t *)nullptr, 0u, (const uint16_t *)nullptr, 0u,
-                           L.tri_block_mesh, 0u, 0u, (const uint64_t *)nullptr);
+                           L.tri_block_mesh, 0u, 0u, (const uint64_t *)nullptr, (uint2 *)nullptr, (uint32_t *)nullptr);
     if (L.tri_blocks)
-        hipLaunchKernelGGL(k_setup<true>, dim3(L.tri_blocks), dim3(256), 0, s, L.meshes, L.tri_block_mesh, L.jobs,
-                           L.tri_blocks);
+        hipLaunchKernelGGL(k_setup<true>, dim3(L.tri_blocks), dim3(256), 0, s, L.meshes, (const uint2 *)L.live,
+                           (const uint32_t *)(L.work + kLiveWord), L.jobs);
     return hipGetLastError();
 }
 

@@ -20,6 +20,7 @@ struct Launch {
     const uint2 *vs_groups;           // group -> (first index into vs_entries, count)
     const uint32_t *vs_entries;       // the mesh entries of each group (one source mesh, one entry per job)
     const uint32_t *tri_block_mesh;   // triangle block -> mesh entry
+    uint2 *live;                      // the triangle blocks that may be in view and their mesh entries, work[kLiveWord] of them
     uint32_t vs_blocks, tri_blocks;
     uint64_t *chunk_views;            // per vertex block: the entries of its group whose view it may be in (null: all)
     const uint16_t *table[ST_COUNT];  // device block -> job tables (null when njobs == 1)
@@ -39,6 +40,8 @@ struct Launch {
 
 // Staging bytes in front of the job table: the launch's work counters.
 constexpr size_t kStageCounterBytes = 64;
+constexpr uint32_t kLiveWord = 15;  // work counter: entries of Launch::live (the others: one per stage)
+static_assert(kLiveWord >= (uint32_t)ST_COUNT && kLiveWord * 4 < kStageCounterBytes, "the counters fit");
 
 // The staging block of a launch of n jobs: work counters, JobDesc[n], each
 // job's FrameCounters (zeros, like the work counters: the upload starts every
@@ -58,7 +61,7 @@ hipError_t launch_clear_keys(unsigned long long *keys, size_t n, hipStream_t s);
 hipError_t launch_mesh_boxes(const float *ivert, const uint32_t *idx, uint32_t ntri, int topology, float4 *boxes,
                              uint4 *reach, uint32_t chunks, hipStream_t s);
 // What a frame left out because nothing of its own reads it: the positions and
-// attributes of vertices out of view, and the other survivors' records.
+// attributes of vertices out of view, survivor flags and the other records.
 hipError_t launch_debug_fill(const Launch &L, hipStream_t s);
 hipError_t launch_interleave_maps(const uint32_t *d, const uint32_t *n, const uint32_t *sp, const uint32_t *g,
                                   uint4 *out, size_t count, hipStream_t s);

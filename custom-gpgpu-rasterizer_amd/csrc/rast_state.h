@@ -58,6 +58,7 @@ struct LaunchPlan {
     DBuf d_block_mesh, d_tables, d_stage;
     DBuf d_alive_part;  // culling survivors per setup block
     DBuf d_chunk_views; // Launch::chunk_views
+    DBuf d_live;        // Launch::live
     // view-independent attributes of the scenes two or more jobs draw (views):
     // 32 bytes per vertex of each such scene, at sattr_off[job] (SIZE_MAX: none)
     DBuf d_sattr;
