@@ -2872,9 +2872,14 @@ __device__ __forceinline__ void shade_pixel(const DevMesh *__restrict__ meshes, 
 }
 
 
-// A block shades 64 x kShadeRows pixels: lane x of wave w takes the pixels
-// (x, w), (x, w + 4), ...  The vis reads of all of them go out first, so each
-// further pixel of a lane waits for three dependent gathers instead of four.
+// A block shades 64 x kShadeRows pixels, a wave 16 of the columns: a lane takes
+// the pixels (x, y), (x, y + 4), ...  The vis reads of all of them go out first,
+// so each further pixel of a lane waits for three dependent gathers instead of
+// four.  The gathers bound the pass (13 of 16 bytes a pixel, returned at 64
+// bytes a cycle and CU), more so where a wave's pixels show many triangles: a
+// 16 x 4 patch shows fewer than a row of 64 (7 views 160 -> 148 us, 1080p of
+// sub-pixel triangles 56 -> 53.5; 8K, where they are large, is even; 8 x 8
+// patches lose in the partial lines of vis and rgba what they gain).
 template <bool kLinear, bool kSplit, bool kFar>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kSplit && !kLinear && !kFar ? 8 : 1))) void k_shade(
     const DevMesh *__restrict__ meshes, const JobDesc *__restrict__ jobs, const uint16_t *__restrict__ table)
@@ -2897,8 +2902,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kSplit && !
     }
     constexpr int P = kShadeRows / 4;
     const uint32_t bw = (fp.width + 63u) / 64u;
-    const uint32_t x = (local % bw) * 64u + (threadIdx.x & 63u);
-    const uint32_t y0 = (local / bw) * (uint32_t)kShadeRows + (threadIdx.x >> 6);
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t x = (local % bw) * 64u + (threadIdx.x >> 6) * 16u + (lane & 15u);
+    const uint32_t y0 = (local / bw) * (uint32_t)kShadeRows + (lane >> 4);
     if (x >= fp.width || y0 >= fp.height) return;
     uint32_t ids[P];
 #pragma unroll
