@@ -1194,6 +1194,7 @@ static int stage_launch(LaunchPlan &P, rast_renderer *const *rs, uint32_t n)
         memcpy(J.block0, &P.block0[(size_t)j * ST_COUNT], sizeof J.block0);
         memcpy(J.nblocks, &P.nblocks[(size_t)j * ST_COUNT], sizeof J.nblocks);
         J.mesh0 = me;
+        r->frame_mesh0 = me;
         J.single = r->last_single || r->last_stride;
         J.stride = r->last_stride;
         J.learned = job_learned(r);
@@ -1393,11 +1394,11 @@ static int complete_debug_of(rast_renderer *r, const std::vector<FrameMesh> &ms)
         vs_group.insert(vs_group.end(), ceil_div(m->nv, kVertexChunk), i);
         for (uint32_t b = 0; b < ceil_div(m->ntri, 256); ++b) {
             live.push_back((uint32_t)live.size() / 2);
-            live.push_back(i);
+            live.push_back(r->frame_mesh0 + i);
         }
         groups.push_back(i);
         groups.push_back(1u);
-        entries.push_back(i);
+        entries.push_back(r->frame_mesh0 + i);
         vb += m->nv;
         tb += m->ntri;
     }
@@ -1433,7 +1434,8 @@ static int complete_debug_of(rast_renderer *r, const std::vector<FrameMesh> &ms)
     Launch L{};
     L.njobs = 1;
     L.jobs = (const JobDesc *)(d + at_job);
-    L.meshes = (const DevMesh *)(d + at_mesh);
+    // the frame's mesh indices (a record's word 15) count over its launch
+    L.meshes = (const DevMesh *)(d + at_mesh) - r->frame_mesh0;
     L.vs_block_group = (const uint32_t *)(d + at_vs);
     L.live = (uint2 *)(d + at_live);
     L.work = (uint32_t *)(d + at_work);

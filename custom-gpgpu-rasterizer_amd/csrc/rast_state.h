@@ -172,7 +172,7 @@ struct rast_renderer {
     // what the last frame was drawn from, until its debug buffers are whole
     std::shared_ptr<const std::vector<FrameMesh>> frame_scene, next_scene;
     rast_camera frame_cam{};
-    uint32_t frame_w = 0, frame_h = 0;
+    uint32_t frame_w = 0, frame_h = 0, frame_mesh0 = 0;
     int32_t frame_cull = 0;
     bool last_single = false;              // capacities predicted (single-pass policies)
     uint32_t last_stride = 0;              // exact binning into fixed regions of this many entries (0: two passes)

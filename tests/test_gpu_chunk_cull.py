@@ -48,7 +48,7 @@ def check_frame(got, sc, cam, opts):
         assert d.max() <= 1
 
 
-def check_debug(r, sc, cam, opts, attributes=True):
+def check_debug(r, sc, cam, opts, attributes=True, first_mesh=0):
     both = [O.vertex_transform(sc, cam, W, H, k) for k in range(len(sc.meshes))]
     opos, oattr = (np.concatenate([b[q] for b in both]) for q in range(2))
     pos = r.debug_read(R.DEBUG_VERTEX_POS, np.uint32).reshape(-1, 4)
@@ -63,6 +63,9 @@ def check_debug(r, sc, cam, opts, attributes=True):
     np.testing.assert_array_equal(r.debug_read(R.DEBUG_TRI_ALIVE, np.uint8), flags)
     live = flags.astype(bool)
     rec = r.debug_read(R.DEBUG_TRI_RECORDS, np.uint32).reshape(-1, 16)[live]
+    # the mesh entry counts over the launch (the views before this one have two meshes each)
+    mesh = np.repeat(np.arange(len(sc.meshes)), [m.num_triangles for m in sc.meshes])[live]
+    np.testing.assert_array_equal(rec[:, 15] & 0x7FFFFFFF, mesh + first_mesh)
     np.testing.assert_array_equal(np.ascontiguousarray(rec[:, [0, 1, 2, 3, 4, 5, 6, 9, 8, 7, 10, 11]]),
                                   np.ascontiguousarray(orec[live]).view(np.uint32))
 
@@ -90,7 +93,7 @@ def test_views_of_one_scene(kind):
             R.render_batch([(r, cam, opts, R.BIN_EXACT, 0) for r, cam in zip(rs, cams)])
             for r, cam in list(zip(rs, cams))[:5] + list(zip(rs, cams))[12:]:
                 check_frame(r.readback(), sc, cam, opts)
-            check_debug(rs[13], sc, cams[13], opts, attributes=False)
+            check_debug(rs[13], sc, cams[13], opts, attributes=False, first_mesh=26)
     finally:
         for r in rs[:0:-1]:
             r.close()
