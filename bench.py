@@ -12,7 +12,7 @@ inputs are resident in HBM when the timed region starts.  Binning parameters com
 (custom-gpgpu-rasterizer_amd/tuning.json) unless given on the command line.
 
 Prints one JSON line: whole-frame Mtris/s (value) for learned single-pass
-binning, the same for exact two-pass binning and for the previous-frame
+binning, the same for exact binning and for the previous-frame
 heuristic, the plain configuration (every triangle binned, no setup-time
 raster) for the binner comparison, shaded Gpix/s, the shading pass against
 the HBM roofline (algorithmic bytes from the committed fixture

@@ -220,7 +220,7 @@ def train_bucket_model(R, jobs, paths, frames: int = 24, log=None):
 
 def tune_queue(R, jobs, paths, frames: int = 16, reps: int = 5, log=None) -> Dict:
     """Fastest (margin, slack) per single-pass policy for one bucket;
-    exact two-pass binning timed alongside on the same frames."""
+    exact binning timed alongside on the same frames."""
     out = {"exact_ms_per_batch": round(time_path(R, jobs, paths, R.BIN_EXACT, frames, reps), 4)}
     model = train_bucket_model(R, jobs, paths, log=log)
     try:

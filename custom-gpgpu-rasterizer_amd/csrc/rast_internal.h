@@ -4,9 +4,8 @@
 // HBM layout of one frame (all device buffers owned by the renderer):
 //   ivert    per mesh, 14 floats / vertex (the 56-byte IVertex, as uploaded)
 //   pos4     float4 / global vertex: NDC x, y, z and clip w        (16 B)
-//   attr     4 x float4 / global vertex, each attribute times 1/w:
-//            u v 1/w n'.x | n'.yz tan'.xy | tan'.z vd | c.rgb 0
-//            (64 B; PBR shading reads the first 48 B)
+//   attr     3 x float4 / global vertex, each attribute times 1/w:
+//            u v 1/w n'.x | n'.yz tan'.xy | tan'.z vd (48 B)
 //   trirec   16 words / global triangle ID (written for the survivors that
 //            are binned or cover a pixel; k_setup<true> writes the others'):
 //            [0..5] screen x0,y0,x1,y1,x2,y2  [6..8] z0,z1,z2  [9] |area|
@@ -15,7 +14,7 @@
 //            bit 31 set where shading must follow the reference's operation
 //            order (a vertex near or behind the camera plane, or a mesh with
 //            large normals / tangents: the fused forms could drift there)
-//   alive    u8 / triangle
+//   alive    u8 / triangle (k_setup<true>: formed when it is read)
 //   tiles    count / offset / cursor / capacity u32 per tile, queue entries
 //            u32 triangle IDs, plus one screen-wide "big" list
 //   keys     u64 per pixel: (z bits << 32) | ~(id + 1), min = visible

@@ -14,11 +14,14 @@
 // CCR/ERenderer.cpp:544-554 applied in ascending triangle order.
 //
 // Pipeline (one launch per stage for all jobs and meshes of a launch):
-//   k_vertex   per vertex: clip/NDC position + shading attributes; beside
-//              it, the setup workgroups whose triangles' box is out of view, single-pass jobs' tile capacities and queue regions, and
-//              the reset of every job's per-tile counts (the frame counters
-//              start at zero with the launch's staging upload)
-//   k_setup    per triangle: assembly, cull, screen setup record; triangles
+//   k_chunk_views  views of large scenes: the views each vertex block may be in
+//   k_vertex   per vertex: clip/NDC position + shading attributes; beside it,
+//              the list of the triangle blocks that may be in view, predicted
+//              tile capacities and queue regions, and the reset of every job's
+//              per-tile counts (the frame counters start at zero with the
+//              launch's staging upload)
+//   k_setup    per triangle of a listed block: assembly, cull, screen setup
+//              record where one is read again; triangles
 //              whose bounding box has at most micro_limit pixels are
 //              rasterized on the spot with 64-bit atomic min into the key
 //              buffer; larger ones are written straight into per-tile queues
@@ -26,9 +29,9 @@
 //              spanning more than big_threshold tiles go to one screen list
 //   k_place    queue regions from the exact counts
 //   k_fill     second pass over the binned triangles (two-pass jobs)
-//   k_resolve  one workgroup per tile: keys -> LDS (and cleared for the next
-//              frame), queued triangles rasterized in LDS (single pass: a
-//              tile whose count exceeded its capacity first gathers its
+//   k_resolve  one workgroup per tile (k_resolve_quarters: per quarter): keys
+//              (cleared for the next frame), queued triangles rasterized in LDS
+//              (a tile whose count exceeded its region first gathers its
 //              remaining entries from the overflow list), vis/depth written
 //   k_shade    per pixel, deferred from the visibility buffer; one instance per
 //              sampling mode; its first block of each job publishes the
