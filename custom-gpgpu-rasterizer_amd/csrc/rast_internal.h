@@ -121,11 +121,12 @@ struct FrameCounters {
     uint32_t num_big;
     uint32_t total_pairs;     // exact queue entries (sum of per-tile counts; formed when published)
     uint32_t overflow_tiles;  // single pass: tiles whose count exceeded capacity
-    uint32_t ovf_entries;     // single pass: queue entries beyond capacity (fallback input)
+    uint32_t ovf_entries;     // single pass: queue entries beyond capacity (and spill region) on the overflow list
     uint32_t pool_used;       // fallback pool entries
     uint32_t storage_overflow;// queue / pool / big list storage exhausted -> frame invalid
     uint32_t capacity_total;  // single pass: capacities as used (their sum fits the queue storage)
     uint32_t capacity_wanted; // single pass: the capacities' sum before that bound (saturated)
+    uint32_t spilled;         // entries beyond capacity that their tiles' spill regions took
     unsigned long long capacity_top;  // queue allocation top: the full sum of the capacities (single pass,
                                       // the two fields above are derived from it when published) or counts
 };
@@ -142,6 +143,7 @@ struct alignas(16) JobDesc {  // 16-byte multiple: staged in 16-byte words
     uint32_t single;             // the tiles' queue regions are known before setup: it fills them directly
     uint32_t stride;             // entries of every tile's region, at tile * stride (0: tile_off, tile_cap)
     uint32_t learned;            // capacities from the MLP (else previous count * margin + slack)
+    uint32_t spill_stride;       // previous-frame capacities: entries of every tile's spill region (0: none)
     uint32_t small_limit;        // tile-clipped pixel count from which resolve goes pixel-parallel (at least half a tile)
     float margin;
     uint32_t slack;
@@ -170,6 +172,7 @@ struct alignas(16) JobDesc {  // 16-byte multiple: staged in 16-byte words
     const uint32_t *prev_count;  // previous frame's exact per-tile counts
     const float *prev_depth;     // previous frame's per-tile min depth
     uint32_t *queue;
+    uint32_t *spill;             // tile t's first spill_stride entries beyond capacity, at t * spill_stride
     uint32_t *pool;
     uint2 *ovf;                  // single pass: (tile, id) entries beyond capacity
     uint32_t *survivors;

@@ -1084,17 +1084,19 @@ __device__ __forceinline__ uint2 tile_region(const JobDesc &J, uint32_t tl)
     return make_uint2(ldg(J.tile_off + tl), ldg(J.tile_cap + tl));
 }
 
-// Writes entry `slot` of tile tl's queue; one past its capacity is kept for
-// the exact fallback (one atomic on the shared counter per wave).
+// Writes entry `slot` of tile tl's queue; one past its capacity goes to the
+// tile's spill region, if it has one, or is kept for the exact fallback (one
+// atomic on the shared counter per wave).
 __device__ __forceinline__ void queue_entry(const JobDesc &J, uint32_t tl, uint32_t gid, uint32_t slot, uint32_t off,
                                             uint32_t cap)
 {
-    const bool fits = slot < cap;
-    const uint64_t om = __ballot(!fits);
-    if (fits) {
+    if (slot < cap) {
         const uint32_t pos = off + slot;
         if (pos < J.queue_cap) stg(J.queue + pos, gid);
+    } else if (slot - cap < J.spill_stride) {
+        stg(J.spill + tl * J.spill_stride + (slot - cap), gid);
     } else {
+        const uint64_t om = __ballot(true);  // the lanes here
         const int leader = __builtin_ctzll(om);
         uint32_t base = 0;
         if (lane_id() == (uint32_t)leader) base = gatomic_add(&J.counters->ovf_entries, (uint32_t)__popcll(om));
@@ -1581,7 +1583,8 @@ __global__ __launch_bounds__(256) void k_fill(const JobDesc *__restrict__ jobs, 
     }
 }
 
-// Single-pass fallback of the previous-frame policy, step 1 (per tile): the
+// Single-pass fallback of the previous-frame policy where it has no spill
+// regions, step 1 (per tile): the
 // exact count of a tile is its final fill cursor; the entries beyond its
 // capacity get a pool region.  The block allocates for its 256 tiles with one
 // atomic and adds its overflowing tiles with one more (no per-wave traffic
@@ -1985,20 +1988,30 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, ui
         }
     }
 
-    // List A: the tile's queue region.  List B: for single-pass binning,
-    // the tile's entries beyond its capacity, which setup appended to the
-    // overflow list as (tile, id) pairs.  Learned and fixed capacities: the
-    // tile's block gathers them itself into a pool region it allocates (one atomic
-    // per overflowing tile; the list is read four entries per thread at a
-    // time), so no placement pass runs.  Previous-frame capacities: the
-    // fallback passes placed them in the tile's pool region.  The order of a
-    // tile's entries does not change the frame (the depth keys order
-    // fragments by depth, then ID).
+    // List A: the tile's queue region.  List B: for single-pass binning, the
+    // tile's entries beyond its capacity.  Previous-frame capacities: the tile's
+    // spill region, where setup put them.  What that has no room for, and for
+    // learned and fixed capacities all of them, setup appended to the overflow
+    // list as (tile, id) pairs, from which the tile's block gathers them itself
+    // into a pool region it allocates (one atomic per overflowing tile; the list
+    // is read four entries per thread at a time), so no placement pass runs.
+    // Frames without room for spill regions: the fallback passes placed the
+    // entries in the tile's pool region.  The order of a tile's entries does not
+    // change the frame (the depth keys order fragments by depth, then ID).
     uint32_t n_a = cnt, n_b = 0;
     const uint32_t *list_a = queue + qoff;
     const uint32_t *list_b = pool;
-    if (J.single) {
-        if (cnt > cp && !J.learned && !J.stride) {
+    if (J.single && cnt > cp) {  // the same for the whole block
+        const uint32_t spill_stride = J.spill_stride;
+        uint32_t *const spill = J.spill + (size_t)tile * spill_stride;
+        if (spill_stride && tid == 0 && part == 0)
+            gatomic_add(&ctr->spilled, cnt - cp < spill_stride ? cnt - cp : spill_stride);
+        if (cnt - cp <= spill_stride) {
+            n_a = cp;
+            n_b = cnt - cp;
+            list_b = spill;
+            if (tid == 0 && part == 0) gatomic_add(&ctr->overflow_tiles, 1u);
+        } else if (!J.learned && !J.stride && !spill_stride) {
             n_a = cp;
             const uint32_t po = ldg(tile_pool + tile);
             if (po != 0xFFFFFFFFu) {
@@ -2007,7 +2020,7 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, ui
                 n_b = cnt - cp;
                 n_b = n_b < room_b ? n_b : room_b;
             }
-        } else if (cnt > cp) {  // the same for the whole block
+        } else {
             n_a = cp;
             const uint32_t want = cnt - cp;
             if (tid == 0) {
@@ -2015,10 +2028,12 @@ __device__ __forceinline__ void resolve_tile(const JobDesc &J, uint32_t tile, ui
                 if (b + want > pool_cap || b + want < b) ctr->storage_overflow = 1;
                 if (part == 0) gatomic_add(&ctr->overflow_tiles, 1u);
                 ovf_base = b;
-                ovf_fill = 0;
+                ovf_fill = spill_stride;  // the spill region's entries come first
             }
             __syncthreads();
             const uint32_t pbase = ovf_base;
+            for (uint32_t i = tid; i < spill_stride; i += NT)
+                if (pbase + i < pool_cap) stg(pool + pbase + i, ldg(spill + i));
             uint32_t ne = ldg(&ctr->ovf_entries);
             ne = ne < J.ovf_cap ? ne : J.ovf_cap;
             for (uint32_t b0 = 0; b0 < ne; b0 += 4u * NT) {

@@ -175,6 +175,8 @@ struct rast_renderer {
     uint32_t frame_w = 0, frame_h = 0, frame_mesh0 = 0;
     int32_t frame_cull = 0;
     bool last_single = false;              // capacities predicted (single-pass policies)
+    uint32_t last_spill = 0;               // previous-frame capacities: entries of every tile's spill region
+    uint32_t last_queue = 0;               // queue storage in front of the spill regions
     uint32_t last_stride = 0;              // exact binning into fixed regions of this many entries (0: two passes)
     bool two_pass = false;                 // the scene overflowed its fixed regions: exact frames take two passes
     bool last_shared_attr = false;  // the last frame's attributes were split (views rendered together)
