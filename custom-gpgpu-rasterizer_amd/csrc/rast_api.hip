@@ -368,7 +368,7 @@ extern "C" int rast_setup_bins(rast_renderer *r, uint32_t tile_size, uint32_t bi
     r->tile = tile_size;
     r->big_threshold = big_threshold ? big_threshold : 256;
     r->have_prev = false;
-    r->two_pass = false;
+    r->two_pass = r->no_spill = false;
     return RAST_OK;
 }
 
@@ -379,7 +379,7 @@ extern "C" int rast_set_tuning(rast_renderer *r, uint32_t micro_limit, uint32_t 
         return rast_set_error(RAST_E_INVALID_ARG, "micro_limit %u / small_limit %u above 1024", micro_limit, small_limit);
     r->micro_limit = micro_limit;
     r->small_limit = small_limit;
-    r->two_pass = false;
+    r->two_pass = r->no_spill = false;
     return RAST_OK;
 }
 
@@ -401,7 +401,7 @@ extern "C" int rast_resize(rast_renderer *r, uint32_t width, uint32_t height)
     r->W = width;
     r->H = height;
     r->have_prev = false;
-    r->two_pass = false;
+    r->two_pass = r->no_spill = false;
     return alloc_framebuffers(r);
 }
 
@@ -633,7 +633,7 @@ static void refresh_layout(rast_renderer *r)
     r->total_tris = (uint32_t)tb;
     r->layout_version = scene_owner(r)->scene_version;
     r->have_prev = false;
-    r->two_pass = false;
+    r->two_pass = r->no_spill = false;
 }
 
 // Exact binning in one pass: where the queue storage gives every tile a fixed
@@ -666,7 +666,7 @@ constexpr uint32_t kSpill = 512, kSpillMin = 128;
 static uint32_t spill_stride(const rast_renderer *r, uint32_t ntiles)
 {
     const uint32_t s = std::min(r->queue_cap / 2 / ntiles, kSpill);
-    return s < kSpillMin || r->two_pass ? 0u : s;
+    return s < kSpillMin || r->no_spill ? 0u : s;
 }
 
 static int ensure_frame_storage(rast_renderer *r, uint32_t ntiles)
@@ -1542,7 +1542,10 @@ static int check_frame(rast_renderer *r)
             // single-pass capacities beyond the queue storage were cut to fit
             // (the frame is exact all the same); the next frame gets room
             // for them, up to 2^28 entries
-            if ((r->last_stride || r->last_spill) && c.ovf_entries > kFixedOverflowMax) r->two_pass = true;
+            if (c.ovf_entries > kFixedOverflowMax) {
+                if (r->last_stride) r->two_pass = true;
+                if (r->last_spill) r->no_spill = true;
+            }
             if (r->last_single && c.capacity_wanted > r->last_queue && r->queue_cap < kQueueGrowLimit)
                 r->queue_cap = (uint32_t)std::min<uint64_t>((uint64_t)c.capacity_wanted * 5 / 4 + 1024 + (r->queue_cap - r->last_queue), kQueueGrowLimit);
             return RAST_OK;

@@ -179,6 +179,7 @@ struct rast_renderer {
     uint32_t last_queue = 0;               // queue storage in front of the spill regions
     uint32_t last_stride = 0;              // exact binning into fixed regions of this many entries (0: two passes)
     bool two_pass = false;                 // the scene overflowed its fixed regions: exact frames take two passes
+    bool no_spill = false;                 // the scene overflowed its spill regions: placed by two passes
     bool last_shared_attr = false;  // the last frame's attributes were split (views rendered together)
     bool prev_valid_before = false;
     bool frame_had_prev = false;  // the last frame had a previous frame (features valid)

@@ -55,3 +55,20 @@ def test_overflowing_tiles(tile, size):
                 assert st["overflow_tiles"] == np.count_nonzero(over)
                 most = max(most, int(over.max()))
         assert most > 0
+
+
+def test_frames_after_a_camera_cut():
+    """The frame after a cut overflows its spill regions; later exact frames of
+    the same view and further previous-frame ones stay the exact frame."""
+    scene, opts = S.Scene([S.terrain(260)]), S.Opts(cull_mode=S.CULL_NONE)
+    with R.Renderer(W, H, tile=32, big_threshold=1024) as r:
+        r.set_tuning(0, 16)
+        r.add_scene(scene)
+        r.render(NEAR, opts, R.BIN_EXACT)
+        want = planes(r)
+        r.set_queue_depth(1.0, 0)
+        r.render(SKY, opts, R.BIN_EXACT, R.FLAG_NO_SHADE)
+        for policy in (R.BIN_PREVFRAME, R.BIN_EXACT, R.BIN_PREVFRAME, R.BIN_EXACT):
+            r.render(NEAR, opts, policy)
+            for a, b in zip(planes(r), want):
+                np.testing.assert_array_equal(a, b)
