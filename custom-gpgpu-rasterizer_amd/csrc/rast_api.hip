@@ -331,7 +331,7 @@ extern "C" int rast_renderer_destroy(rast_renderer *r)
         v.erase(std::remove(v.begin(), v.end(), r), v.end());
     }
     plan_free(r->plan);
-    rast_model_detach_renderer(r->model, r);
+    rast_model_renderer_gone(r);
     // Mesh and texture handles outlive the renderer as empty handles: their
     // device memory goes now, the handle itself with rast_mesh_destroy /
     // rast_texture_destroy, so a caller may destroy the renderer before the
@@ -1809,7 +1809,7 @@ extern "C" int rast_renderer_set_binmodel(rast_renderer *r, rast_binmodel *m, fl
     if (!r) return rast_set_error(RAST_E_INVALID_ARG, "rast_renderer_set_binmodel: null renderer");
     if (!(margin >= 1.f) || margin > 64.f) return rast_set_error(RAST_E_INVALID_ARG, "margin %g not in [1, 64]", margin);
     if (slack > (1u << 20)) return rast_set_error(RAST_E_INVALID_ARG, "slack %u above 2^20", slack);
-    r->model = m;
+    RAST_TRY(rast_model_attach(r, m));
     r->margin = margin;
     r->slack = slack;
     return RAST_OK;

@@ -360,15 +360,20 @@ uint32_t cdiv(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 struct rast_binmodel {
     int device = 0;
     int H = 64;
-    hipStream_t stream = nullptr;
+    hipStream_t stream = nullptr;    // home's; the model's own once that renderer is gone
+    rast_renderer *home = nullptr;   // the renderer it was created on, while that exists
     DBuf params, grad, adam_m, adam_v;
     DBuf X, Y;            // recorded training set
     uint32_t n = 0, cap = 0;
     DBuf partial, loss, io_x, io_y, io_p;  // partial: per workgroup gradients + loss
     uint32_t batch_cap = 0;
     uint64_t adam_t = 0;
-    std::vector<rast_renderer *> users;
+    std::vector<rast_renderer *> users;  // the renderers it is attached to
 };
+
+// Guards every model's users and home, and every renderer's models: a model
+// serves renderers that different threads may attach and destroy.
+static std::mutex g_models_mutex;
 
 namespace rast_detail {
 
@@ -463,11 +468,50 @@ hipError_t launch_tile_features(const FrameParams &fp, const uint32_t *prev_coun
 }  // namespace rast
 
 
-void rast_model_detach_renderer(rast_binmodel *m, rast_renderer *r)
+// r is no longer one of its model's users (g_models_mutex is held).
+static void forget_user(rast_renderer *r)
 {
-    if (!m) return;
-    for (auto &u : m->users)
-        if (u == r) u = nullptr;
+    if (!r->model) return;
+    auto &u = r->model->users;
+    u.erase(std::remove(u.begin(), u.end(), r), u.end());
+    r->model = nullptr;
+}
+
+int rast_model_attach(rast_renderer *r, rast_binmodel *m)
+{
+    if (r->model == m) return RAST_OK;
+    if (r->model) {  // frames still queued read it, and it may be destroyed from here on
+        HIP_TRY(hipSetDevice(r->device));
+        RAST_TRY(rast_settle(r));
+    }
+    std::lock_guard<std::mutex> lock(g_models_mutex);
+    try {
+        if (m) m->users.push_back(r);
+    } catch (const std::bad_alloc &) {
+        return rast_set_error(RAST_E_OUT_OF_MEMORY, "host allocation failed");
+    }
+    forget_user(r);
+    r->model = m;
+    return RAST_OK;
+}
+
+void rast_model_renderer_gone(rast_renderer *r)
+{
+    std::lock_guard<std::mutex> lock(g_models_mutex);
+    forget_user(r);
+    for (rast_binmodel *m : r->models) {
+        m->home = nullptr;
+        m->stream = nullptr;  // made by its next use (model_ready)
+    }
+    r->models.clear();
+}
+
+// Makes the model's device current and sees that it has a stream.
+static int model_ready(rast_binmodel *m)
+{
+    HIP_TRY(hipSetDevice(m->device));
+    if (!m->stream) HIP_TRY(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
+    return RAST_OK;
 }
 
 // --------------------------------------------------------------------- ABI
@@ -503,6 +547,14 @@ extern "C" int rast_binmodel_create(rast_renderer *r, uint32_t hidden, uint32_t 
     if (!m) return rast_set_error(RAST_E_OUT_OF_MEMORY, "host allocation failed");
     m->device = r->device;
     m->H = (int)hidden;
+    try {
+        std::lock_guard<std::mutex> lock(g_models_mutex);
+        r->models.push_back(m);
+    } catch (const std::bad_alloc &) {
+        delete m;
+        return rast_set_error(RAST_E_OUT_OF_MEMORY, "host allocation failed");
+    }
+    m->home = r;
     m->stream = r->stream;
     const size_t np = num_params(m->H);
     std::vector<float> p(np);
@@ -518,7 +570,6 @@ extern "C" int rast_binmodel_create(rast_renderer *r, uint32_t hidden, uint32_t 
         rast_binmodel_destroy(m);
         return rast_set_error(rc, "rast_binmodel_create: allocation failed");
     }
-    m->users.push_back(r);
     *out = m;
     return RAST_OK;
 }
@@ -527,11 +578,20 @@ extern "C" int rast_binmodel_destroy(rast_binmodel *m)
 {
     if (!m) return rast_set_error(RAST_E_INVALID_ARG, "rast_binmodel_destroy: null model");
     (void)hipSetDevice(m->device);
-    for (rast_renderer *r : m->users)
-        if (r) {
+    {
+        std::lock_guard<std::mutex> lock(g_models_mutex);
+        for (rast_renderer *r : m->users) {
             (void)rast_settle(r);
-            if (r->model == m) r->model = nullptr;
+            r->model = nullptr;
         }
+        if (m->home) {
+            (void)rast_settle(m->home);
+            auto &v = m->home->models;
+            v.erase(std::remove(v.begin(), v.end(), m), v.end());
+        }
+    }
+    if (m->stream) (void)hipStreamSynchronize(m->stream);
+    if (m->stream && !m->home) (void)hipStreamDestroy(m->stream);
     DBuf *bufs[] = { &m->params, &m->grad, &m->adam_m, &m->adam_v, &m->X, &m->Y, &m->partial, &m->loss,
                      &m->io_x, &m->io_y, &m->io_p };
     for (DBuf *b : bufs) dfree(*b);
@@ -550,7 +610,7 @@ extern "C" int rast_binmodel_get_params(rast_binmodel *m, float *dst, size_t cou
 {
     if (!m || !dst || count != num_params(m->H))
         return rast_set_error(RAST_E_INVALID_ARG, "rast_binmodel_get_params: bad arguments");
-    HIP_TRY(hipSetDevice(m->device));
+    RAST_TRY(model_ready(m));
     HIP_TRY(hipStreamSynchronize(m->stream));
     HIP_TRY(hipMemcpy(dst, m->params.p, count * 4, hipMemcpyDeviceToHost));
     return RAST_OK;
@@ -560,7 +620,7 @@ extern "C" int rast_binmodel_set_params(rast_binmodel *m, const float *src, size
 {
     if (!m || !src || count != num_params(m->H))
         return rast_set_error(RAST_E_INVALID_ARG, "rast_binmodel_set_params: bad arguments");
-    HIP_TRY(hipSetDevice(m->device));
+    RAST_TRY(model_ready(m));
     HIP_TRY(hipStreamSynchronize(m->stream));
     HIP_TRY(hipMemcpy(m->params.p, src, count * 4, hipMemcpyHostToDevice));
     HIP_TRY(hipMemset(m->adam_m.p, 0, count * 4));
@@ -583,7 +643,7 @@ extern "C" int rast_binmodel_record(rast_binmodel *m, rast_renderer *r)
     if (!r->frame_valid || !r->frame_had_prev || r->model != m)
         return rast_set_error(RAST_E_STATE,
                               "rast_binmodel_record: needs two consecutive frames rendered with this model attached");
-    HIP_TRY(hipSetDevice(m->device));
+    RAST_TRY(model_ready(m));
     const uint32_t tx = (r->W + r->tile - 1) / r->tile, ty = (r->H + r->tile - 1) / r->tile, nt = tx * ty;
     if ((uint64_t)m->n + nt > 0x7FFFFFFFull) return rast_set_error(RAST_E_STATE, "training set full");
     if (m->n + nt > m->cap) {
@@ -630,7 +690,7 @@ extern "C" int rast_binmodel_train(rast_binmodel *m, uint32_t epochs, uint32_t b
     if (!m || batch == 0 || batch > kMaxBatch || !(lr > 0.f) || !(tau > 0.f && tau < 1.f))
         return rast_set_error(RAST_E_INVALID_ARG, "rast_binmodel_train: bad arguments");
     if (m->n == 0) return rast_set_error(RAST_E_STATE, "rast_binmodel_train: no recorded data");
-    HIP_TRY(hipSetDevice(m->device));
+    RAST_TRY(model_ready(m));
     RAST_TRY(ensure_batch(m, batch));
     const uint32_t steps = std::max<uint32_t>(1, (uint32_t)(((uint64_t)m->n * epochs + batch - 1) / batch));
     for (uint32_t st = 0; st < steps; ++st) {
@@ -648,7 +708,7 @@ extern "C" int rast_binmodel_train(rast_binmodel *m, uint32_t epochs, uint32_t b
 extern "C" int rast_binmodel_forward(rast_binmodel *m, const float *x, uint32_t n, float *pred)
 {
     if (!m || !x || !pred || n == 0) return rast_set_error(RAST_E_INVALID_ARG, "rast_binmodel_forward: bad arguments");
-    HIP_TRY(hipSetDevice(m->device));
+    RAST_TRY(model_ready(m));
     RAST_TRY(ensure(m->io_x, (size_t)n * F * 4));
     RAST_TRY(ensure(m->io_p, (size_t)n * 4));
     HIP_TRY(hipMemcpy(m->io_x.p, x, (size_t)n * F * 4, hipMemcpyHostToDevice));
@@ -709,7 +769,7 @@ extern "C" int rast_binmodel_forward_noalloc(rast_binmodel *m, const float *x, u
         return rast_set_error(RAST_E_INVALID_ARG, "rast_binmodel_forward_noalloc: %u samples above the maximum %u", n,
                               kNoAllocMaxSamples);
     std::lock_guard<std::mutex> lock(g_noalloc.mu);
-    HIP_TRY(hipSetDevice(m->device));
+    RAST_TRY(model_ready(m));
     float *base = nullptr;
     RAST_TRY(noalloc_scratch(m->device, &base));
     float *sx = base, *sp = base + (size_t)kNoAllocMaxSamples * F;
@@ -726,7 +786,7 @@ extern "C" int rast_binmodel_loss_grad(rast_binmodel *m, const float *x, const f
 {
     if (!m || !x || !target || !grad || n == 0 || n > kMaxBatch)
         return rast_set_error(RAST_E_INVALID_ARG, "rast_binmodel_loss_grad: bad arguments");
-    HIP_TRY(hipSetDevice(m->device));
+    RAST_TRY(model_ready(m));
     RAST_TRY(ensure(m->io_x, (size_t)n * F * 4));
     RAST_TRY(ensure(m->io_y, (size_t)n * 4));
     HIP_TRY(hipMemcpy(m->io_x.p, x, (size_t)n * F * 4, hipMemcpyHostToDevice));

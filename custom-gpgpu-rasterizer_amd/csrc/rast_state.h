@@ -187,6 +187,7 @@ struct rast_renderer {
     rast_stats stats{};
     // learned capacities
     rast_binmodel *model = nullptr;
+    std::vector<rast_binmodel *> models;   // those created on it
     float margin = 1.25f;
     uint32_t slack = 4;
 };

@@ -28,3 +28,27 @@ def _built_libraries():
     if not os.path.exists(os.path.join(PKG, "lib", "librast_scenes.so")):
         pkg_build.build_scenes()
     yield
+
+
+@pytest.fixture(scope="session")
+def host_library(tmp_path_factory):
+    """The library's host code over the stand-in HIP runtime of tests/hipstub."""
+    sys.path.insert(0, os.path.join(ROOT, "tests", "hipstub"))
+    import hipstub
+
+    if not os.path.exists(hipstub.HIPCC):
+        pytest.skip("no hipcc")
+    return hipstub.build(str(tmp_path_factory.mktemp("hipstub")))
+
+
+@pytest.fixture
+def host(host_library, monkeypatch):
+    """`rast` bound to that library for one test, and the runtime's handle."""
+    import hipstub
+    import rast as R
+
+    monkeypatch.setattr(R, "LIB_PATH", host_library)
+    monkeypatch.setattr(R, "_lib", None)
+    rt = hipstub.Runtime(R.lib())
+    yield rt
+    rt.limit(None)
