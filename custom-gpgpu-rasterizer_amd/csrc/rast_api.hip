@@ -360,6 +360,14 @@ extern "C" int rast_renderer_destroy(rast_renderer *r)
     return RAST_OK;
 }
 
+// What earlier frames left beyond their regions says nothing about the next one.
+static void forget_overflow(rast_renderer *r)
+{
+    r->two_pass = r->no_spill = 0;
+    __atomic_store_n(&r->h_counters->past_fixed, kNotMeasured, __ATOMIC_RELAXED);
+    __atomic_store_n(&r->h_counters->past_spill, kNotMeasured, __ATOMIC_RELAXED);
+}
+
 extern "C" int rast_setup_bins(rast_renderer *r, uint32_t tile_size, uint32_t big_threshold)
 {
     if (!r) return rast_set_error(RAST_E_INVALID_ARG, "rast_setup_bins: null renderer");
@@ -368,7 +376,7 @@ extern "C" int rast_setup_bins(rast_renderer *r, uint32_t tile_size, uint32_t bi
     r->tile = tile_size;
     r->big_threshold = big_threshold ? big_threshold : 256;
     r->have_prev = false;
-    r->two_pass = r->no_spill = false;
+    forget_overflow(r);
     return RAST_OK;
 }
 
@@ -379,7 +387,7 @@ extern "C" int rast_set_tuning(rast_renderer *r, uint32_t micro_limit, uint32_t 
         return rast_set_error(RAST_E_INVALID_ARG, "micro_limit %u / small_limit %u above 1024", micro_limit, small_limit);
     r->micro_limit = micro_limit;
     r->small_limit = small_limit;
-    r->two_pass = r->no_spill = false;
+    forget_overflow(r);
     return RAST_OK;
 }
 
@@ -401,7 +409,7 @@ extern "C" int rast_resize(rast_renderer *r, uint32_t width, uint32_t height)
     r->W = width;
     r->H = height;
     r->have_prev = false;
-    r->two_pass = r->no_spill = false;
+    forget_overflow(r);
     return alloc_framebuffers(r);
 }
 
@@ -633,7 +641,7 @@ static void refresh_layout(rast_renderer *r)
     r->total_tris = (uint32_t)tb;
     r->layout_version = scene_owner(r)->scene_version;
     r->have_prev = false;
-    r->two_pass = r->no_spill = false;
+    forget_overflow(r);
 }
 
 // Exact binning in one pass: where the queue storage gives every tile a fixed
@@ -643,15 +651,15 @@ static void refresh_layout(rast_renderer *r)
 // binned triangles and the placement before it (480p frame of 4,032
 // triangles: 3.2 + 6.7 us of 51, its frame 64.6 -> 50.5; 8K terrain: 5.6 + 22,
 // resolve 10 us more, its frame 720 -> 678).  Two passes remain for
-// frames of so many tiles that the regions would be shorter, and for a
-// renderer whose last checked frame left more than kFixedOverflowMax entries
-// beyond them: each overflowing tile reads that list once.
-constexpr uint32_t kFixedRegion = 1024, kFixedRegionMin = 512, kFixedOverflowMax = 1u << 15;
+// frames of so many tiles that the regions would be shorter, and after a frame
+// that left more than kOverflowMax entries beyond them (note_overflow): each
+// overflowing tile reads that list once.
+constexpr uint32_t kFixedRegion = 1024, kFixedRegionMin = 512;
 
 static uint32_t fixed_stride(const rast_renderer *r, uint32_t ntiles)
 {
     const uint32_t s = r->queue_cap / ntiles;
-    return s < kFixedRegionMin || r->two_pass ? 0u : std::min(s, std::max<uint32_t>(r->total_tris, 1u));
+    return s < kFixedRegionMin ? 0u : std::min(s, std::max<uint32_t>(r->total_tris, 1u));
 }
 
 // Previous-frame capacities: half of the queue storage gives every tile a spill
@@ -659,14 +667,35 @@ static uint32_t fixed_stride(const rast_renderer *r, uint32_t ntiles)
 // capacity as setup writes them.  Without it two passes place them from the
 // overflow list (9.4 us of a frame: 2561 x 1439 terrain 165 -> 155 us, 1.3 M
 // triangles without shading 107 -> 98); they remain for frames of so many
-// tiles that the regions would be shorter, and for a renderer whose last checked
-// frame left more than kFixedOverflowMax entries beyond them.
+// tiles that the regions would be shorter, and after a frame that left more than
+// kOverflowMax entries beyond them.
 constexpr uint32_t kSpill = 512, kSpillMin = 128;
 
 static uint32_t spill_stride(const rast_renderer *r, uint32_t ntiles)
 {
     const uint32_t s = std::min(r->queue_cap / 2 / ntiles, kSpill);
-    return s < kSpillMin || r->no_spill ? 0u : s;
+    return s < kSpillMin ? 0u : s;
+}
+
+// A frame that left more than kOverflowMax entries beyond its regions makes the
+// following ones take two passes, until kFitFrames in a row would have fitted (a
+// frame of two passes measures that too).  The counters are those of the last
+// frame that has ended, read or not: a later frame's may just be arriving, which
+// moves the change by a frame at most.
+constexpr uint32_t kOverflowMax = 1u << 15, kFitFrames = 16;
+
+static bool past_regions(uint32_t past) { return past != kNotMeasured && past > kOverflowMax; }
+
+static void note_overflow(uint32_t &left, uint32_t past)
+{
+    if (past_regions(past)) left = kFitFrames;
+    else if (past != kNotMeasured && left) --left;
+}
+
+static void note_overflow(rast_renderer *r)
+{
+    note_overflow(r->two_pass, __atomic_load_n(&r->h_counters->past_fixed, __ATOMIC_RELAXED));
+    note_overflow(r->no_spill, __atomic_load_n(&r->h_counters->past_spill, __ATOMIC_RELAXED));
 }
 
 static int ensure_frame_storage(rast_renderer *r, uint32_t ntiles)
@@ -805,6 +834,7 @@ static int prepare_job(rast_renderer *r)
     HIP_TRY(hipSetDevice(r->device));
     if (scene_meshes(r).empty()) return rast_set_error(RAST_E_STATE, "rast_render: no meshes loaded");
     RAST_TRY(note_scene(r));
+    note_overflow(r);
     if (r->layout_version != scene_owner(r)->scene_version) refresh_layout(r);
     RAST_TRY(ensure_tex_quads(r));
     const uint32_t ntiles = ceil_div(r->W, r->tile) * ceil_div(r->H, r->tile);
@@ -813,8 +843,13 @@ static int prepare_job(rast_renderer *r)
     bool single = r->last_opts.bin_policy != RAST_BIN_EXACT && r->have_prev;
     if (r->last_opts.bin_policy == RAST_BIN_LEARNED && !r->model) single = false;
     r->last_single = single;
-    r->last_stride = single ? 0u : fixed_stride(r, ntiles);
-    r->last_spill = single && r->last_opts.bin_policy == RAST_BIN_PREVFRAME ? spill_stride(r, ntiles) : 0u;
+    // regions of known length, or two passes that measure what those would do
+    const uint32_t regions = !single ? fixed_stride(r, ntiles)
+                             : r->last_opts.bin_policy == RAST_BIN_PREVFRAME ? spill_stride(r, ntiles) : 0u;
+    const bool passes = (single ? r->no_spill : r->two_pass) != 0;
+    r->last_stride = single || passes ? 0u : regions;
+    r->last_spill = single && !passes ? regions : 0u;
+    r->last_trial = passes ? regions : 0u;
     r->last_queue = r->queue_cap - ntiles * r->last_spill;
     return RAST_OK;
 }
@@ -1221,6 +1256,7 @@ static int stage_launch(LaunchPlan &P, rast_renderer *const *rs, uint32_t n)
         J.slack = r->slack;
         J.queue_cap = r->last_queue;
         J.spill_stride = r->last_spill;
+        J.trial_stride = r->last_trial;
         J.spill = (uint32_t *)r->queue.p + r->last_queue;
         J.pool_cap = r->pool_cap;
         J.big_cap = r->big_cap;
@@ -1542,19 +1578,22 @@ static int check_frame(rast_renderer *r)
             // single-pass capacities beyond the queue storage were cut to fit
             // (the frame is exact all the same); the next frame gets room
             // for them, up to 2^28 entries
-            if (c.ovf_entries > kFixedOverflowMax) {
-                if (r->last_stride) r->two_pass = true;
-                if (r->last_spill) r->no_spill = true;
-            }
             if (r->last_single && c.capacity_wanted > r->last_queue && r->queue_cap < kQueueGrowLimit)
                 r->queue_cap = (uint32_t)std::min<uint64_t>((uint64_t)c.capacity_wanted * 5 / 4 + 1024 + (r->queue_cap - r->last_queue), kQueueGrowLimit);
             return RAST_OK;
         }
         const uint64_t need_q = std::max<uint64_t>(c.total_pairs, c.capacity_total);
         if (need_q >= r->queue_cap) r->queue_cap = (uint32_t)std::min<uint64_t>(need_q + need_q / 4 + 1024, 0xFFFFFFF0ull);
-        if (c.pool_used >= r->pool_cap) r->pool_cap = (uint32_t)std::min<uint64_t>((uint64_t)c.pool_used * 5 / 4 + 1024, 0xFFFFFFF0ull);
         if (c.num_big >= r->big_cap) r->big_cap = (uint32_t)std::min<uint64_t>((uint64_t)c.num_big * 5 / 4 + 1024, 0xFFFFFFF0ull);
-        if (c.ovf_entries >= r->ovf_cap) r->ovf_cap = (uint32_t)std::min<uint64_t>((uint64_t)c.ovf_entries * 5 / 4 + 1024, 0x1FFFFFF0ull);
+        // A frame far beyond its regions is not drawn again with a longer list,
+        // which every overflowing tile would read, but by two passes: after
+        // fixed regions they need no list, after spill regions one of all
+        // entries beyond the capacities.
+        uint64_t list = c.ovf_entries, pool = c.pool_used;
+        if (r->last_stride && past_regions(c.past_fixed)) list = pool = 0;
+        if (r->last_spill && past_regions(c.past_spill)) list = pool = list + c.spilled;
+        if (pool >= r->pool_cap) r->pool_cap = (uint32_t)std::min<uint64_t>(pool * 5 / 4 + 1024, 0xFFFFFFF0ull);
+        if (list >= r->ovf_cap) r->ovf_cap = (uint32_t)std::min<uint64_t>(list * 5 / 4 + 1024, 0x1FFFFFF0ull);
         r->cur ^= 1;  // redo the same frame into the same buffers
         r->have_prev = r->prev_valid_before;
         ++r->rerenders;

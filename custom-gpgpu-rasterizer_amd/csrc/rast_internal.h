@@ -114,6 +114,8 @@ enum Stage : int {
     ST_COUNT
 };
 
+constexpr uint32_t kNotMeasured = 0xFFFFFFFFu;
+
 // Device-side frame counters, read back once per frame.
 struct FrameCounters {
     uint32_t num_alive;       // survivors of culling
@@ -127,6 +129,9 @@ struct FrameCounters {
     uint32_t capacity_total;  // single pass: capacities as used (their sum fits the queue storage)
     uint32_t capacity_wanted; // single pass: the capacities' sum before that bound (saturated)
     uint32_t spilled;         // entries beyond capacity that their tiles' spill regions took
+    // entries beyond the fixed regions, and beyond the spill regions, of a frame
+    // that has them or that takes two passes in their place (kNotMeasured: neither)
+    uint32_t past_fixed, past_spill;
     unsigned long long capacity_top;  // queue allocation top: the full sum of the capacities (single pass,
                                       // the two fields above are derived from it when published) or counts
 };
@@ -144,6 +149,7 @@ struct alignas(16) JobDesc {  // 16-byte multiple: staged in 16-byte words
     uint32_t stride;             // entries of every tile's region, at tile * stride (0: tile_off, tile_cap)
     uint32_t learned;            // capacities from the MLP (else previous count * margin + slack)
     uint32_t spill_stride;       // previous-frame capacities: entries of every tile's spill region (0: none)
+    uint32_t trial_stride;       // a frame of two passes: the region it would have without them (0: none)
     uint32_t small_limit;        // tile-clipped pixel count from which resolve goes pixel-parallel (at least half a tile)
     float margin;
     uint32_t slack;

@@ -311,6 +311,9 @@ __device__ __forceinline__ void publish_counters(const JobDesc &J, uint32_t *red
     constexpr uint32_t kPairs = offsetof(FrameCounters, total_pairs) / 4;
     constexpr uint32_t kCapTotal = offsetof(FrameCounters, capacity_total) / 4;
     constexpr uint32_t kCapWanted = offsetof(FrameCounters, capacity_wanted) / 4;
+    constexpr uint32_t kOvf = offsetof(FrameCounters, ovf_entries) / 4;
+    constexpr uint32_t kPastFixed = offsetof(FrameCounters, past_fixed) / 4;
+    constexpr uint32_t kPastSpill = offsetof(FrameCounters, past_spill) / 4;
     const uint32_t alive = block_sum<NW>(J.alive_part + J.alive_part0, J.alive_parts, red);
     const uint32_t pairs = J.single ? block_sum<NW>(J.tile_count, J.fp.tiles_x * J.fp.tiles_y, red) : 0u;
     if (threadIdx.x < W) {
@@ -324,6 +327,9 @@ __device__ __forceinline__ void publish_counters(const JobDesc &J, uint32_t *red
             if (threadIdx.x == kCapTotal) v = (uint32_t)(top < J.queue_cap ? top : J.queue_cap);
             if (threadIdx.x == kCapWanted) v = top32;
         }
+        const uint32_t ovf = reinterpret_cast<const uint32_t *>(J.counters)[kOvf];
+        if (threadIdx.x == kPastFixed) v = J.stride ? ovf : !J.single && J.trial_stride ? v : kNotMeasured;
+        if (threadIdx.x == kPastSpill) v = J.spill_stride ? ovf : J.single && J.trial_stride ? v : kNotMeasured;
         reinterpret_cast<volatile uint32_t *>(J.host_counters)[threadIdx.x] = v;
     }
 }
@@ -1530,6 +1536,20 @@ __global__ __launch_bounds__(256) void k_setup(const DevMesh *__restrict__ meshe
     }
 }
 
+// Adds to *past the entries of the wave's tiles (all 64 lanes call it) beyond
+// the first J.trial_stride: whether the frame would fit regions of that many.  A
+// tile and a wave count for no more than kPastMax, so the sum over the at most
+// 65,536 waves of a frame holds in 32 bits.
+constexpr uint32_t kPastMax = 40000;
+
+__device__ __forceinline__ void add_past(const JobDesc &J, uint32_t n, uint32_t *past)
+{
+    if (!J.trial_stride) return;
+    const uint32_t over = n > J.trial_stride ? n - J.trial_stride : 0u;
+    const uint32_t sum = wave_incl_sum(over < kPastMax ? over : kPastMax);
+    if (lane_id() == 63u && sum) gatomic_add(past, sum < kPastMax ? sum : kPastMax);
+}
+
 // Queue regions of the two-pass jobs' tiles, from their exact counts (256
 // tiles per block); the fill cursors are zeroed on the way.  Counts beyond the
 // queue storage set storage_overflow (the frame is rendered again with a
@@ -1550,6 +1570,7 @@ __global__ __launch_bounds__(256) void k_place(const JobDesc *__restrict__ jobs,
         J.tile_cursor[t] = 0;
         if (start + c > limit) J.counters->storage_overflow = 1;
     }
+    add_past(J, (uint32_t)c, &J.counters->past_fixed);
 }
 
 // Exact second pass over the binned triangles (the order inside a queue is
@@ -1610,6 +1631,7 @@ __global__ __launch_bounds__(256) void k_fallback_alloc(const JobDesc *__restric
         const uint32_t c = count[t];
         excess = c > cap[t] ? c - cap[t] : 0;
     }
+    add_past(J, excess, &ctr->past_spill);
     // inclusive wave prefix of the excess; wave total of overflowed tiles
     uint32_t incl = excess;
     for (int o = 1; o < 64; o <<= 1) {

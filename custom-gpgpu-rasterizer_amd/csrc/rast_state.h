@@ -178,8 +178,10 @@ struct rast_renderer {
     uint32_t last_spill = 0;               // previous-frame capacities: entries of every tile's spill region
     uint32_t last_queue = 0;               // queue storage in front of the spill regions
     uint32_t last_stride = 0;              // exact binning into fixed regions of this many entries (0: two passes)
-    bool two_pass = false;                 // the scene overflowed its fixed regions: exact frames take two passes
-    bool no_spill = false;                 // the scene overflowed its spill regions: placed by two passes
+    // frames that still take two passes because one left much beyond its fixed
+    // regions, or beyond its spill regions (note_overflow)
+    uint32_t two_pass = 0, no_spill = 0;
+    uint32_t last_trial = 0;               // the last frame took two passes: the region it would have had (0: none)
     bool last_shared_attr = false;  // the last frame's attributes were split (views rendered together)
     bool prev_valid_before = false;
     bool frame_had_prev = false;  // the last frame had a previous frame (features valid)

@@ -50,7 +50,9 @@ class Runtime:
         self.lib = lib
         for name, res, args in (("stub_limit", None, [C.c_size_t]), ("stub_used", C.c_size_t, []),
                                 ("stub_pinned", C.c_size_t, []), ("stub_mallocs", C.c_size_t, []),
-                                ("stub_pinned_of", C.c_void_p, [C.c_size_t, C.c_size_t])):
+                                ("stub_pinned_of", C.c_void_p, [C.c_size_t, C.c_size_t]),
+                                ("layout_counters_size", C.c_size_t, []),
+                                ("layout_counter", C.c_size_t, [C.c_char_p])):
             getattr(lib, name).restype, getattr(lib, name).argtypes = res, args
         self.launches = []
         self.on_launch = None
@@ -82,3 +84,9 @@ class Runtime:
 
     def mallocs(self):
         return self.lib.stub_mallocs()
+
+    def counters(self, k=0, **values):
+        """Sets words of the counters that the k-th renderer's last frame left."""
+        p = self.lib.stub_pinned_of(self.lib.layout_counters_size(), k)
+        for name, v in values.items():
+            C.c_uint32.from_address(p + self.lib.layout_counter(name.encode())).value = v

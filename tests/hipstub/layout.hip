@@ -2,20 +2,21 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <cstdint>
+#include <cstring>
 
 #include "rast_launch.h"
 
 extern "C" size_t layout_counters_size() { return sizeof(rast::FrameCounters); }
 
-extern "C" size_t layout_counter(int k)
+// The byte offset of a frame counter (SIZE_MAX: there is none of that name).
+extern "C" size_t layout_counter(const char *name)
 {
     using F = rast::FrameCounters;
-    switch (k) {
-    case 0: return offsetof(F, total_pairs);
-    case 1: return offsetof(F, ovf_entries);
-    case 2: return offsetof(F, pool_used);
-    case 3: return offsetof(F, storage_overflow);
-    case 4: return offsetof(F, spilled);
-    default: return sizeof(F);
-    }
+#define FIELD(f) \
+    if (!strcmp(name, #f)) return offsetof(F, f);
+    FIELD(num_big) FIELD(total_pairs) FIELD(overflow_tiles) FIELD(ovf_entries) FIELD(pool_used) FIELD(storage_overflow)
+    FIELD(capacity_wanted) FIELD(spilled) FIELD(past_fixed) FIELD(past_spill)
+#undef FIELD
+    return SIZE_MAX;
 }
