@@ -179,6 +179,50 @@ int rast_settle(rast_renderer *r)
     return RAST_OK;
 }
 
+// Geometry that only frames already drawn hold (its mesh is destroyed), and the
+// lock under which it is read for their debug buffers or given back.
+static std::mutex g_retained_mutex;
+static std::vector<std::weak_ptr<MeshMemory>> g_retained;
+
+bool MeshMemory::release()
+{
+    const bool any = ivert14 || idx;
+    if (ivert14) (void)hipFree(ivert14);
+    if (idx) (void)hipFree(idx);
+    ivert14 = nullptr;
+    idx = nullptr;
+    boxes = nullptr;
+    reach = nullptr;
+    return any;
+}
+
+// A destroyed mesh's geometry: freed now if no frame holds it.
+static void retain(std::shared_ptr<MeshMemory> mem)
+{
+    std::lock_guard<std::mutex> lock(g_retained_mutex);
+    g_retained.erase(std::remove_if(g_retained.begin(), g_retained.end(), [](const auto &w) { return w.expired(); }),
+                     g_retained.end());
+    try {
+        g_retained.emplace_back(mem);
+    } catch (const std::bad_alloc &) {
+        (void)mem->release();  // without a note of it, it would stay
+    }
+}
+
+hipError_t rast_dev_malloc(void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    std::lock_guard<std::mutex> lock(g_retained_mutex);
+    bool any = false;
+    for (const auto &w : g_retained)
+        if (auto mem = w.lock()) any |= mem->release();
+    g_retained.clear();
+    if (!any) return e;
+    (void)hipGetLastError();
+    return hipMalloc(p, bytes);
+}
+
 static hipError_t grow(rast_renderer *r, DBuf &b, size_t bytes, bool *synced)
 {
     if (b.p && b.n >= bytes) return hipSuccess;
@@ -189,7 +233,7 @@ static hipError_t grow(rast_renderer *r, DBuf &b, size_t bytes, bool *synced)
     }
     dfree(b);
     size_t nb = bytes < 256 ? 256 : bytes;
-    hipError_t e = hipMalloc(&b.p, nb);
+    hipError_t e = rast_dev_malloc(&b.p, nb);
     if (e != hipSuccess) { b.p = nullptr; return e; }
     b.n = nb;
     return hipSuccess;
@@ -296,23 +340,11 @@ extern "C" int rast_renderer_create_view(rast_renderer *owner, uint32_t width, u
     return new_renderer(owner->device, width, height, owner, out);
 }
 
-static void free_mesh(rast_mesh *m)
-{
-    if (m->ivert14) (void)hipFree(m->ivert14);
-    if (m->idx) (void)hipFree(m->idx);
-    delete m;
-}
-
-// Frees a mesh's device memory and detaches it from its renderer; the handle
-// stays allocated until rast_mesh_destroy.
+// Detaches a mesh from its renderer, whose frames are gone, and with it its
+// device memory; the handle stays allocated until rast_mesh_destroy.
 static void orphan_mesh(rast_mesh *m)
 {
-    if (m->ivert14) (void)hipFree(m->ivert14);
-    if (m->idx) (void)hipFree(m->idx);
-    m->ivert14 = nullptr;
-    m->idx = nullptr;
-    m->boxes = nullptr;
-    m->reach = nullptr;
+    m->mem.reset();
     for (auto &t : m->tex) t = nullptr;
     m->texq = nullptr;
     m->r = nullptr;
@@ -450,7 +482,18 @@ extern "C" int rast_mesh_create(rast_renderer *r, const rast_ivertex *verts, uin
         }
     }
     rast_mesh *m = new (std::nothrow) rast_mesh();
-    if (!m) return rast_set_error(RAST_E_OUT_OF_MEMORY, "host allocation failed");
+    MeshMemory *mem = m ? new (std::nothrow) MeshMemory() : nullptr;
+    if (mem) {
+        try {
+            m->mem.reset(mem);
+        } catch (const std::bad_alloc &) {  // (mem is deleted)
+            mem = nullptr;
+        }
+    }
+    if (!mem) {
+        delete m;
+        return rast_set_error(RAST_E_OUT_OF_MEMORY, "host allocation failed");
+    }
     m->r = r;
     m->nv = num_verts;
     m->ni = num_indices;
@@ -458,21 +501,21 @@ extern "C" int rast_mesh_create(rast_renderer *r, const rast_ivertex *verts, uin
     m->topology = topology;
     m->attr_max = attr_max;
     for (int i = 0; i < 16; ++i) m->world[i] = world ? world[i] : ((i % 5 == 0) ? 1.f : 0.f);
-    hipError_t e = hipMalloc((void **)&m->ivert14, v14.size() * sizeof(float));
+    hipError_t e = rast_dev_malloc((void **)&mem->ivert14, v14.size() * sizeof(float));
     const size_t idx_bytes = ((size_t)num_indices * 4 + 15) & ~(size_t)15;
     const size_t box_bytes = (size_t)ceil_div(ntri, 256) * 32, reach_bytes = (size_t)ceil_div(num_verts, kVertexChunk) * 32;
-    if (e == hipSuccess) e = hipMalloc((void **)&m->idx, idx_bytes + box_bytes + reach_bytes);
-    if (e == hipSuccess) e = hipMemcpy(m->ivert14, v14.data(), v14.size() * sizeof(float), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(m->idx, indices, (size_t)num_indices * 4, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = rast_dev_malloc((void **)&mem->idx, idx_bytes + box_bytes + reach_bytes);
+    if (e == hipSuccess) e = hipMemcpy(mem->ivert14, v14.data(), v14.size() * sizeof(float), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(mem->idx, indices, (size_t)num_indices * 4, hipMemcpyHostToDevice);
     if (e == hipSuccess) {  // on the copies' stream; done before any frame's stream can read them
-        m->boxes = reinterpret_cast<float4 *>(reinterpret_cast<char *>(m->idx) + idx_bytes);
-        m->reach = reinterpret_cast<uint4 *>(reinterpret_cast<char *>(m->boxes) + box_bytes);
-        e = launch_mesh_boxes(m->ivert14, m->idx, ntri, topology, m->boxes, m->reach, ceil_div(num_verts, kVertexChunk),
-                              nullptr);
+        mem->boxes = reinterpret_cast<float4 *>(reinterpret_cast<char *>(mem->idx) + idx_bytes);
+        mem->reach = reinterpret_cast<uint4 *>(reinterpret_cast<char *>(mem->boxes) + box_bytes);
+        e = launch_mesh_boxes(mem->ivert14, mem->idx, ntri, topology, mem->boxes, mem->reach,
+                              ceil_div(num_verts, kVertexChunk), nullptr);
     }
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) {
-        free_mesh(m);
+        delete m;
         return rast_set_error(e == hipErrorOutOfMemory ? RAST_E_OUT_OF_MEMORY : RAST_E_HIP, "mesh upload: %s",
                     hipGetErrorString(e));
     }
@@ -482,8 +525,6 @@ extern "C" int rast_mesh_create(rast_renderer *r, const rast_ivertex *verts, uin
     *out = m;
     return RAST_OK;
 }
-
-static int complete_debug(rast_renderer *r);
 
 extern "C" int rast_mesh_destroy(rast_mesh *m)
 {
@@ -498,16 +539,13 @@ extern "C" int rast_mesh_destroy(rast_mesh *m)
     for (rast_renderer *v : r->views) {
         HIP_TRY(renderer_wait(v));
         v->have_prev = false;
+        v->next_scene.reset();
     }
-    // the last frames' debug buffers are completed while the mesh is there (as
-    // far as there is memory for it)
-    (void)complete_debug(r);
-    for (rast_renderer *v : r->views) (void)complete_debug(v);
-    r->frame_scene.reset();
-    for (rast_renderer *v : r->views) v->frame_scene.reset();
+    r->next_scene.reset();
     r->drawn.reset();
     r->meshes.erase(std::remove(r->meshes.begin(), r->meshes.end(), m), r->meshes.end());
-    free_mesh(m);
+    retain(std::move(m->mem));
+    delete m;
     ++r->scene_version;
     r->have_prev = false;
     r->frame_valid = false;
@@ -574,7 +612,7 @@ extern "C" int rast_texture_create_pitched(rast_renderer *r, const void *rgba8, 
     t->h = h;
     const size_t row = (size_t)w * 4;
     // stored packed (pitch = width): the sampler addresses texel x + y * w
-    hipError_t e = hipMalloc((void **)&t->texels, row * h);
+    hipError_t e = rast_dev_malloc((void **)&t->texels, row * h);
     if (e == hipSuccess) e = hipMemcpy2D(t->texels, row, rgba8, pitch_bytes, row, h, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         if (t->texels) (void)hipFree(t->texels);
@@ -779,7 +817,7 @@ static int ensure_tex_quads(rast_renderer *r)
         if (!found) {
             TexQuad q = { { t[0], t[1], t[2], t[3] }, nullptr };
             const size_t n = (size_t)w * h;
-            const hipError_t me = hipMalloc((void **)&q.texels, n * sizeof(uint4));
+            const hipError_t me = rast_dev_malloc((void **)&q.texels, n * sizeof(uint4));
             if (me == hipErrorOutOfMemory) {
                 // the copy is an optimisation only: without room for it the
                 // frame samples the four separate maps
@@ -813,11 +851,9 @@ static int note_scene(rast_renderer *r)
     std::lock_guard<std::mutex> lock(g_drawn_mutex);
     if (!o->drawn || o->drawn_scene != o->scene_version || o->drawn_world != o->world_version) {
         try {
-            auto v = std::make_shared<std::vector<FrameMesh>>(o->meshes.size());
-            for (size_t i = 0; i < v->size(); ++i) {
-                (*v)[i].m = o->meshes[i];
-                memcpy((*v)[i].world, o->meshes[i]->world, sizeof (*v)[i].world);
-            }
+            auto v = std::make_shared<std::vector<MeshShape>>();
+            v->reserve(o->meshes.size());
+            for (const rast_mesh *m : o->meshes) v->push_back(*m);
             o->drawn = std::move(v);
         } catch (const std::bad_alloc &) {
             return rast_set_error(RAST_E_OUT_OF_MEMORY, "host allocation failed");
@@ -826,6 +862,12 @@ static int note_scene(rast_renderer *r)
         o->drawn_world = o->world_version;
     }
     r->next_scene = o->drawn;
+    // the last frame's scene goes before the next frame is queued: the geometry
+    // of destroyed meshes is freed with it, which waits for the device
+    if (r->frame_scene && r->frame_scene_version != o->scene_version) {
+        r->frame_scene.reset();
+        r->debug_lost = true;
+    }
     return RAST_OK;
 }
 
@@ -943,7 +985,7 @@ static int dev_alloc(DBuf &b, size_t bytes)
 {
     if (b.p && b.n >= bytes) return RAST_OK;
     dfree(b);
-    HIP_TRY(hipMalloc(&b.p, bytes < 256 ? 256 : bytes));
+    HIP_TRY(rast_dev_malloc(&b.p, bytes < 256 ? 256 : bytes));
     b.n = bytes < 256 ? 256 : bytes;
     return RAST_OK;
 }
@@ -1179,29 +1221,29 @@ static int build_plan(LaunchPlan &P, rast_renderer *const *rs, uint32_t n, int h
 }
 
 // A mesh's entry: its geometry and matrices (not its textures).
-static void fill_mesh(DevMesh &d, const rast_mesh *m, const float *world, const rast_frame_consts &fc, uint32_t vert_base,
-                      uint32_t tri_base, uint32_t vs_block0, uint32_t tri_block0)
+static void fill_mesh(DevMesh &d, const MeshShape &m, const rast_frame_consts &fc, uint32_t vert_base, uint32_t tri_base,
+                      uint32_t vs_block0, uint32_t tri_block0)
 {
+    const float *world = m.world;
     memset(&d, 0, sizeof d);
-    d.ivert = m->ivert14;
-    d.boxes = m->boxes;
-    d.reach = m->reach;
-    d.idx = m->idx;
-    d.num_verts = m->nv;
-    d.num_tris = m->ntri;
+    d.ivert = m.mem->ivert14;
+    d.boxes = m.mem->boxes;
+    d.reach = m.mem->reach;
+    d.idx = m.mem->idx;
+    d.num_verts = m.nv;
+    d.num_tris = m.ntri;
     d.vert_base = vert_base;
     d.tri_base = tri_base;
     d.vs_block0 = vs_block0;
     d.tri_block0 = tri_block0;
-    d.topology = m->topology;
-    d.has_diffuse = m->tex[0] != nullptr;
+    d.topology = m.topology;
     // the rotated normal / tangent stays below attr_max times the
     // largest row sum of the world matrix's 3x3 part
     float rowsum = 0.f;
     for (int row = 0; row < 3; ++row)
         rowsum = std::max(rowsum, std::fabs(M4c(world, row, 0)) + std::fabs(M4c(world, row, 1)) +
                                       std::fabs(M4c(world, row, 2)));
-    d.shade_exact = !(m->attr_max * rowsum <= 4.f);
+    d.shade_exact = !(m.attr_max * rowsum <= 4.f);
     mat4_mul(fc.viewproj, world, d.wvp);  // CCR/CUDARenderer.cu:241
     memcpy(d.world, world, sizeof d.world);
     for (int q = 0; q < 3; ++q) {
@@ -1310,8 +1352,9 @@ static int stage_launch(LaunchPlan &P, rast_renderer *const *rs, uint32_t n)
         for (size_t i = 0; i < meshes.size(); ++i, ++me) {
             const rast_mesh *m = meshes[i];
             DevMesh &d = dm[me];
-            fill_mesh(d, m, m->world, fc, vb, (uint32_t)m->tri_base, P.vs_block0[me], P.tri_block0[me]);
+            fill_mesh(d, *m, fc, vb, (uint32_t)m->tri_base, P.vs_block0[me], P.tri_block0[me]);
             d.job = j;
+            d.has_diffuse = m->tex[0] != nullptr;
             for (int q = 0; q < 4; ++q) {
                 if (m->tex[q]) d.tex[q] = { m->tex[q]->texels, m->tex[q]->w, m->tex[q]->h };
                 else d.tex[q] = { dflt + q, 1u, 1u };
@@ -1424,16 +1467,25 @@ static void finish_enqueue(rast_renderer *r)
     r->have_prev = true;
     r->cur ^= 1;
     r->frame_scene = std::move(r->next_scene);
+    r->frame_scene_version = scene_owner(r)->drawn_scene;
+    r->debug_lost = false;
     r->frame_cam = r->last_cam;
     r->frame_w = r->W;
     r->frame_h = r->H;
     r->frame_cull = r->last_opts.cull_mode;
 }
 
+static int debug_gone(rast_renderer *r)
+{
+    r->frame_scene.reset();
+    r->debug_lost = true;
+    return rast_set_error(RAST_E_STATE, "rast_debug_read: the last frame's scene is gone");
+}
+
 // Completes the last frame's debug buffers: positions and attributes of the
 // vertices out of view, survivor flags, the records of the survivors that
 // nothing of the frame reads (launch_debug_fill).  r's GPU work is done.
-static int complete_debug_of(rast_renderer *r, const std::vector<FrameMesh> &ms)
+static int complete_debug_of(rast_renderer *r, const std::vector<MeshShape> &ms)
 {
     // one job, a vertex group per mesh: [job][meshes][vertex block -> group]
     // [triangle blocks][groups][entries][work counters]
@@ -1445,23 +1497,24 @@ static int complete_debug_of(rast_renderer *r, const std::vector<FrameMesh> &ms)
     memset(&J, 0, sizeof J);
     uint32_t vb = 0, tb = 0;
     for (uint32_t i = 0; i < ms.size(); ++i) {
-        const rast_mesh *m = ms[i].m;
-        fill_mesh(rows[i], m, ms[i].world, fc, vb, tb, (uint32_t)vs_group.size(), (uint32_t)live.size() / 2);
-        vs_group.insert(vs_group.end(), ceil_div(m->nv, kVertexChunk), i);
-        for (uint32_t b = 0; b < ceil_div(m->ntri, 256); ++b) {
+        const MeshShape &m = ms[i];
+        if (!m.mem->ivert14) return debug_gone(r);
+        fill_mesh(rows[i], m, fc, vb, tb, (uint32_t)vs_group.size(), (uint32_t)live.size() / 2);
+        vs_group.insert(vs_group.end(), ceil_div(m.nv, kVertexChunk), i);
+        for (uint32_t b = 0; b < ceil_div(m.ntri, 256); ++b) {
             live.push_back((uint32_t)live.size() / 2);
             live.push_back(r->frame_mesh0 + i);
         }
         groups.push_back(i);
         groups.push_back(1u);
         entries.push_back(r->frame_mesh0 + i);
-        vb += m->nv;
-        tb += m->ntri;
+        vb += m.nv;
+        tb += m.ntri;
     }
     // (a later frame that failed may have lost them)
     if (r->pos4.n < (size_t)vb * 16 || r->attr.n < (size_t)vb * 48 || r->trirec.n < (size_t)tb * kTriRecWords * 4 ||
         r->alive.n < tb)
-        return RAST_OK;
+        return debug_gone(r);
     J.fp.width = r->frame_w;
     J.fp.height = r->frame_h;
     J.fp.cull_mode = r->frame_cull;
@@ -1510,9 +1563,12 @@ static int complete_debug_of(rast_renderer *r, const std::vector<FrameMesh> &ms)
 
 static int complete_debug(rast_renderer *r)
 {
+    if (r->debug_lost) return debug_gone(r);
     if (!r->frame_scene) return RAST_OK;
     try {
-        RAST_TRY(complete_debug_of(r, *r->frame_scene));
+        std::lock_guard<std::mutex> lock(g_retained_mutex);  // no geometry is given back meanwhile
+        const auto scene = r->frame_scene;
+        RAST_TRY(complete_debug_of(r, *scene));
     } catch (const std::bad_alloc &) {
         return rast_set_error(RAST_E_OUT_OF_MEMORY, "host allocation failed");
     }
@@ -1664,7 +1720,7 @@ static bool read_slots(rast_renderer *r, size_t bytes)
     hipError_t e = hipHostMalloc((void **)&r->h_read, kReadSlots * slot + flags, hipHostMallocCoherent);
     if (e != hipSuccess) r->h_read = nullptr;
     if (e == hipSuccess && !r->read_count.p) {
-        e = hipMalloc(&r->read_count.p, flags);
+        e = rast_dev_malloc(&r->read_count.p, flags);
         if (e != hipSuccess) r->read_count.p = nullptr;
         if (e == hipSuccess) e = hipMemset(r->read_count.p, 0, flags);  // from here on the kernel resets them
     }

@@ -381,7 +381,7 @@ int ensure(DBuf &b, size_t bytes)
 {
     if (b.p && b.n >= bytes) return RAST_OK;
     dfree(b);
-    HIP_TRY(hipMalloc(&b.p, bytes < 256 ? 256 : bytes));
+    HIP_TRY(rast_dev_malloc(&b.p, bytes < 256 ? 256 : bytes));
     b.n = bytes < 256 ? 256 : bytes;
     return RAST_OK;
 }
@@ -649,9 +649,9 @@ extern "C" int rast_binmodel_record(rast_binmodel *m, rast_renderer *r)
     if (m->n + nt > m->cap) {
         const uint32_t ncap = std::max<uint32_t>(m->cap * 2, m->n + nt);
         DBuf nx, ny;
-        if (hipMalloc(&nx.p, (size_t)ncap * F * 4) != hipSuccess) return rast_set_error(RAST_E_OUT_OF_MEMORY, "training set");
+        if (rast_dev_malloc(&nx.p, (size_t)ncap * F * 4) != hipSuccess) return rast_set_error(RAST_E_OUT_OF_MEMORY, "training set");
         nx.n = (size_t)ncap * F * 4;
-        if (hipMalloc(&ny.p, (size_t)ncap * 4) != hipSuccess) {
+        if (rast_dev_malloc(&ny.p, (size_t)ncap * 4) != hipSuccess) {
             dfree(nx);
             return rast_set_error(RAST_E_OUT_OF_MEMORY, "training set");
         }

@@ -96,27 +96,41 @@ struct TexQuad {
     uint4 *texels;
 };
 
-struct rast_mesh {
-    rast_renderer *r = nullptr;
+// A mesh's geometry on the device.  The mesh and the frames that drew it share it:
+// after rast_mesh_destroy it stays, for the frames' debug buffers, until each
+// renderer's next frame, or until an allocation needs the room (null pointers
+// from then on).
+struct MeshMemory {
     float *ivert14 = nullptr;  // 14 floats per vertex (the 56-byte IVertex as given) + 16 bytes of padding
     uint32_t *idx = nullptr;   // the indices, then (16-byte aligned) the boxes and reaches
     float4 *boxes = nullptr;   // object-space box (lo, hi) of every 256 triangles
     uint4 *reach = nullptr;    // behind them: the boxes the triangles of every kVertexChunk vertices lie in
-    uint32_t nv = 0, ni = 0, ntri = 0;
+    MeshMemory() = default;
+    MeshMemory(const MeshMemory &) = delete;
+    MeshMemory &operator=(const MeshMemory &) = delete;
+    ~MeshMemory() { release(); }
+    bool release();  // whether there was any
+};
+
+// What a frame's geometry stages read of a mesh.
+struct MeshShape {
+    std::shared_ptr<MeshMemory> mem;
+    uint32_t nv = 0, ntri = 0;
     int topology = 0;
+    float attr_max = 0.f;  // largest |component| of the input normals and tangents
     float world[16];
+};
+
+struct rast_mesh : MeshShape {
+    rast_renderer *r = nullptr;
+    uint32_t ni = 0;
     rast_texture *tex[4] = { nullptr, nullptr, nullptr, nullptr };
     const uint4 *texq = nullptr;  // interleaved maps for tex[0..3], set by prepare_job
-    float attr_max = 0.f;         // largest |component| of the input normals and tangents
     uint64_t tri_base = 0;
 };
 
-// The meshes of a frame and their world matrices, for data of the frame that is
-// formed only when it is asked for.
-struct FrameMesh {
-    const rast_mesh *m;
-    float world[16];
-};
+// hipMalloc that gives back retained geometry (MeshMemory) before it fails.
+hipError_t rast_dev_malloc(void **p, size_t bytes);
 
 struct rast_renderer {
     int device = 0;
@@ -133,7 +147,7 @@ struct rast_renderer {
     uint64_t layout_version = 0;           // scene version the block tables were built for
     uint64_t world_version = 1;            // bumped when a mesh's world matrix changes
     // the scene as of these versions, shared by the frames that drew it
-    std::shared_ptr<const std::vector<FrameMesh>> drawn;
+    std::shared_ptr<const std::vector<MeshShape>> drawn;
     uint64_t drawn_scene = 0, drawn_world = 0;
     hipEvent_t join = nullptr;             // orders a batch after this renderer's earlier work
     uint64_t batch_seq = 0;                // batch that rendered the last frame (0: none pending)
@@ -170,7 +184,10 @@ struct rast_renderer {
     bool frame_pending = false;
     bool frame_valid = false;
     // what the last frame was drawn from, until its debug buffers are whole
-    std::shared_ptr<const std::vector<FrameMesh>> frame_scene, next_scene;
+    // (debug_lost: it is gone before they were)
+    std::shared_ptr<const std::vector<MeshShape>> frame_scene, next_scene;
+    uint64_t frame_scene_version = 0;
+    bool debug_lost = false;
     rast_camera frame_cam{};
     uint32_t frame_w = 0, frame_h = 0, frame_mesh0 = 0;
     int32_t frame_cull = 0;

@@ -20,6 +20,7 @@
 
 #include <hip/hip_runtime_api.h>
 
+#ifndef STUB_PLAIN_DELETE  // (with a sanitizer, which does this better)
 void *operator new(size_t n)
 {
     if (void *p = malloc(n ? n : 1)) return p;
@@ -34,6 +35,7 @@ void operator delete(void *p) noexcept
             static_cast<volatile uint64_t *>(p)[i] = 0xA5A5A5A5A5A50000ull + 64 * i;
 }
 void operator delete(void *p, size_t) noexcept { operator delete(p); }
+#endif
 
 namespace {
 
