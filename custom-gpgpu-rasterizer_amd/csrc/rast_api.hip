@@ -213,14 +213,15 @@ hipError_t rast_dev_malloc(void **p, size_t bytes)
 {
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
     std::lock_guard<std::mutex> lock(g_retained_mutex);
     bool any = false;
     for (const auto &w : g_retained)
         if (auto mem = w.lock()) any |= mem->release();
     g_retained.clear();
-    if (!any) return e;
-    (void)hipGetLastError();
-    return hipMalloc(p, bytes);
+    if (any) e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
 }
 
 static hipError_t grow(rast_renderer *r, DBuf &b, size_t bytes, bool *synced)
@@ -317,6 +318,7 @@ static int new_renderer(int device, uint32_t width, uint32_t height, rast_render
     if (rc == RAST_OK) rc = alloc_framebuffers(r);
     if (rc != RAST_OK) {
         rast_renderer_destroy(r);
+        (void)hipGetLastError();
         return rast_set_error(rc, "rast_renderer_create: HIP resource allocation failed");
     }
     memset(r->h_counters, 0, sizeof(FrameCounters));
@@ -516,6 +518,7 @@ extern "C" int rast_mesh_create(rast_renderer *r, const rast_ivertex *verts, uin
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) {
         delete m;
+        (void)hipGetLastError();
         return rast_set_error(e == hipErrorOutOfMemory ? RAST_E_OUT_OF_MEMORY : RAST_E_HIP, "mesh upload: %s",
                     hipGetErrorString(e));
     }
@@ -617,6 +620,7 @@ extern "C" int rast_texture_create_pitched(rast_renderer *r, const void *rgba8, 
     if (e != hipSuccess) {
         if (t->texels) (void)hipFree(t->texels);
         delete t;
+        (void)hipGetLastError();
         return rast_set_error(e == hipErrorOutOfMemory ? RAST_E_OUT_OF_MEMORY : RAST_E_HIP, "texture upload: %s",
                     hipGetErrorString(e));
     }
@@ -831,6 +835,7 @@ static int ensure_tex_quads(rast_renderer *r)
             if (e == hipSuccess) e = hipStreamSynchronize(r->stream);
             if (e != hipSuccess) {
                 (void)hipFree(q.texels);
+                (void)hipGetLastError();
                 return rast_set_error(RAST_E_HIP, "interleaving the maps: %s", hipGetErrorString(e));
             }
             owner->tex_quads.push_back(q);
@@ -1813,7 +1818,10 @@ static float elapsed(rast_renderer *r, int a, int b)
 {
     if (!r->ev_used[a] || !r->ev_used[b]) return 0.f;
     float ms = 0.f;
-    if (hipEventElapsedTime(&ms, r->ev[a], r->ev[b]) != hipSuccess) return 0.f;
+    if (hipEventElapsedTime(&ms, r->ev[a], r->ev[b]) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0.f;
+    }
     return ms;
 }
 

@@ -567,6 +567,7 @@ extern "C" int rast_binmodel_create(rast_renderer *r, uint32_t hidden, uint32_t 
     if (rc == RAST_OK && hipMemset(m->adam_m.p, 0, np * 4) != hipSuccess) rc = RAST_E_HIP;
     if (rc == RAST_OK && hipMemset(m->adam_v.p, 0, np * 4) != hipSuccess) rc = RAST_E_HIP;
     if (rc != RAST_OK) {
+        (void)hipGetLastError();
         rast_binmodel_destroy(m);
         return rast_set_error(rc, "rast_binmodel_create: allocation failed");
     }

@@ -15,12 +15,16 @@
 // returns `code`.
 int rast_set_error(int code, const char *fmt, ...);
 
+// (the runtime's own last error is taken too: left there, the next kernel launch,
+// which asks for it, would report it as its own)
 #define HIP_TRY(expr)                                                                                      \
     do {                                                                                                   \
         hipError_t e_ = (expr);                                                                            \
-        if (e_ != hipSuccess)                                                                              \
+        if (e_ != hipSuccess) {                                                                            \
+            (void)hipGetLastError();                                                                       \
             return rast_set_error(e_ == hipErrorOutOfMemory ? RAST_E_OUT_OF_MEMORY : RAST_E_HIP,           \
                                   "%s: %s (%s:%d)", #expr, hipGetErrorString(e_), __FILE__, __LINE__);     \
+        }                                                                                                  \
     } while (0)
 
 #define RAST_TRY(expr)                  \
