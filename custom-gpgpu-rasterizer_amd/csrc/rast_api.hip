@@ -279,17 +279,32 @@ enum { EV_START, EV_VERTEX, EV_MODEL, EV_SETUP, EV_SCANCNT, EV_FILL, EV_FALLBACK
 enum { EV_TIMER_START = EV_COUNT, EV_TIMER_STOP, EV_ALL };
 static_assert(EV_ALL <= (int)(sizeof(((rast_renderer *)nullptr)->ev) / sizeof(hipEvent_t)), "renderer event slots");
 
+static bool have_framebuffers(const rast_renderer *r)
+{
+    const size_t P = (size_t)r->W * r->H;
+    return r->vis.n >= P * 4 && r->depth.n >= P * 4 && r->rgba.n >= P * 4 && r->keys.n >= P * 8;
+}
+
 static int alloc_framebuffers(rast_renderer *r)
 {
     bool synced = false;
     const size_t P = (size_t)r->W * r->H;
-    HIP_TRY(grow(r, r->vis, P * 4, &synced));
-    HIP_TRY(grow(r, r->depth, P * 4, &synced));
-    HIP_TRY(grow(r, r->rgba, P * 4, &synced));
-    HIP_TRY(grow(r, r->keys, P * 8, &synced));
+    hipError_t e = grow(r, r->vis, P * 4, &synced);
+    if (e == hipSuccess) e = grow(r, r->depth, P * 4, &synced);
+    if (e == hipSuccess) e = grow(r, r->rgba, P * 4, &synced);
+    if (e == hipSuccess) e = grow(r, r->keys, P * 8, &synced);
     r->keys_dirty = true;
     r->frame_valid = false;
+    if (e != hipSuccess) r->frame_pending = false;  // the last frame's buffers are not all there any more
+    HIP_TRY(e);
     return RAST_OK;
+}
+
+// Frames and copies of frames need the buffers, which a resize without memory
+// for them leaves missing: tried again then.
+static int need_framebuffers(rast_renderer *r)
+{
+    return have_framebuffers(r) ? RAST_OK : alloc_framebuffers(r);
 }
 
 static int new_renderer(int device, uint32_t width, uint32_t height, rast_renderer *scene_src, rast_renderer **out)
@@ -880,6 +895,7 @@ static int prepare_job(rast_renderer *r)
 {
     HIP_TRY(hipSetDevice(r->device));
     if (scene_meshes(r).empty()) return rast_set_error(RAST_E_STATE, "rast_render: no meshes loaded");
+    RAST_TRY(need_framebuffers(r));
     RAST_TRY(note_scene(r));
     note_overflow(r);
     if (r->layout_version != scene_owner(r)->scene_version) refresh_layout(r);
@@ -1952,6 +1968,7 @@ extern "C" int rast_draw_texture(rast_renderer *r, const rast_texture *t, int mo
         return rast_set_error(RAST_E_INVALID_ARG, "rast_draw_texture: sample_state %d", sample_state);
     HIP_TRY(hipSetDevice(r->device));
     if (r->frame_pending) RAST_TRY(check_frame(r));
+    RAST_TRY(need_framebuffers(r));
     HIP_TRY(renderer_wait(r));  // earlier frames (also from batches) are done with the buffers
     HIP_TRY(launch_draw_texture((uint32_t *)r->vis.p, (float *)r->depth.p, (uint32_t *)r->rgba.p, r->W, r->H,
                                 t->texels, t->w, t->h, mode, stretch != 0, sample_state, r->stream));

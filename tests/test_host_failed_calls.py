@@ -55,3 +55,26 @@ def test_frames_after_a_refused_debug_read(renderer):
     with pytest.raises(R.RastError):  # more tiles than the last frame had
         renderer.debug_read(R.DEBUG_TILE_COUNTS)
     frames(renderer)
+
+
+@pytest.mark.parametrize("room", [0, 80 << 20, 150 << 20, 210 << 20])  # none, or vis, depth, colours
+@pytest.mark.parametrize("read", [False, True])
+def test_a_resize_without_memory_leaves_no_frame(host, renderer, room, read):
+    """Its buffers may be gone: nothing draws into them or copies from them."""
+    r = renderer
+    if read:
+        r.readback()
+    host.limit(room)
+    with pytest.raises(R.RastError):
+        R.check(R.lib().rast_resize(r.h, 4096, 4096))
+    r.width = r.height = 4096
+    host.launches.clear()
+    for call in (r.readback, lambda: r.render(S.Camera(), S.Opts()), r.readback,
+                 lambda: r.draw_texture(np.zeros((4, 4), np.uint32)),
+                 lambda: R.render_batch([(r, S.Camera(), S.Opts(), R.BIN_EXACT, 0)]),
+                 lambda: R.check(R.lib().rast_frame_buffers(r.h, None, None, None))):
+        with pytest.raises(R.RastError):
+            call()
+    assert host.names() == []
+    host.limit(None)
+    frames(r)
