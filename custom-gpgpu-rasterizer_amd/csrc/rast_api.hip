@@ -413,6 +413,7 @@ extern "C" int rast_renderer_destroy(rast_renderer *r)
 static void forget_overflow(rast_renderer *r)
 {
     r->two_pass = r->no_spill = 0;
+    r->queue_tight = false;
     __atomic_store_n(&r->h_counters->past_fixed, kNotMeasured, __ATOMIC_RELAXED);
     __atomic_store_n(&r->h_counters->past_spill, kNotMeasured, __ATOMIC_RELAXED);
 }
@@ -715,8 +716,8 @@ constexpr uint32_t kFixedRegion = 1024, kFixedRegionMin = 512;
 
 static uint32_t fixed_stride(const rast_renderer *r, uint32_t ntiles)
 {
-    const uint32_t s = r->queue_cap / ntiles;
-    return s < kFixedRegionMin ? 0u : std::min(s, std::max<uint32_t>(r->total_tris, 1u));
+    const uint32_t s = r->queue_cap / ntiles, tris = std::max<uint32_t>(r->total_tris, 1u);
+    return s < std::min(kFixedRegionMin, tris) ? 0u : std::min(s, tris);
 }
 
 // Previous-frame capacities: half of the queue storage gives every tile a spill
@@ -730,8 +731,27 @@ constexpr uint32_t kSpill = 512, kSpillMin = 128;
 
 static uint32_t spill_stride(const rast_renderer *r, uint32_t ntiles)
 {
-    const uint32_t s = std::min(r->queue_cap / 2 / ntiles, kSpill);
-    return s < kSpillMin ? 0u : s;
+    const uint32_t s = std::min(r->queue_cap / 2 / ntiles, kSpill), tris = std::max<uint32_t>(r->total_tris, 1u);
+    return s < std::min(kSpillMin, tris) ? 0u : std::min(s, tris);
+}
+
+// Queue storage (entries) that gives every tile a region of the length worth
+// having, 4 KB a tile in large scenes, up to 256 MB; 0 where no frame of the
+// policy has regions, where so many tiles share that limit that theirs would be
+// too short, and after it was found that there is no memory for it.
+static uint32_t queue_wish(const rast_renderer *r, uint32_t ntiles)
+{
+    constexpr uint64_t kMost = 1u << 26;
+    const int policy = r->last_opts.bin_policy;
+    if (r->queue_tight || (policy == RAST_BIN_LEARNED && r->model)) return 0u;
+    // spill regions take half of the storage
+    const bool spill = policy == RAST_BIN_PREVFRAME;
+    if (spill ? r->no_spill : r->two_pass) return 0u;
+    const uint32_t tris = std::max<uint32_t>(r->total_tris, 1u);
+    const uint64_t want = spill ? 2u * std::min(kSpill, tris) : std::min(kFixedRegion, tris);
+    const uint64_t least = spill ? 2u * std::min(kSpillMin, tris) : std::min(kFixedRegionMin, tris);
+    if (ntiles * least > kMost) return 0u;
+    return (uint32_t)std::min(ntiles * want, kMost);
 }
 
 // A frame that left more than kOverflowMax entries beyond its regions makes the
@@ -781,12 +801,17 @@ static int ensure_frame_storage(rast_renderer *r, uint32_t ntiles)
     HIP_TRY(grow(r, r->tile_cursor, tb, &synced));
     HIP_TRY(grow(r, r->tile_keys, tb, &synced));
     if (r->queue_cap == 0) r->queue_cap = std::max<uint32_t>(1u << 20, std::min<uint64_t>(4ull * nt, 0x7FFFFFFFull));
-    // room for fixed regions (fixed_stride) in frames of many tiles: 4 KB a tile, up to 256 MB
-    r->queue_cap = std::max<uint32_t>(r->queue_cap, std::min<uint64_t>((uint64_t)ntiles * kFixedRegion, 1u << 26));
     if (r->pool_cap == 0) r->pool_cap = 1u << 20;
     if (r->big_cap == 0) r->big_cap = 1u << 16;
     if (r->ovf_cap == 0) r->ovf_cap = 1u << 20;
     HIP_TRY(grow(r, r->ovf, (size_t)r->ovf_cap * 8, &synced));
+    const uint32_t wish = queue_wish(r, ntiles);
+    if (wish > r->queue_cap) {  // without room for it, the frame takes two passes
+        const hipError_t e = grow(r, r->queue, (size_t)wish * 4, &synced);
+        if (e == hipSuccess) r->queue_cap = wish;
+        else if (e == hipErrorOutOfMemory) r->queue_tight = true;
+        else HIP_TRY(e);
+    }
     HIP_TRY(grow(r, r->queue, (size_t)r->queue_cap * 4, &synced));
     HIP_TRY(grow(r, r->pool, (size_t)r->pool_cap * 4, &synced));
     HIP_TRY(grow(r, r->big, (size_t)r->big_cap * 4, &synced));

@@ -202,6 +202,7 @@ struct rast_renderer {
     // frames that still take two passes because one left much beyond its fixed
     // regions, or beyond its spill regions (note_overflow)
     uint32_t two_pass = 0, no_spill = 0;
+    bool queue_tight = false;              // no memory for longer regions (queue_wish)
     uint32_t last_trial = 0;               // the last frame took two passes: the region it would have had (0: none)
     bool last_shared_attr = false;  // the last frame's attributes were split (views rendered together)
     bool prev_valid_before = false;
