@@ -307,6 +307,9 @@ static int need_framebuffers(rast_renderer *r)
     return have_framebuffers(r) ? RAST_OK : alloc_framebuffers(r);
 }
 
+static void count_renderer(rast_renderer *r);
+static void uncount_renderer(rast_renderer *r);
+
 static int new_renderer(int device, uint32_t width, uint32_t height, rast_renderer *scene_src, rast_renderer **out)
 {
     if (!out) return rast_set_error(RAST_E_INVALID_ARG, "rast_renderer_create: null output");
@@ -337,6 +340,7 @@ static int new_renderer(int device, uint32_t width, uint32_t height, rast_render
         return rast_set_error(rc, "rast_renderer_create: HIP resource allocation failed");
     }
     memset(r->h_counters, 0, sizeof(FrameCounters));
+    count_renderer(r);
     if (scene_src) {
         r->scene_src = scene_src;
         scene_src->views.push_back(r);
@@ -397,14 +401,14 @@ extern "C" int rast_renderer_destroy(rast_renderer *r)
                      &r->alive, &r->survivors, &r->tile_count[0], &r->tile_count[1], &r->tile_off, &r->tile_cap,
                      &r->tile_pool, &r->tile_cursor, &r->tile_keys, &r->tile_min_depth[0], &r->tile_min_depth[1], &r->keys,
                      &r->queue, &r->pool, &r->big, &r->bigp, &r->bige, &r->ovf, &r->vis, &r->depth,
-                     &r->rgba, &r->read_count };
+                     &r->rgba };
     for (DBuf *b : bufs) dfree(*b);
     if (r->h_counters) (void)hipHostFree(r->h_counters);
-    if (r->h_read) (void)hipHostFree(r->h_read);
     for (hipEvent_t &e : r->ev)
         if (e) (void)hipEventDestroy(e);
     if (r->join) (void)hipEventDestroy(r->join);
     if (r->stream) (void)hipStreamDestroy(r->stream);
+    uncount_renderer(r);
     delete r;
     return RAST_OK;
 }
@@ -1754,30 +1758,98 @@ static bool ordinary_memory(const void *p)
     return a.type == hipMemoryTypeUnregistered;
 }
 
-// The slots of r for pieces of up to `bytes`, their flags behind them; false
-// without memory for them (the copies are hipMemcpy's then).
-static bool read_slots(rast_renderer *r, size_t bytes)
+// The slots of one readback, their flags behind them.  Made by the first readback
+// that finds none, for pieces of up to `bytes`; up to kKeptPerDevice (33 MB) are
+// kept for the next one, of any renderer of the device, until its last renderer
+// is destroyed.
+struct ReadSlots {
+    int device = -1;
+    char *h = nullptr;
+    size_t bytes = 0;
+    uint32_t *count = nullptr;
+    uint32_t epoch = 0;
+};
+constexpr int kKeptPerDevice = 2, kKept = 16, kSlotDevices = 64;  // (none are kept for further devices)
+static std::mutex g_slots_mutex;
+static ReadSlots g_kept[kKept];  // device < 0: none
+static uint32_t g_renderers[kSlotDevices];
+
+static void free_slots(ReadSlots &s)
 {
-    if (r->read_bytes >= bytes) return true;
-    if (r->h_read) (void)hipHostFree(r->h_read);
-    r->h_read = nullptr;
-    r->read_bytes = 0;
+    if (s.h) (void)hipHostFree(s.h);
+    if (s.count) (void)hipFree(s.count);
+    s = ReadSlots();
+}
+
+static void count_renderer(rast_renderer *r)
+{
+    if (r->device >= kSlotDevices) return;
+    std::lock_guard<std::mutex> lock(g_slots_mutex);
+    ++g_renderers[r->device];
+    r->counted = true;
+}
+
+static void uncount_renderer(rast_renderer *r)
+{
+    if (!r->counted) return;
+    ReadSlots gone[kKept];
+    {
+        std::lock_guard<std::mutex> lock(g_slots_mutex);
+        if (--g_renderers[r->device]) return;
+        for (int k = 0; k < kKept; ++k)
+            if (g_kept[k].device == r->device) std::swap(gone[k], g_kept[k]);
+    }
+    for (ReadSlots &s : gone) free_slots(s);
+}
+
+// False without memory for them (the copies are hipMemcpy's then).
+static bool take_slots(int device, size_t bytes, ReadSlots &s)
+{
+    {
+        std::lock_guard<std::mutex> lock(g_slots_mutex);
+        ReadSlots *best = nullptr;
+        for (ReadSlots &k : g_kept)
+            if (k.device == device && (!best || k.bytes > best->bytes)) best = &k;
+        if (best) std::swap(s, *best);
+    }
     const size_t slot = (bytes + 15) & ~(size_t)15, flags = kReadSlots * kReadChunks * 4;
-    hipError_t e = hipHostMalloc((void **)&r->h_read, kReadSlots * slot + flags, hipHostMallocCoherent);
-    if (e != hipSuccess) r->h_read = nullptr;
-    if (e == hipSuccess && !r->read_count.p) {
-        e = rast_dev_malloc(&r->read_count.p, flags);
-        if (e != hipSuccess) r->read_count.p = nullptr;
-        if (e == hipSuccess) e = hipMemset(r->read_count.p, 0, flags);  // from here on the kernel resets them
+    hipError_t e = hipSuccess;
+    if (s.bytes < slot) {
+        if (s.h) (void)hipHostFree(s.h);
+        s.h = nullptr;
+        e = hipHostMalloc((void **)&s.h, kReadSlots * slot + flags, hipHostMallocCoherent);
+        if (e != hipSuccess) s.h = nullptr;
+        else memset(s.h + kReadSlots * slot, 0, flags);
+        s.bytes = slot;
+    }
+    if (e == hipSuccess && !s.count) {
+        e = rast_dev_malloc((void **)&s.count, flags);
+        if (e != hipSuccess) s.count = nullptr;
+        else e = hipMemset(s.count, 0, flags);  // from here on the kernel resets them
     }
     if (e != hipSuccess) {
         (void)hipGetLastError();
-        dfree(r->read_count);
+        free_slots(s);
         return false;
     }
-    memset(r->h_read + kReadSlots * slot, 0, flags);
-    r->read_bytes = slot;
+    s.device = device;
     return true;
+}
+
+// After a failed copy the flags and counts may be left anyhow: not kept.
+static void give_slots(ReadSlots &s, bool ok)
+{
+    {
+        std::lock_guard<std::mutex> lock(g_slots_mutex);
+        int kept = 0;
+        ReadSlots *room = nullptr;
+        for (ReadSlots &k : g_kept) {
+            kept += k.device == s.device;
+            if (k.device < 0) room = &k;
+        }
+        if (ok && room && kept < kKeptPerDevice && s.device < kSlotDevices) std::swap(s, *room);
+    }
+    free_slots(s);
 }
 
 // Waits for a chunk's flag.  Should the kernel end without it (a failed
@@ -1800,10 +1872,10 @@ static int wait_chunk(const uint32_t *flag, uint32_t epoch)
     return RAST_OK;
 }
 
-static int copy_to_host(rast_renderer *r, const HostCopy *c, int n)
+static int copy_to_host(ReadSlots &slots, const HostCopy *c, int n)
 {
-    const size_t slot_bytes = r->read_bytes;
-    uint32_t *const flags = (uint32_t *)(r->h_read + kReadSlots * slot_bytes);
+    const size_t slot_bytes = slots.bytes;
+    uint32_t *const flags = (uint32_t *)(slots.h + kReadSlots * slot_bytes);
     HostCopy queued[kReadSlots] = {};
     uint32_t epoch[kReadSlots] = {};
     int k = 0, rc = RAST_OK;
@@ -1813,11 +1885,11 @@ static int copy_to_host(rast_renderer *r, const HostCopy *c, int n)
         if (k < n && issued - taken < (uint32_t)kReadSlots) {
             const uint32_t s = issued % kReadSlots;
             const size_t b = std::min(std::min(kReadPiece, slot_bytes), c[k].bytes - off);
-            char *const stage = r->h_read + s * slot_bytes;
+            char *const stage = slots.h + s * slot_bytes;
             queued[s] = { stage, c[k].dst + off, b };
-            epoch[s] = ++r->read_epoch;
+            epoch[s] = ++slots.epoch;
             // on the null stream, as hipMemcpy: after the caller's work on blocking streams
-            const hipError_t e = launch_read_out(c[k].src + off, stage, b, (uint32_t *)r->read_count.p + s * kReadChunks,
+            const hipError_t e = launch_read_out(c[k].src + off, stage, b, slots.count + s * kReadChunks,
                                                  flags + s * kReadChunks, epoch[s], nullptr);
             if (e != hipSuccess) rc = rast_set_error(RAST_E_HIP, "rast_readback: %s", hipGetErrorString(e));
             else ++issued;
@@ -1849,10 +1921,18 @@ extern "C" int rast_readback(rast_renderer *r, uint32_t *vis, float *depth, uint
     int n = 0;
     for (const HostCopy &c : all) {
         if (!c.dst) continue;
-        if (bytes >= kReadStaged && ordinary_memory(c.dst) && read_slots(r, std::min(bytes, kReadPiece))) staged[n++] = c;
+        if (bytes >= kReadStaged && ordinary_memory(c.dst)) staged[n++] = c;
         else HIP_TRY(hipMemcpy(c.dst, c.src, bytes, hipMemcpyDeviceToHost));
     }
-    return n ? copy_to_host(r, staged, n) : RAST_OK;
+    if (n == 0) return RAST_OK;
+    ReadSlots slots;
+    if (!take_slots(r->device, std::min(bytes, kReadPiece), slots)) {
+        for (int k = 0; k < n; ++k) HIP_TRY(hipMemcpy(staged[k].dst, staged[k].src, bytes, hipMemcpyDeviceToHost));
+        return RAST_OK;
+    }
+    const int rc = copy_to_host(slots, staged, n);
+    give_slots(slots, rc == RAST_OK);
+    return rc;
 }
 
 static float elapsed(rast_renderer *r, int a, int b)

@@ -171,12 +171,7 @@ struct rast_renderer {
     bool have_prev = false;
     rast::FrameCounters *h_counters = nullptr;  // pinned, written by the launch
     rast::FrameCounters *d_counters_host = nullptr;  // device address of h_counters
-    // pinned slots of read_bytes each that a readback passes through (made by
-    // the first that does), and the chunk flags behind them
-    char *h_read = nullptr;
-    size_t read_bytes = 0;
-    uint32_t read_epoch = 0;
-    DBuf read_count;
+    bool counted = false;  // one of its device's renderers (ReadSlots are kept while there is one)
     // timing
     hipEvent_t ev[12] = {};
     bool timing = false;

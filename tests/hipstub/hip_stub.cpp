@@ -1,7 +1,7 @@
 // A stand-in for the HIP runtime, for tests of the library's host code on a
 // machine without a GPU: memory is host memory, kernels are reported to a
-// callback (by name, with their grid) instead of run, streams and events only
-// have a lifetime.  Every handle and pointer handed in is checked against the
+// callback (by name, with their grid) instead of run (but for the readback's copy,
+// which the host waits for), streams and events only have a lifetime.  Every handle and pointer handed in is checked against the
 // live ones; a wrong one ends the process with a message.  Deleted objects are
 // overwritten and never handed out again, so that a late use shows.
 #include <cstdint>
@@ -58,6 +58,7 @@ using Graph = std::vector<Launch>;
 std::recursive_mutex g_mutex;
 std::map<char *, size_t> g_device, g_pinned;
 size_t g_used = 0, g_limit = SIZE_MAX, g_mallocs = 0;
+bool g_lose_copies = false;
 std::set<void *> g_streams, g_events, g_graphs, g_execs;
 std::map<Stream *, Stream *> g_joined;  // side stream -> the capturing one it was forked from
 // (filled by the library's static constructors, which may run before this file's)
@@ -137,6 +138,7 @@ extern "C" {
 // ------------------------------------------------------------- test control
 void stub_callback(Callback c) { g_callback = c; }
 void stub_limit(size_t bytes) { g_limit = bytes; }
+void stub_lose_copies(int lose) { g_lose_copies = lose != 0; }  // readbacks raise no flags
 size_t stub_used() { return g_used; }
 size_t stub_pinned()
 {
@@ -349,11 +351,28 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *sh, hipStream_t *
     *g = t_config.grid, *b = t_config.block, *sh = t_config.shared, *s = t_config.stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **, size_t, hipStream_t s)
+// k_read_out(src, dst, words, count, flags, epoch): the copy, and a flag per 256 KB.
+static void read_out(void **args)
+{
+    const char *src = *static_cast<const char **>(args[0]);
+    char *dst = *static_cast<char **>(args[1]);
+    const size_t bytes = 4 * (size_t)*static_cast<uint32_t *>(args[2]);
+    uint32_t *flags = *static_cast<uint32_t **>(args[4]);
+    if (room(g_device, src) < bytes) wrong("readback from", src);
+    if (room(g_pinned, dst) < bytes) wrong("readback to", dst);
+    memcpy(dst, src, bytes);
+    if (g_lose_copies) return;
+    for (size_t c = 0; c * (256u << 10) < bytes; ++c) flags[c] = *static_cast<uint32_t *>(args[5]);
+}
+hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t, hipStream_t s)
 {
     Stream *p = s ? live<Stream>(g_streams, s, "stream") : nullptr;
     const Launch l{ names().at(f), g.x, b.x };
     if (!g.x || !b.x) return ret(hipErrorInvalidConfiguration);
+    if (l.name.find("k_read_out") != std::string::npos) {
+        std::lock_guard<std::recursive_mutex> lock(g_mutex);
+        read_out(args);
+    }
     if (Stream *c = capture_of(p)) c->graph.push_back(l);
     else if (g_callback) g_callback(l.name.c_str(), l.grid, l.block);
     return hipSuccess;
