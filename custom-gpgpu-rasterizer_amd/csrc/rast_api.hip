@@ -1040,8 +1040,8 @@ static int dev_alloc(DBuf &b, size_t bytes)
     return RAST_OK;
 }
 
-// Launches of at most this many 32x32 tiles in all (two per CU) are resolved in
-// quarters.  Resolve, quarters against whole tiles: 300 tiles (a sphere in 480p)
+// The 32x32 tiles of launches of at most this many tiles in all (two per CU), of
+// any size, are resolved in quarters.  Resolve, quarters against whole tiles: 300 tiles (a sphere in 480p)
 // 8.3 and 14.0 us, 350 tiles of up to 1,191 triangles 17.8 and 25.9; 768 light
 // tiles 8.2 and 6.1; 2,040 tiles 32.2 and 32.6 (terrain), 17.0 and 14.0 (no
 // queues); 8,160 tiles 116 and 69.
@@ -1080,13 +1080,13 @@ static int build_plan(LaunchPlan &P, rast_renderer *const *rs, uint32_t n, int h
     uint64_t grid[ST_COUNT] = {};
     uint32_t mesh_entry = 0;
     std::vector<uint32_t> job_tiles(n);
-    uint64_t tiles32 = 0;
+    uint64_t tiles = 0;
     for (uint32_t j = 0; j < n; ++j) {
         job_tiles[j] = ceil_div(rs[j]->W, rs[j]->tile) * ceil_div(rs[j]->H, rs[j]->tile);
-        if (rs[j]->tile == 32) tiles32 += job_tiles[j];
+        tiles += job_tiles[j];
     }
     // (a persistent launch keeps whole tiles)
-    const bool few_tiles = tiles32 <= kQuarterTiles && rs[0]->resolve_mode == RAST_RESOLVE_PER_TILE;
+    const bool few_tiles = tiles <= kQuarterTiles && rs[0]->resolve_mode == RAST_RESOLVE_PER_TILE;
     for (uint32_t j = 0; j < n; ++j) {
         rast_renderer *r = rs[j];
         const uint32_t ntiles = job_tiles[j];
