@@ -948,6 +948,10 @@ static int prepare_job(rast_renderer *r)
 
 static bool job_learned(const rast_renderer *r) { return r->last_single && r->last_opts.bin_policy == RAST_BIN_LEARNED; }
 static bool job_shades(const rast_renderer *r) { return !(r->last_opts.flags & RAST_FLAG_NO_SHADE); }
+static bool job_far(const rast_renderer *r)
+{
+    return (r->last_opts.flags & RAST_FLAG_FAR) || far_records(r->total_verts, r->total_tris);
+}
 
 // Structure of a launch: whatever fixes its grids, block tables and kernel
 // instances (the shading kernel has one per sampling mode).
@@ -968,7 +972,7 @@ static uint64_t plan_key(rast_renderer *const *rs, uint32_t n, int hidden)
         mix((uint64_t)r->W << 32 | r->H);
         mix((uint64_t)r->last_opts.sample_state << 16 | (uint64_t)r->tile << 8 | (uint64_t)r->last_single << 4 | (uint64_t)(r->last_stride != 0) << 5 |
             (uint64_t)(r->last_spill != 0) << 6 |
-            (uint64_t)job_learned(r) << 2 | job_shades(r));
+            (uint64_t)job_far(r) << 3 | (uint64_t)job_learned(r) << 2 | job_shades(r));
         const std::vector<rast_mesh *> &ms = scene_meshes(const_cast<rast_renderer *>(r));
         mix(ms.size());
         for (const rast_mesh *m : ms) {
@@ -1236,13 +1240,9 @@ static int build_plan(LaunchPlan &P, rast_renderer *const *rs, uint32_t n, int h
     }
     // shading instances: bit (sampling mode + 2 for the shared-scene layout + 4 for far records)
     for (uint32_t j = 0; j < n; ++j)
-        if (P.nblocks[(size_t)j * ST_COUNT + ST_SHADE]) {
-            FrameParams fp{};
-            fp.num_verts = rs[j]->total_verts;
-            fp.num_tris = rs[j]->total_tris;
+        if (P.nblocks[(size_t)j * ST_COUNT + ST_SHADE])
             L.shade_modes |= 1u << (rs[j]->last_opts.sample_state + (P.sattr_off[j] != SIZE_MAX ? 2 : 0) +
-                                    (far_records(fp) ? 4 : 0));
-        }
+                                    (job_far(rs[j]) ? 4 : 0));
     // resolve form: the persistent kernels are sized to what the device holds
     L.resolve_mode = n ? rs[0]->resolve_mode : 0;
     L.fused_shade = 0;
@@ -1336,6 +1336,7 @@ static int stage_launch(LaunchPlan &P, rast_renderer *const *rs, uint32_t n)
         fp.num_tris = r->total_tris;
         fp.num_verts = r->total_verts;
         fp.num_meshes = (uint32_t)meshes.size();
+        fp.far = job_far(r);
         memcpy(J.block0, &P.block0[(size_t)j * ST_COUNT], sizeof J.block0);
         memcpy(J.nblocks, &P.nblocks[(size_t)j * ST_COUNT], sizeof J.nblocks);
         J.mesh0 = me;

@@ -88,14 +88,15 @@ struct FrameParams {
     uint32_t num_tris;        // all meshes
     uint32_t num_verts;
     uint32_t num_meshes;
+    uint32_t far;             // shaded with 64-bit record addresses
 };
 
 // Whether a frame's attribute records (48 bytes a vertex) or setup records (64
 // bytes a triangle) reach past a 32-bit byte offset: shaded by instances that
-// form 64-bit addresses.
-__host__ __device__ inline bool far_records(const FrameParams &fp)
+// form 64-bit addresses (FrameParams::far).
+inline bool far_records(uint32_t num_verts, uint32_t num_tris)
 {
-    return fp.num_verts > 0xFFFFFFFFu / 48u || fp.num_tris > (1u << 26);
+    return num_verts > 0xFFFFFFFFu / 48u || num_tris > (1u << 26);
 }
 
 // Launch stages whose grids are shared by all jobs of a launch: block b of

@@ -2724,7 +2724,7 @@ __device__ __forceinline__ uint32_t light_pixel_exact(const MapColours &c, float
 }
 
 // Byte offset of vertex i's 48-byte attribute record, where 32 bits hold it
-// (kFar = false: far_records): a wave addresses the records from a scalar base,
+// (kFar = false): a wave addresses the records from a scalar base,
 // without the quarter-rate 64-bit multiplies.  With the wave-uniform mesh's
 // fields read by scalar loads: 8K terrain 285 -> 279 us, 4K 78.4 -> 76.4, 7
 // views 165 -> 161.
@@ -2932,7 +2932,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kSplit && !
     const FrameParams &fp = J.fp;
     // another instance shades this frame: the other sampling mode's, or one
     // for the other attribute layout or the other reach
-    if ((fp.sample_state != 0) != kLinear || (J.sattr != nullptr) != kSplit || far_records(fp) != kFar) return;
+    if ((fp.sample_state != 0) != kLinear || (J.sattr != nullptr) != kSplit || (fp.far != 0) != kFar) return;
     // the frame's counters are final once resolve has run: the job's first
     // block copies them to the renderer's pinned host block (k_publish does
     // this for jobs that are not shaded)

@@ -24,7 +24,7 @@ RAST_OK = 0
 VIS_NONE = 0xFFFFFFFF
 BIN_EXACT, BIN_LEARNED, BIN_PREVFRAME = 0, 1, 2
 DRAW_TEXTURE, DRAW_TEXTURE_GLOBAL = 0, 1
-FLAG_TIMING, FLAG_NO_SHADE, FLAG_GRAPH = 1, 2, 4
+FLAG_TIMING, FLAG_NO_SHADE, FLAG_GRAPH, FLAG_FAR = 1, 2, 4, 8
 RESOLVE_PER_TILE, RESOLVE_PERSISTENT, RESOLVE_PERSISTENT_SHADE = 0, 1, 2
 DEBUG_VERTEX_POS, DEBUG_VERTEX_ATTR, DEBUG_TRI_RECORDS, DEBUG_TRI_ALIVE, DEBUG_TILE_COUNTS, DEBUG_BIG_LIST, DEBUG_TILE_CAPS = range(7)
 

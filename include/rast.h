@@ -103,6 +103,9 @@ typedef struct {
  * reference counterpart: it replaces the per-stage launches of
  * CCR/CUDARenderer.cu:237-330 with one graph launch.  Ignored with TIMING. */
 #define RAST_FLAG_GRAPH 4u
+/* Shade with the 64-bit record addresses of scenes above 89 million vertices or
+ * 67 million triangles, whatever the scene's size (the same frame; for tests). */
+#define RAST_FLAG_FAR 8u
 
 /* Frame statistics: CCR/CUDARenderer.h:63-64 (visible / total triangles) and
  * the per-stage milliseconds of the BENCHMARK build (CCR/CUDARenderer.cu:344-353). */
