@@ -38,6 +38,7 @@
 //              frame counters to the host (k_publish for unshaded jobs)
 #include <hip/hip_runtime.h>
 
+#include "rast_bounds.h"
 #include "rast_capacity.h"
 #include "rast_launch.h"
 
@@ -360,14 +361,6 @@ __device__ __forceinline__ uint32_t claim_slot(uint32_t *cursor, uint32_t t)
 __device__ __forceinline__ float m4(const float *m, int r, int c) { return m[c * 4 + r]; }
 
 // Normalize (CCR/Vector.h:41-55): m = sqrt(Dot(v,v)); v *= 1/m; zero stays zero.
-__device__ __forceinline__ void normalize3(float &x, float &y, float &z)
-{
-    const float m = sqrtf(x * x + y * y + z * z);
-    if (m == 0.f) { x = 0.f; y = 0.f; z = 0.f; return; }
-    const float inv = 1.f / m;
-    x *= inv; y *= inv; z *= inv;
-}
-
 __device__ __forceinline__ bool all_outside(float a, float b, float c, float lo, float hi)
 {
     return (a < lo && b < lo && c < lo) || (a > hi && b > hi && c > hi);
@@ -716,52 +709,6 @@ __global__ __launch_bounds__(256) void k_vertex_boxes(const uint32_t *__restrict
     }
 }
 
-// Whether every triangle with corners in the box [lo, hi] fails the evaluated
-// frustum test: all its corners outside one plane of the view volume.  An
-// evaluated clip coordinate is within 4.0003 u S of the exact affine value (S:
-// its row's term magnitudes, largest over the box; u = 2^-24), its quotient by
-// w within u more, and the values formed here, at the box's eight corners,
-// within 4.0003 u S too: with all corners' w on one side of zero by 16 u Sw
-// and, after multiplying by that sign, x + w, w - x and so on beyond 32 u (Sx
-// + Sw), each evaluated quotient of every point of the box is on the far side
-// of its plane.  A box reaching across w = 0, or with values that overflow or
-// are not finite, is not culled.
-__device__ __forceinline__ bool box_outside(const float *wvp, const float4 lo, const float4 hi)
-{
-    const float u = 1.0f / 16777216.0f;
-    const float ax = fmaxf(fabsf(lo.x), fabsf(hi.x)), ay = fmaxf(fabsf(lo.y), fabsf(hi.y));
-    const float az = fmaxf(fabsf(lo.z), fabsf(hi.z));
-    float m[16], S[4];
-#pragma unroll
-    for (int k = 0; k < 16; ++k) m[k] = ldg(wvp + k);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) S[r] = fabsf(m[r]) * ax + fabsf(m[4 + r]) * ay + fabsf(m[8 + r]) * az + fabsf(m[12 + r]);
-    if (!(S[0] < 1.0e30f && S[1] < 1.0e30f && S[2] < 1.0e30f && S[3] < 1.0e30f)) return false;
-    const float ew = 16.0f * u * S[3] + 1.0e-30f;
-    const float ex = 32.0f * u * (S[0] + S[3]), ey = 32.0f * u * (S[1] + S[3]), ez = 32.0f * u * (S[2] + S[3]);
-    uint32_t out = 0xFFu;  // planes every corner so far is beyond; bits 6, 7: w > 0, w < 0
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const float x = c & 1 ? hi.x : lo.x, y = c & 2 ? hi.y : lo.y, z = c & 4 ? hi.z : lo.z;
-        float v[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = m[r] * x + m[4 + r] * y + m[8 + r] * z + m[12 + r];
-        const float sg = v[3] < 0.f ? -1.f : 1.f, w = fabsf(v[3]);
-        const float X = v[0] * sg, Y = v[1] * sg, Z = v[2] * sg;
-        uint32_t b = 0;
-        b |= X + w < -ex ? 1u : 0u;
-        b |= X - w > ex ? 2u : 0u;
-        b |= Y + w < -ey ? 4u : 0u;
-        b |= Y - w > ey ? 8u : 0u;
-        b |= Z < -ez ? 16u : 0u;
-        b |= Z - w > ez ? 32u : 0u;
-        b |= v[3] > ew ? 64u : 0u;
-        b |= v[3] < -ew ? 128u : 0u;
-        out &= b;
-    }
-    return (out & 0xC0u) != 0u && (out & 0x3Fu) != 0u;
-}
-
 // The cull stage, workgroups of the vertex launch: one thread per block of 256
 // triangles tests its box and puts a block that may be in view on the setup
 // pass's list (block, mesh entry); the others have no survivors.  In a
@@ -781,7 +728,13 @@ __device__ __forceinline__ void cull_block(const DevMesh *__restrict__ meshes, c
         mi = ldg(block_mesh + b);
         const DevMesh *M = meshes + mi;
         const float4 *box = ldg(&M->boxes) + 2 * (size_t)(b - ldg(&M->tri_block0));
-        in = !box_outside(M->wvp, ldg(box), ldg(box + 1));
+        const float4 lo = ldg(box), hi = ldg(box + 1);
+        float m[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) m[k] = ldg(M->wvp + k);
+        const float3 a = make_float3(lo.x, lo.y, lo.z), c = make_float3(hi.x, hi.y, hi.z);
+        const BoxMargins g = box_margins(m, a, c, 1.f);
+        in = !box_culled(box_beyond(m, a, c, g), g);
         if (!in) stg(ldg(&jobs[ldg(&M->job)].alive_part) + b, 0u);
     }
     // places on the list: one atomic per workgroup (per wave, 7 views' 1,700
@@ -799,18 +752,12 @@ __device__ __forceinline__ void cull_block(const DevMesh *__restrict__ meshes, c
 
 // The entries [0, min(n, 64)) of a vertex group whose view the reach [lo, hi] of a
 // chunk of its vertices may be in, as bits; a chunk out of a view is not
-// transformed for it.  Eight entries at a time, one box corner per lane, with
-// the tests of box_outside at twice its margins: then the exact values at every
-// point of the reach, within 4.0003 u S of the ones formed here, clear
-// box_outside's margins by more than its own error, so that every box inside
-// this one is culled too, and the setup pass reads no position that was not
-// written.  (box_outside's S are no larger, the boxes lying inside this one.)
+// transformed for it.  Eight entries at a time, one box corner per lane, at twice
+// the cull stage's margins: then every box inside this one is culled too, and
+// the setup pass reads no position that was not written.
 __device__ __forceinline__ uint64_t entries_in_view(const DevMesh *__restrict__ meshes,
                                                     const uint32_t *__restrict__ entries, uint32_t n, float3 lo, float3 hi)
 {
-    const float u = 1.0f / 16777216.0f;
-    const float ax = fmaxf(fabsf(lo.x), fabsf(hi.x)), ay = fmaxf(fabsf(lo.y), fabsf(hi.y));
-    const float az = fmaxf(fabsf(lo.z), fabsf(hi.z));
     const uint32_t lane = lane_id();
     const float x = lane & 1u ? hi.x : lo.x, y = lane & 2u ? hi.y : lo.y, z = lane & 4u ? hi.z : lo.z;
     n = n < 64u ? n : 64u;
@@ -818,34 +765,18 @@ __device__ __forceinline__ uint64_t entries_in_view(const DevMesh *__restrict__ 
     for (uint32_t e0 = 0; e0 < n; e0 += 8u) {
         const uint32_t e = e0 + (lane >> 3);
         const float *wvp = meshes[ldg(entries + (e < n ? e : e0))].wvp;
-        float v[4], S[4];
+        float m[16];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float mx = ldg(wvp + r), my = ldg(wvp + 4 + r), mz = ldg(wvp + 8 + r), mw = ldg(wvp + 12 + r);
-            S[r] = fabsf(mx) * ax + fabsf(my) * ay + fabsf(mz) * az + fabsf(mw);
-            v[r] = mx * x + my * y + mz * z + mw;
-        }
-        const bool fine = S[0] < 1.0e30f && S[1] < 1.0e30f && S[2] < 1.0e30f && S[3] < 1.0e30f;
-        const float ew = 32.0f * u * S[3] + 2.0e-30f;
-        const float ex = 64.0f * u * (S[0] + S[3]), ey = 64.0f * u * (S[1] + S[3]), ez = 64.0f * u * (S[2] + S[3]);
-        const float sg = v[3] < 0.f ? -1.f : 1.f, w = fabsf(v[3]);
-        const float X = v[0] * sg, Y = v[1] * sg, Z = v[2] * sg;
-        uint32_t b = 0;  // planes this corner is beyond; bits 6, 7: w > 0, w < 0
-        b |= X + w < -ex ? 1u : 0u;
-        b |= X - w > ex ? 2u : 0u;
-        b |= Y + w < -ey ? 4u : 0u;
-        b |= Y - w > ey ? 8u : 0u;
-        b |= Z < -ez ? 16u : 0u;
-        b |= Z - w > ez ? 32u : 0u;
-        b |= v[3] > ew ? 64u : 0u;
-        b |= v[3] < -ew ? 128u : 0u;
+        for (int k = 0; k < 16; ++k) m[k] = ldg(wvp + k);
+        const BoxMargins g = box_margins(m, lo, hi, 2.f);
+        uint32_t b = beyond_planes(m, x, y, z, g);
         // over the entry's eight corners: pairs, quads, then the quad beside
         b &= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b, 0xB1, 0xF, 0xF, false);
         b &= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b, 0x4E, 0xF, 0xF, false);
         b &= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b, 0x141, 0xF, 0xF, false);
-        const uint64_t in = __ballot(e < n && !(fine && (b & 0xC0u) != 0u && (b & 0x3Fu) != 0u));
+        const uint64_t in = __ballot(e < n && !box_culled(b, g));
 #pragma unroll
-        for (uint32_t g = 0; g < 8; ++g) keep |= (in >> (8u * g) & 1ull) << (e0 + g);
+        for (uint32_t k = 0; k < 8; ++k) keep |= (in >> (8u * k) & 1ull) << (e0 + k);
     }
     return keep;
 }
@@ -1110,56 +1041,6 @@ __device__ __forceinline__ void queue_entry(const JobDesc &J, uint32_t tl, uint3
         if (o < J.ovf_cap) stg(J.ovf + o, make_uint2(tl, gid));
         else J.counters->storage_overflow = 1;
     }
-}
-
-// Whether the face normal (fx, fy, fz), normalized as normalize3 does, makes a
-// dot product above 0 (sign = 1) or below 0 (sign = -1) with the camera's
-// forward c, decided as the binary32 evaluation decides it.  With s the dot
-// product of the unnormalized normal, evaluated in binary32, T the sum of its
-// terms' magnitudes and u = 2^-24: s is within 3.0001 u T of the exact product
-// E, and the evaluated product of the normalized normal within 4.0001 u T inv
-// of E inv (one rounding each in the scaled component and the term, two in the
-// sum), so where |s| > 8 u T both have E's sign.  T > 1e-18 and components
-// below 1e18 keep the squares and the products in range.  Elsewhere the
-// normalized form itself is evaluated (a square root and a division).
-__device__ __forceinline__ bool faces(const float *c, float fx, float fy, float fz, float sign)
-{
-    const float p0 = c[0] * fx, p1 = c[1] * fy, p2 = c[2] * fz;
-    const float s = (p0 + p1) + p2;
-    const float T = (fabsf(p0) + fabsf(p1)) + fabsf(p2);
-    if (fabsf(s) > T * (8.0f / 16777216.0f) && T > 1.0e-18f && fmaxf(fmaxf(fabsf(fx), fabsf(fy)), fabsf(fz)) < 1.0e18f)
-        return s * sign > 0.f;
-    normalize3(fx, fy, fz);
-    const float cv = c[0] * fx + c[1] * fy + c[2] * fz;
-    return sign > 0.f ? !(cv <= 0.f) : !(cv >= 0.f);
-}
-
-// How far left of (or above) a triangle's smallest corner coordinate a pixel
-// of its range may lie and still pass the three evaluated edge tests.  A pixel
-// d > 0 left of all corners has barycentric weights summing to 1 whose
-// x-offsets, all at least d, sum to 0: the negative weights sum to at least
-// d / w in magnitude (w, h the corners' extent), so one exact edge value is at
-// most -A d / (2 w), A the exact |area|; with the opposite winding one is at
-// most -A / 3.  The evaluated edge value is within 4.0002 u ((w + 2) h +
-// (h + 2) w) <= 8.001 u (w + 2)(h + 2) of the exact one (u = 2^-24; the range
-// reaches at most 2 pixels past the corners; roundings of the differences,
-// the products and their difference), and area within 8.001 u w h of A.  So
-// the pixel fails where d > 32.01 u max(w, 2)(w + 2)(h + 2) / area: an area
-// too small to be trusted (below 16 u w h) makes that more than the 2 pixels
-// in question, and as d <= 2 a larger one leaves A / 3 above the edge values'
-// error.  34 u and the larger extent cover both axes and the roundings made
-// here.
-__device__ __forceinline__ float edge_reach(float w, float h, float area)
-{
-    return (34.0f / 16777216.0f) * fmaxf(fmaxf(w, h), 2.f) * ((w + 2.f) * (h + 2.f)) * __builtin_amdgcn_rcpf(area);
-}
-
-// The first pixel at or after lo that a triangle with smallest corner
-// coordinate mn can cover: pixels before mn - reach - 2^-22 |mn| are passed
-// over (the last term covers the rounding of the difference).
-__device__ __forceinline__ int first_pixel(float mn, float reach, int lo)
-{
-    return (int)ceilf(fmaxf(mn - (reach + fabsf(mn) * (4.0f / 16777216.0f)), (float)lo));
 }
 
 // TA_Kernel + TB_Kernel (CCR/CUDARenderer.cu:702-796,903-988) on the CPU

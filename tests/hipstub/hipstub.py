@@ -22,9 +22,9 @@ def run(cmd):
 
 
 def build(out_dir, extra=(), link=()):
-    """librast_host.so in out_dir, of SOURCES, layout.hip and the stub."""
+    """librast_host.so in out_dir, of SOURCES, layout.hip, bounds.hip and the stub."""
     objs = []
-    for src in SOURCES + [os.path.join(HERE, "layout.hip")]:
+    for src in SOURCES + [os.path.join(HERE, "layout.hip"), os.path.join(HERE, "bounds.hip")]:
         o = os.path.join(out_dir, os.path.basename(src) + ".o")
         run([HIPCC, *FLAGS, *extra, "-c", src, "-o", o])
         objs.append(o)
