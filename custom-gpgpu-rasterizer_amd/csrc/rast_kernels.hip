@@ -315,12 +315,24 @@ __device__ __forceinline__ void publish_counters(const JobDesc &J, uint32_t *red
     constexpr uint32_t kOvf = offsetof(FrameCounters, ovf_entries) / 4;
     constexpr uint32_t kPastFixed = offsetof(FrameCounters, past_fixed) / 4;
     constexpr uint32_t kPastSpill = offsetof(FrameCounters, past_spill) / 4;
+    // the words as they are, in flight beside the sums' loads: what lies beyond
+    // the regions of a frame that has them is on its overflow list
+    uint32_t word = threadIdx.x < W ? threadIdx.x : 0u;
+    bool measured = true;
+    if (word == kPastFixed) {
+        measured = J.stride || (!J.single && J.trial_stride);
+        if (J.stride) word = kOvf;
+    } else if (word == kPastSpill) {
+        measured = J.spill_stride || (J.single && J.trial_stride);
+        if (J.spill_stride) word = kOvf;
+    }
+    uint32_t v = ldg(reinterpret_cast<const uint32_t *>(J.counters) + word);
+    const unsigned long long top = J.counters->capacity_top;
     const uint32_t alive = block_sum<NW>(J.alive_part + J.alive_part0, J.alive_parts, red);
     const uint32_t pairs = J.single ? block_sum<NW>(J.tile_count, J.fp.tiles_x * J.fp.tiles_y, red) : 0u;
     if (threadIdx.x < W) {
-        uint32_t v = reinterpret_cast<const uint32_t *>(J.counters)[threadIdx.x];
         if (threadIdx.x == 0) v = alive;
-        const unsigned long long top = J.counters->capacity_top;
+        if (!measured) v = kNotMeasured;
         const uint32_t top32 = (uint32_t)(top < 0xFFFFFFFFull ? top : 0xFFFFFFFFull);
         if (threadIdx.x == kPairs) v = J.single ? pairs : top32;
         if (J.single) {
@@ -328,9 +340,6 @@ __device__ __forceinline__ void publish_counters(const JobDesc &J, uint32_t *red
             if (threadIdx.x == kCapTotal) v = (uint32_t)(top < J.queue_cap ? top : J.queue_cap);
             if (threadIdx.x == kCapWanted) v = top32;
         }
-        const uint32_t ovf = reinterpret_cast<const uint32_t *>(J.counters)[kOvf];
-        if (threadIdx.x == kPastFixed) v = J.stride ? ovf : !J.single && J.trial_stride ? v : kNotMeasured;
-        if (threadIdx.x == kPastSpill) v = J.spill_stride ? ovf : J.single && J.trial_stride ? v : kNotMeasured;
         reinterpret_cast<volatile uint32_t *>(J.host_counters)[threadIdx.x] = v;
     }
 }
