@@ -38,3 +38,10 @@ def random_triangle_scene(seed, n_tris, spread=1.2, zmin=-6.0, zmax=-1.5):
             pts.append((float(c[0] + d[0]) * -z / 2, float(c[1] + d[1]) * -z / 2, float(z + rng.normal(0, 0.3))))
         tris.append((3 * t, 3 * t + 1, 3 * t + 2))
     return S.Scene([mesh(pts, tris)])
+
+
+def turned(scene):
+    """The scene with every triangle's corner order reversed (its other side drawn)."""
+    for m in scene.meshes:
+        m.indices = np.ascontiguousarray(m.indices.reshape(-1, 3)[:, ::-1]).ravel()
+    return scene

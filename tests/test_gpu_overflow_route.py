@@ -6,7 +6,7 @@ import pytest
 
 import rast as R
 import scenes as S
-from scene_util import screen_camera
+from scene_util import screen_camera, turned
 from test_gpu_fixed_regions import check, pixel_triangles
 
 pytestmark = pytest.mark.gpu
@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 def test_first_frame_beyond_the_overflow_list(policy):
     # 64 tiles of 16,384 entries each, most of them wanted by 60,000 triangles
     W = H = 64
-    scene = pixel_triangles(np.random.default_rng(5), 60000, 0.5, 0.5, 63.5, 63.5, 45.0, W, H)
+    scene = turned(pixel_triangles(np.random.default_rng(5), 60000, 0.5, 0.5, 63.5, 63.5, 45.0, W, H))
     cam, opts = screen_camera(), S.Opts(cull_mode=S.CULL_NONE)
     away = S.Camera(position=(0.0, 0.0, 400.0), forward=cam.forward, fov_deg=cam.fov_deg, near_z=cam.near_z, far_z=1e4)
     with R.Renderer(W, H, tile=8, big_threshold=1024) as r:
@@ -27,6 +27,7 @@ def test_first_frame_beyond_the_overflow_list(policy):
         counts = check(r, scene, cam, opts, W, H, 8)
         assert np.maximum(counts.astype(np.int64) - 16384, 0).sum() > 1 << 20
         assert r.stats()["rerenders"] == 1
+        assert np.count_nonzero(r.readback()[0] != R.VIS_NONE) > W * H // 2
         for _ in range(20):  # they fit
             r.render(away, opts, policy)
         check(r, scene, away, opts, W, H, 8)
