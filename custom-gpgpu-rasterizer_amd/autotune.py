@@ -11,7 +11,7 @@ given class of frames fastest on the device at hand:
               screen-wide list instead of per-tile queues     rast_setup_bins
   micro       bounding-box pixel count up to which a
               triangle is rasterized at setup, unbinned       rast_set_tuning
-  small       tile-clipped pixel count from which the
+  small       tile-clipped pixel count (at least half the tile) from which the
               resolve pass rasterizes a triangle per pixel    rast_set_tuning
 
 and, for the single-pass policies, the per-tile queue depth, capacity =
@@ -123,7 +123,15 @@ def queue_depth(width: int, height: int, tris: int, policy: str = "learned",
 
 
 def candidates(tiles=TILES, micros=MICROS, smalls=SMALLS, bigs=BIGS) -> List[Params]:
-    return [Params(t, m, s, b) for t, m, s, b in itertools.product(tiles, micros, smalls, bigs)]
+    """Every combination, but of the small limits that act alike in a tile (those
+    below half its pixels, and those above all of them) the first only."""
+    out, seen = [], set()
+    for t, m, s, b in itertools.product(tiles, micros, smalls, bigs):
+        key = (t, m, min(max(s, t * t // 2), t * t + 1), b)
+        if key not in seen:
+            seen.add(key)
+            out.append(Params(t, m, s, b))
+    return out
 
 
 def time_batch(R, jobs, reps: int) -> float:

@@ -175,9 +175,11 @@ int rast_setup_bins(rast_renderer *r, uint32_t tile_size, uint32_t big_threshold
  * per-thread pixel coverage from the bin size, CCR/main.cpp:372-389):
  * triangles whose bounding box has at most micro_limit pixels are rasterized
  * directly at setup with 64-bit atomic min (0 = bin every triangle); inside a
- * tile, triangles covering at most small_limit pixels of it are rasterized one
- * per lane, larger ones one pixel per lane.  Defaults 16 / 16.  The output
- * does not depend on either value. */
+ * tile, triangles whose pixel range holds less than small_limit pixels of it are
+ * rasterized as a list of their pixels, larger ones one pixel per lane.  A
+ * small_limit below half the tile's pixels (32, 128 or 512; 128 where a 32-pixel
+ * tile is resolved in quarters) acts as that half.  Defaults 16 / 16.  The
+ * output does not depend on either value. */
 int rast_set_tuning(rast_renderer *r, uint32_t micro_limit, uint32_t small_limit);
 /* Resolve-stage launch form (the persistent kernel of the reference's TODO,
  * CCR/CUDARenderer.cu:284-285): RAST_RESOLVE_PER_TILE (default) one
