@@ -1996,8 +1996,11 @@ extern "C" int rast_debug_read(rast_renderer *r, int which, void *dst, size_t by
     size_t size = 0;
     const void *src = nullptr;
     std::vector<uint32_t> tmp;
-    if (dst && (which == RAST_DEBUG_VERTEX_POS || which == RAST_DEBUG_VERTEX_ATTR || which == RAST_DEBUG_TRI_RECORDS ||
-                which == RAST_DEBUG_TRI_ALIVE))
+    if (which == (RAST_DEBUG_VERTEX_POS | RAST_DEBUG_AS_DRAWN) || which == (RAST_DEBUG_VERTEX_ATTR | RAST_DEBUG_AS_DRAWN) ||
+        which == (RAST_DEBUG_TRI_RECORDS | RAST_DEBUG_AS_DRAWN))
+        which &= ~RAST_DEBUG_AS_DRAWN;
+    else if (dst && (which == RAST_DEBUG_VERTEX_POS || which == RAST_DEBUG_VERTEX_ATTR || which == RAST_DEBUG_TRI_RECORDS ||
+                     which == RAST_DEBUG_TRI_ALIVE))
         RAST_TRY(complete_debug(r));
     switch (which) {
     case RAST_DEBUG_VERTEX_POS: size = (size_t)r->total_verts * 16; src = r->pos4.p; break;

@@ -27,6 +27,7 @@ DRAW_TEXTURE, DRAW_TEXTURE_GLOBAL = 0, 1
 FLAG_TIMING, FLAG_NO_SHADE, FLAG_GRAPH, FLAG_FAR = 1, 2, 4, 8
 RESOLVE_PER_TILE, RESOLVE_PERSISTENT, RESOLVE_PERSISTENT_SHADE = 0, 1, 2
 DEBUG_VERTEX_POS, DEBUG_VERTEX_ATTR, DEBUG_TRI_RECORDS, DEBUG_TRI_ALIVE, DEBUG_TILE_COUNTS, DEBUG_BIG_LIST, DEBUG_TILE_CAPS = range(7)
+DEBUG_AS_DRAWN = 256
 
 EXPORTS = [
     "rast_last_error", "rast_device_query", "rast_renderer_create", "rast_renderer_destroy", "rast_setup_bins",

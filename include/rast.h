@@ -265,7 +265,11 @@ enum {
     RAST_DEBUG_TRI_ALIVE = 3,   /* u8 per triangle */
     RAST_DEBUG_TILE_COUNTS = 4, /* u32 per tile: queue length */
     RAST_DEBUG_BIG_LIST = 5,    /* u32 count followed by the IDs */
-    RAST_DEBUG_TILE_CAPS = 6    /* u32 per tile: single-pass queue capacity of the last frame */
+    RAST_DEBUG_TILE_CAPS = 6,   /* u32 per tile: single-pass queue capacity of the last frame */
+    /* A frame forms only what it reads of positions, attributes and records; the
+     * rest is formed by rast_debug_read.  Or'd with one of these three: as the frame
+     * left it (an entry it did not form holds what was there before). */
+    RAST_DEBUG_AS_DRAWN = 256
 };
 int rast_debug_read(rast_renderer *r, int which, void *dst, size_t bytes, size_t *size_out);
 
