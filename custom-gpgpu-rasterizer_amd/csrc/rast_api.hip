@@ -1033,7 +1033,7 @@ static int plan_wait(LaunchPlan &P)
     return plan_wait_block(P, 1);
 }
 
-constexpr uint64_t kViewChunks = 16384;
+constexpr uint64_t kViewChunks = 16384;  // (build_plan has the figures)
 
 static int dev_alloc(DBuf &b, size_t bytes)
 {
@@ -1193,7 +1193,11 @@ static int build_plan(LaunchPlan &P, rast_renderer *const *rs, uint32_t n, int h
     // in only.  The test is a launch of its own, 5 to 9 us, so it takes a vertex
     // pass that is several times that (7 views of 1.35 M vertices, 74 K chunks to
     // transform: 110 -> 9 + 64 us; 12 views of a small object, 3.8 K chunks: 15 us
-    // in all).  A frame of one view mostly sees its scene.
+    // in all).  A frame of one view mostly sees its scene.  Launches with the test
+    // and without it, a 1080p view and six cube-map faces over terrain: 9.7 K chunks
+    // 792 and 788 us, 20 K 1,093 and 1,095, 40 K 1,531 and 1,540, 74 K 2,077 and
+    // 2,107.  Views that all see the whole scene pay for it: 48 of an object, 61 K
+    // chunks, 294 and 288.
     uint64_t view_chunks = 0;
     for (uint32_t g : vs_group)
         if (members[g].size() > 1) view_chunks += members[g].size();
