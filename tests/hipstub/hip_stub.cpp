@@ -217,12 +217,14 @@ hipError_t hipMemcpy2D(void *d, size_t dp, const void *s, size_t sp, size_t w, s
 }
 hipError_t hipMemset(void *d, int v, size_t n)
 {
+    std::lock_guard<std::recursive_mutex> l(g_mutex);
     if (room(g_device, d) < n) wrong("set of", d);
     return memset(d, v, n), hipSuccess;
 }
 hipError_t hipGetSymbolAddress(void **p, const void *)
 {
     static char *mem = nullptr;
+    std::lock_guard<std::recursive_mutex> l(g_mutex);
     if (!mem) {
         mem = (char *)calloc(1, 64u << 20);
         g_device[mem] = 64u << 20;
@@ -321,6 +323,7 @@ hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t g, hipGraphNode_t *
 hipError_t hipGraphDestroy(hipGraph_t g)
 {
     Graph *p = live<Graph>(g_graphs, g, "graph");
+    std::lock_guard<std::recursive_mutex> l(g_mutex);
     g_graphs.erase(p);
     delete p;
     return hipSuccess;
@@ -328,6 +331,7 @@ hipError_t hipGraphDestroy(hipGraph_t g)
 hipError_t hipGraphExecDestroy(hipGraphExec_t e)
 {
     Graph *p = live<Graph>(g_execs, e, "graph instance");
+    std::lock_guard<std::recursive_mutex> l(g_mutex);
     g_execs.erase(p);
     delete p;
     return hipSuccess;
@@ -369,12 +373,10 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t, h
     Stream *p = s ? live<Stream>(g_streams, s, "stream") : nullptr;
     const Launch l{ names().at(f), g.x, b.x };
     if (!g.x || !b.x) return ret(hipErrorInvalidConfiguration);
-    if (l.name.find("k_read_out") != std::string::npos) {
-        std::lock_guard<std::recursive_mutex> lock(g_mutex);
-        read_out(args);
-    }
+    std::unique_lock<std::recursive_mutex> lock(g_mutex);
+    if (l.name.find("k_read_out") != std::string::npos) read_out(args);
     if (Stream *c = capture_of(p)) c->graph.push_back(l);
-    else if (g_callback) g_callback(l.name.c_str(), l.grid, l.block);
+    else if (lock.unlock(); g_callback) g_callback(l.name.c_str(), l.grid, l.block);
     return hipSuccess;
 }
 void **__hipRegisterFatBinary(const void *) { static void *m[1]; return m; }
