@@ -15,7 +15,6 @@
 #include <memory>
 #include <mutex>
 #include <new>
-#include <string>
 #include <thread>
 #include <unordered_map>
 #include <vector>
@@ -29,25 +28,23 @@ using namespace rast;
 
 // ----------------------------------------------------------------- errors
 
-static thread_local std::string g_last_error;
+static thread_local char g_last_error[512];
 
 int rast_set_error(int code, const char *fmt, ...)
 {
-    char buf[512];
     va_list ap;
     va_start(ap, fmt);
-    vsnprintf(buf, sizeof buf, fmt, ap);
+    vsnprintf(g_last_error, sizeof g_last_error, fmt, ap);
     va_end(ap);
-    g_last_error = buf;
     return code;
 }
 
 extern "C" int rast_last_error(char *buf, size_t n)
 {
-    const size_t len = g_last_error.size();
+    const size_t len = strlen(g_last_error);
     if (buf && n) {
         const size_t c = len < n - 1 ? len : n - 1;
-        memcpy(buf, g_last_error.data(), c);
+        memcpy(buf, g_last_error, c);
         buf[c] = 0;
     }
     return (int)len;
@@ -320,6 +317,7 @@ static int new_renderer(int device, uint32_t width, uint32_t height, rast_render
     if (hipGetDeviceCount(&n) != hipSuccess || n == 0) return rast_set_error(RAST_E_NO_DEVICE, "no HIP device");
     if (device < 0 || device >= n) return rast_set_error(RAST_E_INVALID_ARG, "device %d out of range", device);
     HIP_TRY(hipSetDevice(device));
+    if (scene_src) scene_src->views.reserve(scene_src->views.size() + 1);
     rast_renderer *r = new (std::nothrow) rast_renderer();
     if (!r) return rast_set_error(RAST_E_OUT_OF_MEMORY, "host allocation failed");
     r->device = device;
@@ -350,16 +348,16 @@ static int new_renderer(int device, uint32_t width, uint32_t height, rast_render
 }
 
 extern "C" int rast_renderer_create(int device, uint32_t width, uint32_t height, rast_renderer **out)
-{
+try {
     return new_renderer(device, width, height, nullptr, out);
-}
+} RAST_CATCH
 
 extern "C" int rast_renderer_create_view(rast_renderer *owner, uint32_t width, uint32_t height, rast_renderer **out)
-{
+try {
     if (!owner) return rast_set_error(RAST_E_INVALID_ARG, "rast_renderer_create_view: null owner");
     if (owner->scene_src) owner = owner->scene_src;  // a view of a view draws the same scene
     return new_renderer(owner->device, width, height, owner, out);
-}
+} RAST_CATCH
 
 // Detaches a mesh from its renderer, whose frames are gone, and with it its
 // device memory; the handle stays allocated until rast_mesh_destroy.
@@ -455,7 +453,7 @@ extern "C" int rast_set_resolve_mode(rast_renderer *r, int mode)
 }
 
 extern "C" int rast_resize(rast_renderer *r, uint32_t width, uint32_t height)
-{
+try {
     if (!r) return rast_set_error(RAST_E_INVALID_ARG, "rast_resize: null renderer");
     if (width == 0 || height == 0 || width > 16384 || height > 16384)
         return rast_set_error(RAST_E_INVALID_ARG, "framebuffer %ux%u out of range (1..16384)", width, height);
@@ -465,14 +463,14 @@ extern "C" int rast_resize(rast_renderer *r, uint32_t width, uint32_t height)
     r->have_prev = false;
     forget_overflow(r);
     return alloc_framebuffers(r);
-}
+} RAST_CATCH
 
 // ------------------------------------------------------------------ meshes
 
 extern "C" int rast_mesh_create(rast_renderer *r, const rast_ivertex *verts, uint32_t num_verts,
                                 const uint32_t *indices, uint32_t num_indices, int topology, const float world[16],
                                 rast_mesh **out)
-{
+try {
     if (!out) return rast_set_error(RAST_E_INVALID_ARG, "rast_mesh_create: null output");
     *out = nullptr;
     if (!r || !verts || !indices || num_verts == 0 || num_indices == 0)
@@ -503,6 +501,7 @@ extern "C" int rast_mesh_create(rast_renderer *r, const rast_ivertex *verts, uin
             if (a != a || b != b) attr_max = INFINITY;
         }
     }
+    r->meshes.reserve(r->meshes.size() + 1);
     rast_mesh *m = new (std::nothrow) rast_mesh();
     MeshMemory *mem = m ? new (std::nothrow) MeshMemory() : nullptr;
     if (mem) {
@@ -547,10 +546,10 @@ extern "C" int rast_mesh_create(rast_renderer *r, const rast_ivertex *verts, uin
     r->have_prev = false;
     *out = m;
     return RAST_OK;
-}
+} RAST_CATCH
 
 extern "C" int rast_mesh_destroy(rast_mesh *m)
-{
+try {
     if (!m) return rast_set_error(RAST_E_INVALID_ARG, "rast_mesh_destroy: null mesh");
     rast_renderer *r = m->r;
     if (!r) {  // its renderer is gone (and with it the device memory)
@@ -573,7 +572,7 @@ extern "C" int rast_mesh_destroy(rast_mesh *m)
     r->have_prev = false;
     r->frame_valid = false;
     return RAST_OK;
-}
+} RAST_CATCH
 
 extern "C" int rast_mesh_set_world(rast_mesh *m, const float world[16])
 {
@@ -619,7 +618,7 @@ extern "C" int rast_mesh_triangle_base(const rast_mesh *m, uint64_t *out)
 
 extern "C" int rast_texture_create_pitched(rast_renderer *r, const void *rgba8, uint32_t w, uint32_t h,
                                            size_t pitch_bytes, rast_texture **out)
-{
+try {
     if (!out) return rast_set_error(RAST_E_INVALID_ARG, "rast_texture_create: null output");
     *out = nullptr;
     if (!r || !rgba8 || !w || !h || w > 32768 || h > 32768)
@@ -628,6 +627,7 @@ extern "C" int rast_texture_create_pitched(rast_renderer *r, const void *rgba8, 
         return rast_set_error(RAST_E_INVALID_ARG, "rast_texture_create: pitch %zu below 4 x width or not a multiple of 4",
                               pitch_bytes);
     HIP_TRY(hipSetDevice(r->device));
+    r->textures.reserve(r->textures.size() + 1);
     rast_texture *t = new (std::nothrow) rast_texture();
     if (!t) return rast_set_error(RAST_E_OUT_OF_MEMORY, "host allocation failed");
     t->r = r;
@@ -647,13 +647,13 @@ extern "C" int rast_texture_create_pitched(rast_renderer *r, const void *rgba8, 
     r->textures.push_back(t);
     *out = t;
     return RAST_OK;
-}
+} RAST_CATCH
 
 extern "C" int rast_texture_create(rast_renderer *r, const uint32_t *rgba8, uint32_t w, uint32_t h,
                                    rast_texture **out)
-{
+try {
     return rast_texture_create_pitched(r, rgba8, w, h, (size_t)w * 4, out);
-}
+} RAST_CATCH
 
 extern "C" int rast_texture_destroy(rast_texture *t)
 {
@@ -863,6 +863,7 @@ static int ensure_tex_quads(rast_renderer *r)
         for (TexQuad &q : owner->tex_quads)
             if (q.t[0] == t[0] && q.t[1] == t[1] && q.t[2] == t[2] && q.t[3] == t[3]) found = &q;
         if (!found) {
+            owner->tex_quads.reserve(owner->tex_quads.size() + 1);
             TexQuad q = { { t[0], t[1], t[2], t[3] }, nullptr };
             const size_t n = (size_t)w * h;
             const hipError_t me = rast_dev_malloc((void **)&q.texels, n * sizeof(uint4));
@@ -1714,7 +1715,7 @@ static int check_frame(rast_renderer *r)
 }
 
 extern "C" int rast_render(rast_renderer *r, const rast_camera *cam, const rast_frame_opts *opts)
-{
+try {
     if (!r || !cam || !opts) return rast_set_error(RAST_E_INVALID_ARG, "rast_render: null argument");
     RAST_TRY(validate_opts(opts));
     RAST_TRY(validate_camera(cam));
@@ -1726,16 +1727,16 @@ extern "C" int rast_render(rast_renderer *r, const rast_camera *cam, const rast_
     r->last_opts = *opts;
     r->prev_valid_before = r->have_prev;
     return enqueue_frame(r);
-}
+} RAST_CATCH
 
 extern "C" int rast_sync(rast_renderer *r)
-{
+try {
     if (!r) return rast_set_error(RAST_E_INVALID_ARG, "rast_sync: null renderer");
     HIP_TRY(hipSetDevice(r->device));
     if (r->frame_pending) return check_frame(r);
     HIP_TRY(renderer_wait(r));
     return RAST_OK;
-}
+} RAST_CATCH
 
 // A frame's copy to ordinary host memory passes through pinned slots: one
 // kernel writes a piece of it in address order and raises a flag per chunk
@@ -1914,7 +1915,7 @@ static int copy_to_host(ReadSlots &slots, const HostCopy *c, int n)
 }
 
 extern "C" int rast_readback(rast_renderer *r, uint32_t *vis, float *depth, uint32_t *rgba)
-{
+try {
     if (!r) return rast_set_error(RAST_E_INVALID_ARG, "rast_readback: null renderer");
     RAST_TRY(rast_sync(r));
     if (!r->frame_valid) return rast_set_error(RAST_E_STATE, "rast_readback: no rendered frame");
@@ -1938,7 +1939,7 @@ extern "C" int rast_readback(rast_renderer *r, uint32_t *vis, float *depth, uint
     const int rc = copy_to_host(slots, staged, n);
     give_slots(slots, rc == RAST_OK);
     return rc;
-}
+} RAST_CATCH
 
 static float elapsed(rast_renderer *r, int a, int b)
 {
@@ -1952,7 +1953,7 @@ static float elapsed(rast_renderer *r, int a, int b)
 }
 
 extern "C" int rast_get_stats(rast_renderer *r, rast_stats *out)
-{
+try {
     if (!r || !out) return rast_set_error(RAST_E_INVALID_ARG, "rast_get_stats: null argument");
     RAST_TRY(rast_sync(r));
     const FrameCounters c = *r->h_counters;
@@ -1976,10 +1977,10 @@ extern "C" int rast_get_stats(rast_renderer *r, rast_stats *out)
     s.ms_total = elapsed(r, EV_START, EV_SHADE);
     *out = s;
     return RAST_OK;
-}
+} RAST_CATCH
 
 extern "C" int rast_frame_buffers(rast_renderer *r, void **vis, void **depth, void **rgba)
-{
+try {
     if (!r) return rast_set_error(RAST_E_INVALID_ARG, "rast_frame_buffers: null renderer");
     // the frame is finished and checked first (re-rendered if its queue
     // storage overflowed), as for rast_readback
@@ -1989,10 +1990,10 @@ extern "C" int rast_frame_buffers(rast_renderer *r, void **vis, void **depth, vo
     if (depth) *depth = r->depth.p;
     if (rgba) *rgba = r->rgba.p;
     return RAST_OK;
-}
+} RAST_CATCH
 
 extern "C" int rast_debug_read(rast_renderer *r, int which, void *dst, size_t bytes, size_t *size_out)
-{
+try {
     if (!r) return rast_set_error(RAST_E_INVALID_ARG, "rast_debug_read: null renderer");
     RAST_TRY(rast_sync(r));
     const uint32_t ntiles = ceil_div(r->W, r->tile) * ceil_div(r->H, r->tile);
@@ -2034,10 +2035,10 @@ extern "C" int rast_debug_read(rast_renderer *r, int which, void *dst, size_t by
     if (size_out) *size_out = size;
     if (dst && size && src) HIP_TRY(hipMemcpy(dst, src, std::min(size, bytes), hipMemcpyDeviceToHost));
     return RAST_OK;
-}
+} RAST_CATCH
 
 extern "C" int rast_renderer_set_binmodel(rast_renderer *r, rast_binmodel *m, float margin, uint32_t slack)
-{
+try {
     if (!r) return rast_set_error(RAST_E_INVALID_ARG, "rast_renderer_set_binmodel: null renderer");
     if (!(margin >= 1.f) || margin > 64.f) return rast_set_error(RAST_E_INVALID_ARG, "margin %g not in [1, 64]", margin);
     if (slack > (1u << 20)) return rast_set_error(RAST_E_INVALID_ARG, "slack %u above 2^20", slack);
@@ -2045,7 +2046,7 @@ extern "C" int rast_renderer_set_binmodel(rast_renderer *r, rast_binmodel *m, fl
     r->margin = margin;
     r->slack = slack;
     return RAST_OK;
-}
+} RAST_CATCH
 
 // ------------------------------------------------------------ timer, hooks
 
@@ -2072,7 +2073,7 @@ extern "C" int rast_timer_stop(rast_renderer *r, float *ms)
 }
 
 extern "C" int rast_draw_texture(rast_renderer *r, const rast_texture *t, int mode, int stretch, int sample_state)
-{
+try {
     if (!r || !t) return rast_set_error(RAST_E_INVALID_ARG, "rast_draw_texture: null argument");
     if (!t->r || !t->texels) return rast_set_error(RAST_E_STATE, "rast_draw_texture: the texture's renderer was destroyed");
     if (mode != RAST_DRAW_TEXTURE && mode != RAST_DRAW_TEXTURE_GLOBAL)
@@ -2089,7 +2090,7 @@ extern "C" int rast_draw_texture(rast_renderer *r, const rast_texture *t, int mo
     r->frame_pending = false;
     r->frame_valid = true;
     return RAST_OK;
-}
+} RAST_CATCH
 
 // ----------------------------------------------------------------- batching
 
@@ -2106,7 +2107,7 @@ static BatchCache g_batch;
 static std::mutex g_batch_mutex;
 
 extern "C" int rast_render_batch(const rast_job *jobs, uint32_t n)
-{
+try {
     if (!jobs || n == 0) return rast_set_error(RAST_E_INVALID_ARG, "rast_render_batch: no jobs");
     if (n > 65535) return rast_set_error(RAST_E_INVALID_ARG, "rast_render_batch: at most 65535 jobs");
     const int device = jobs[0].target ? jobs[0].target->device : 0;
@@ -2184,4 +2185,4 @@ extern "C" int rast_render_batch(const rast_job *jobs, uint32_t n)
         finish_enqueue(t);
     }
     return RAST_OK;
-}
+} RAST_CATCH

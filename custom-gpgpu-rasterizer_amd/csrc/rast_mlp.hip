@@ -536,13 +536,16 @@ static void init_params(std::vector<float> &p, int H, uint32_t seed)
 }
 
 extern "C" int rast_binmodel_create(rast_renderer *r, uint32_t hidden, uint32_t seed, rast_binmodel **out)
-{
+try {
     if (!out) return rast_set_error(RAST_E_INVALID_ARG, "rast_binmodel_create: null output");
     *out = nullptr;
     if (!r) return rast_set_error(RAST_E_INVALID_ARG, "rast_binmodel_create: null renderer");
     if (hidden != 16 && hidden != 32 && hidden != 64)
         return rast_set_error(RAST_E_INVALID_ARG, "hidden size %u not in {16, 32, 64}", hidden);
     HIP_TRY(hipSetDevice(r->device));
+    const size_t np = num_params((int)hidden);
+    std::vector<float> p(np);
+    init_params(p, (int)hidden, seed);
     rast_binmodel *m = new (std::nothrow) rast_binmodel();
     if (!m) return rast_set_error(RAST_E_OUT_OF_MEMORY, "host allocation failed");
     m->device = r->device;
@@ -556,9 +559,6 @@ extern "C" int rast_binmodel_create(rast_renderer *r, uint32_t hidden, uint32_t 
     }
     m->home = r;
     m->stream = r->stream;
-    const size_t np = num_params(m->H);
-    std::vector<float> p(np);
-    init_params(p, m->H, seed);
     int rc = ensure(m->params, np * 4);
     if (rc == RAST_OK) rc = ensure(m->grad, np * 4);
     if (rc == RAST_OK) rc = ensure(m->adam_m, np * 4);
@@ -573,7 +573,7 @@ extern "C" int rast_binmodel_create(rast_renderer *r, uint32_t hidden, uint32_t 
     }
     *out = m;
     return RAST_OK;
-}
+} RAST_CATCH
 
 extern "C" int rast_binmodel_destroy(rast_binmodel *m)
 {
@@ -618,7 +618,7 @@ extern "C" int rast_binmodel_get_params(rast_binmodel *m, float *dst, size_t cou
 }
 
 extern "C" int rast_binmodel_set_params(rast_binmodel *m, const float *src, size_t count)
-{
+try {
     if (!m || !src || count != num_params(m->H))
         return rast_set_error(RAST_E_INVALID_ARG, "rast_binmodel_set_params: bad arguments");
     RAST_TRY(model_ready(m));
@@ -628,7 +628,7 @@ extern "C" int rast_binmodel_set_params(rast_binmodel *m, const float *src, size
     HIP_TRY(hipMemset(m->adam_v.p, 0, count * 4));
     m->adam_t = 0;
     return RAST_OK;
-}
+} RAST_CATCH
 
 extern "C" int rast_binmodel_clear_data(rast_binmodel *m)
 {
@@ -638,7 +638,7 @@ extern "C" int rast_binmodel_clear_data(rast_binmodel *m)
 }
 
 extern "C" int rast_binmodel_record(rast_binmodel *m, rast_renderer *r)
-{
+try {
     if (!m || !r) return rast_set_error(RAST_E_INVALID_ARG, "rast_binmodel_record: null argument");
     RAST_TRY(rast_sync(r));
     if (!r->frame_valid || !r->frame_had_prev || r->model != m)
@@ -683,11 +683,11 @@ extern "C" int rast_binmodel_record(rast_binmodel *m, rast_renderer *r)
     HIP_TRY(hipStreamSynchronize(r->stream));
     m->n += nt;
     return RAST_OK;
-}
+} RAST_CATCH
 
 extern "C" int rast_binmodel_train(rast_binmodel *m, uint32_t epochs, uint32_t batch, float lr, float tau,
                                    float *final_loss)
-{
+try {
     if (!m || batch == 0 || batch > kMaxBatch || !(lr > 0.f) || !(tau > 0.f && tau < 1.f))
         return rast_set_error(RAST_E_INVALID_ARG, "rast_binmodel_train: bad arguments");
     if (m->n == 0) return rast_set_error(RAST_E_STATE, "rast_binmodel_train: no recorded data");
@@ -704,10 +704,10 @@ extern "C" int rast_binmodel_train(rast_binmodel *m, uint32_t epochs, uint32_t b
     HIP_TRY(hipStreamSynchronize(m->stream));
     if (final_loss) HIP_TRY(hipMemcpy(final_loss, m->loss.p, 4, hipMemcpyDeviceToHost));
     return RAST_OK;
-}
+} RAST_CATCH
 
 extern "C" int rast_binmodel_forward(rast_binmodel *m, const float *x, uint32_t n, float *pred)
-{
+try {
     if (!m || !x || !pred || n == 0) return rast_set_error(RAST_E_INVALID_ARG, "rast_binmodel_forward: bad arguments");
     RAST_TRY(model_ready(m));
     RAST_TRY(ensure(m->io_x, (size_t)n * F * 4));
@@ -718,7 +718,7 @@ extern "C" int rast_binmodel_forward(rast_binmodel *m, const float *x, uint32_t 
     HIP_TRY(hipStreamSynchronize(m->stream));
     HIP_TRY(hipMemcpy(pred, m->io_p.p, (size_t)n * 4, hipMemcpyDeviceToHost));
     return RAST_OK;
-}
+} RAST_CATCH
 
 // ------------------------------------------------ allocation-free forward
 
@@ -763,7 +763,7 @@ int noalloc_scratch(int device, float **out)
 }  // namespace
 
 extern "C" int rast_binmodel_forward_noalloc(rast_binmodel *m, const float *x, uint32_t n, float *pred)
-{
+try {
     if (!m || !x || !pred || n == 0)
         return rast_set_error(RAST_E_INVALID_ARG, "rast_binmodel_forward_noalloc: bad arguments");
     if (n > kNoAllocMaxSamples)
@@ -780,11 +780,11 @@ extern "C" int rast_binmodel_forward_noalloc(rast_binmodel *m, const float *x, u
     HIP_TRY(hipMemcpyAsync(pred, sp, (size_t)n * 4, hipMemcpyDeviceToHost, m->stream));
     HIP_TRY(hipStreamSynchronize(m->stream));
     return RAST_OK;
-}
+} RAST_CATCH
 
 extern "C" int rast_binmodel_loss_grad(rast_binmodel *m, const float *x, const float *target, uint32_t n, float tau,
                                        float *loss, float *grad)
-{
+try {
     if (!m || !x || !target || !grad || n == 0 || n > kMaxBatch)
         return rast_set_error(RAST_E_INVALID_ARG, "rast_binmodel_loss_grad: bad arguments");
     RAST_TRY(model_ready(m));
@@ -798,7 +798,7 @@ extern "C" int rast_binmodel_loss_grad(rast_binmodel *m, const float *x, const f
     HIP_TRY(hipMemcpy(grad, m->grad.p, num_params(m->H) * 4, hipMemcpyDeviceToHost));
     if (loss) HIP_TRY(hipMemcpy(loss, m->loss.p, 4, hipMemcpyDeviceToHost));
     return RAST_OK;
-}
+} RAST_CATCH
 
 int rast_model_hidden(const rast_binmodel *m) { return m ? m->H : 0; }
 const float *rast_model_params(const rast_binmodel *m) { return m ? (const float *)m->params.p : nullptr; }

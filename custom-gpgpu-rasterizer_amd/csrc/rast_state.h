@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <memory>
+#include <new>
 #include <vector>
 
 #include "rast.h"
@@ -32,6 +33,14 @@ int rast_set_error(int code, const char *fmt, ...);
         int rc_ = (expr);               \
         if (rc_ != RAST_OK) return rc_; \
     } while (0)
+
+// End of an entry point that allocates host memory (a function try block):
+// nothing is thrown across the ABI.
+#define RAST_CATCH                                                                                  \
+    catch (const std::bad_alloc &)                                                                  \
+    {                                                                                               \
+        return rast_set_error(RAST_E_OUT_OF_MEMORY, "%s: host allocation failed", __func__);        \
+    }
 
 struct DBuf {
     void *p = nullptr;

@@ -20,13 +20,27 @@
 
 #include <hip/hip_runtime_api.h>
 
-#ifndef STUB_PLAIN_DELETE  // (with a sanitizer, which does this better)
+namespace {
+thread_local int t_in_stub = 0;   // the stand-in's own allocations never fail
+thread_local long t_fail_in = -1;  // the library's that many from now does, once
+struct InStub {
+    InStub() { ++t_in_stub; }
+    ~InStub() { --t_in_stub; }
+};
+}  // namespace
+
+#ifndef STUB_PLAIN_DELETE  // (with a sanitizer, which does the rest better)
+static void *allocate(size_t n) noexcept
+{
+    if (!t_in_stub && t_fail_in >= 0 && t_fail_in-- == 0) return nullptr;
+    return malloc(n ? n : 1);
+}
 void *operator new(size_t n)
 {
-    if (void *p = malloc(n ? n : 1)) return p;
+    if (void *p = allocate(n)) return p;
     throw std::bad_alloc();
 }
-void *operator new(size_t n, const std::nothrow_t &) noexcept { return malloc(n ? n : 1); }
+void *operator new(size_t n, const std::nothrow_t &) noexcept { return allocate(n); }
 void operator delete(void *p) noexcept
 {
     // rising words: no two pointers left in it are equal, and none is an address
@@ -137,6 +151,8 @@ extern "C" {
 
 // ------------------------------------------------------------- test control
 void stub_callback(Callback c) { g_callback = c; }
+void stub_fail_new(long n) { t_fail_in = n; }  // negative: none
+long stub_fail_left() { return t_fail_in; }
 void stub_limit(size_t bytes) { g_limit = bytes; }
 void stub_lose_copies(int lose) { g_lose_copies = lose != 0; }  // readbacks raise no flags
 size_t stub_used() { return g_used; }
@@ -158,6 +174,7 @@ void *stub_pinned_of(size_t bytes, size_t k)
 // ------------------------------------------------------------------- memory
 hipError_t hipMalloc(void **p, size_t n)
 {
+    InStub in_stub;
     std::lock_guard<std::recursive_mutex> l(g_mutex);
     ++g_mallocs;
     if (g_used + n > g_limit) return *p = nullptr, ret(hipErrorOutOfMemory);
@@ -169,6 +186,7 @@ hipError_t hipMalloc(void **p, size_t n)
 }
 hipError_t hipFree(void *p)
 {
+    InStub in_stub;
     std::lock_guard<std::recursive_mutex> l(g_mutex);
     if (!p) return hipSuccess;
     auto it = g_device.find((char *)p);
@@ -180,6 +198,7 @@ hipError_t hipFree(void *p)
 }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned)
 {
+    InStub in_stub;
     std::lock_guard<std::recursive_mutex> l(g_mutex);
     *p = calloc(1, n ? n : 1);
     g_pinned[(char *)*p] = n;
@@ -187,15 +206,17 @@ hipError_t hipHostMalloc(void **p, size_t n, unsigned)
 }
 hipError_t hipHostFree(void *p)
 {
+    InStub in_stub;
     std::lock_guard<std::recursive_mutex> l(g_mutex);
     if (!p) return hipSuccess;
     if (!g_pinned.erase((char *)p)) wrong("pinned memory", p);
     free(p);
     return hipSuccess;
 }
-hipError_t hipHostGetDevicePointer(void **d, void *h, unsigned) { return *d = h, hipSuccess; }
+hipError_t hipHostGetDevicePointer(void **d, void *h, unsigned) { InStub in_stub; return *d = h, hipSuccess; }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p)
 {
+    InStub in_stub;
     std::lock_guard<std::recursive_mutex> l(g_mutex);
     memset(a, 0, sizeof *a);
     a->type = hipMemoryTypeUnregistered;
@@ -203,26 +224,30 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p)
         if ((char *)p >= q.first && (char *)p < q.first + q.second) a->type = hipMemoryTypeHost;
     return hipSuccess;
 }
-hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) { return copy(d, s, n, k); }
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) { InStub in_stub; return copy(d, s, n, k); }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t st)
 {
+    InStub in_stub;
     if (st) live<Stream>(g_streams, st, "stream");
     return copy(d, s, n, k);
 }
 hipError_t hipMemcpy2D(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h, hipMemcpyKind k)
 {
+    InStub in_stub;
     hipError_t e = hipSuccess;
     for (size_t y = 0; y < h && e == hipSuccess; ++y) e = copy((char *)d + y * dp, (const char *)s + y * sp, w, k);
     return e;
 }
 hipError_t hipMemset(void *d, int v, size_t n)
 {
+    InStub in_stub;
     std::lock_guard<std::recursive_mutex> l(g_mutex);
     if (room(g_device, d) < n) wrong("set of", d);
     return memset(d, v, n), hipSuccess;
 }
 hipError_t hipGetSymbolAddress(void **p, const void *)
 {
+    InStub in_stub;
     static char *mem = nullptr;
     std::lock_guard<std::recursive_mutex> l(g_mutex);
     if (!mem) {
@@ -233,29 +258,32 @@ hipError_t hipGetSymbolAddress(void **p, const void *)
 }
 
 // ------------------------------------------------------------------- device
-hipError_t hipGetDeviceCount(int *n) { return *n = 1, hipSuccess; }
-hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
-hipError_t hipSetDevice(int) { return hipSuccess; }
-hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) { return *v = 256, hipSuccess; }
+hipError_t hipGetDeviceCount(int *n) { InStub in_stub; return *n = 1, hipSuccess; }
+hipError_t hipGetDevice(int *d) { InStub in_stub; return *d = 0, hipSuccess; }
+hipError_t hipSetDevice(int) { InStub in_stub; return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) { InStub in_stub; return *v = 256, hipSuccess; }
 hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *p, int)
 {
+    InStub in_stub;
     memset(p, 0, sizeof *p);
     p->multiProcessorCount = 256;
     return hipSuccess;
 }
-hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, int, size_t) { return *n = 4, hipSuccess; }
+hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, int, size_t) { InStub in_stub; return *n = 4, hipSuccess; }
 const char *hipGetErrorString(hipError_t) { return "hip stub error"; }
 hipError_t hipGetLastError()
 {
+    InStub in_stub;
     const hipError_t e = t_last;
     t_last = hipSuccess;
     return e;
 }
 
 // ---------------------------------------------------------- streams, events
-hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return *s = (hipStream_t)made(g_streams, new Stream), hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { InStub in_stub; return *s = (hipStream_t)made(g_streams, new Stream), hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s)
 {
+    InStub in_stub;
     Stream *p = live<Stream>(g_streams, s, "stream");
     std::lock_guard<std::recursive_mutex> l(g_mutex);
     g_streams.erase(p);
@@ -264,22 +292,25 @@ hipError_t hipStreamDestroy(hipStream_t s)
 }
 hipError_t hipStreamSynchronize(hipStream_t s)
 {
+    InStub in_stub;
     if (s) live<Stream>(g_streams, s, "stream");
     return hipSuccess;
 }
-hipError_t hipStreamQuery(hipStream_t s) { return hipStreamSynchronize(s); }
+hipError_t hipStreamQuery(hipStream_t s) { InStub in_stub; return hipStreamSynchronize(s); }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned)
 {
+    InStub in_stub;
     Stream *p = live<Stream>(g_streams, s, "stream");
     Event *v = live<Event>(g_events, e, "event");
     std::lock_guard<std::recursive_mutex> l(g_mutex);
     if (v->captured_on && p != v->captured_on) g_joined[p] = v->captured_on;
     return hipSuccess;
 }
-hipError_t hipEventCreate(hipEvent_t *e) { return *e = (hipEvent_t)made(g_events, new Event), hipSuccess; }
-hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventCreate(hipEvent_t *e) { InStub in_stub; return *e = (hipEvent_t)made(g_events, new Event), hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { InStub in_stub; return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t e)
 {
+    InStub in_stub;
     Event *v = live<Event>(g_events, e, "event");
     std::lock_guard<std::recursive_mutex> l(g_mutex);
     g_events.erase(v);
@@ -288,6 +319,7 @@ hipError_t hipEventDestroy(hipEvent_t e)
 }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s)
 {
+    InStub in_stub;
     Event *v = live<Event>(g_events, e, "event");
     Stream *p = s ? live<Stream>(g_streams, s, "stream") : nullptr;
     std::lock_guard<std::recursive_mutex> l(g_mutex);
@@ -295,12 +327,13 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t s)
     v->captured_on = capture_of(p);
     return hipSuccess;
 }
-hipError_t hipEventSynchronize(hipEvent_t e) { return live<Event>(g_events, e, "event"), hipSuccess; }
-hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { return *ms = 1.f, hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t e) { InStub in_stub; return live<Event>(g_events, e, "event"), hipSuccess; }
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { InStub in_stub; return *ms = 1.f, hipSuccess; }
 
 // ------------------------------------------------------------------- graphs
 hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode)
 {
+    InStub in_stub;
     Stream *p = live<Stream>(g_streams, s, "stream");
     p->capturing = true;
     p->graph.clear();
@@ -308,6 +341,7 @@ hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode)
 }
 hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t *g)
 {
+    InStub in_stub;
     Stream *p = live<Stream>(g_streams, s, "stream");
     std::lock_guard<std::recursive_mutex> l(g_mutex);
     p->capturing = false;
@@ -317,11 +351,13 @@ hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t *g)
 }
 hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t g, hipGraphNode_t *, char *, size_t)
 {
+    InStub in_stub;
     *e = (hipGraphExec_t)made(g_execs, new Graph(*live<Graph>(g_graphs, g, "graph")));
     return hipSuccess;
 }
 hipError_t hipGraphDestroy(hipGraph_t g)
 {
+    InStub in_stub;
     Graph *p = live<Graph>(g_graphs, g, "graph");
     std::lock_guard<std::recursive_mutex> l(g_mutex);
     g_graphs.erase(p);
@@ -330,6 +366,7 @@ hipError_t hipGraphDestroy(hipGraph_t g)
 }
 hipError_t hipGraphExecDestroy(hipGraphExec_t e)
 {
+    InStub in_stub;
     Graph *p = live<Graph>(g_execs, e, "graph instance");
     std::lock_guard<std::recursive_mutex> l(g_mutex);
     g_execs.erase(p);
@@ -338,6 +375,7 @@ hipError_t hipGraphExecDestroy(hipGraphExec_t e)
 }
 hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t s)
 {
+    InStub in_stub;
     live<Stream>(g_streams, s, "stream");
     for (const Launch &l : *live<Graph>(g_execs, e, "graph instance"))
         if (g_callback) g_callback(l.name.c_str(), l.grid, l.block);
@@ -347,11 +385,13 @@ hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t s)
 // ----------------------------------------------------------------- launches
 hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t sh, hipStream_t s)
 {
+    InStub in_stub;
     t_config = { g, b, sh, s };
     return hipSuccess;
 }
 hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *sh, hipStream_t *s)
 {
+    InStub in_stub;
     *g = t_config.grid, *b = t_config.block, *sh = t_config.shared, *s = t_config.stream;
     return hipSuccess;
 }
@@ -370,6 +410,7 @@ static void read_out(void **args)
 }
 hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t, hipStream_t s)
 {
+    InStub in_stub;
     Stream *p = s ? live<Stream>(g_streams, s, "stream") : nullptr;
     const Launch l{ names().at(f), g.x, b.x };
     if (!g.x || !b.x) return ret(hipErrorInvalidConfiguration);
@@ -383,6 +424,7 @@ void **__hipRegisterFatBinary(const void *) { static void *m[1]; return m; }
 void __hipUnregisterFatBinary(void **) {}
 void __hipRegisterFunction(void **, const void *f, char *, const char *name, unsigned, void *, void *, void *, void *, int *)
 {
+    InStub in_stub;
     names()[f] = name;
 }
 void __hipRegisterVar(void **, void *, char *, const char *, int, size_t, int, int) {}

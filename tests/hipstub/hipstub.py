@@ -48,7 +48,8 @@ class Runtime:
 
     def __init__(self, lib):
         self.lib = lib
-        for name, res, args in (("stub_limit", None, [C.c_size_t]), ("stub_used", C.c_size_t, []),
+        for name, res, args in (("stub_fail_new", None, [C.c_long]), ("stub_fail_left", C.c_long, []),
+                                ("stub_limit", None, [C.c_size_t]), ("stub_used", C.c_size_t, []),
                                 ("stub_pinned", C.c_size_t, []), ("stub_mallocs", C.c_size_t, []),
                                 ("stub_pinned_of", C.c_void_p, [C.c_size_t, C.c_size_t]),
                                 ("layout_counters_size", C.c_size_t, []),
