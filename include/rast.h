@@ -203,6 +203,8 @@ int rast_resize(rast_renderer *r, uint32_t width, uint32_t height);
 int rast_mesh_create(rast_renderer *r, const rast_ivertex *verts, uint32_t num_verts,
                      const uint32_t *indices, uint32_t num_indices, int topology,
                      const float world[16], rast_mesh **out);
+/* Its device memory goes with the next frame of its renderer and of each view, or
+ * when an allocation needs it (debug reads of their last frames are refused then). */
 int rast_mesh_destroy(rast_mesh *m);
 /* CUDAMesh::GetWorld() (CCR/CUDAMesh.h:31). */
 int rast_mesh_set_world(rast_mesh *m, const float world[16]);
@@ -300,8 +302,9 @@ int rast_draw_texture(rast_renderer *r, const rast_texture *t, int mode, int str
 /* No reference counterpart (the reference sizes queues statically,
  * CCR/DEFINES.h:21-23, CCR/main.cpp:372-389): a per-tile MLP in -> H -> H -> 1
  * that predicts log(1 + queue length) from per-tile features (previous-frame
- * queue lengths and min depth, current projected-vertex density), trained on
- * the GPU from exact counts. */
+ * queue lengths and min depth, tile position), trained on the GPU from exact
+ * counts.  A model serves every renderer of its device that it is attached to;
+ * it and they, the one it was created on included, are destroyed in any order. */
 int rast_binmodel_create(rast_renderer *r, uint32_t hidden, uint32_t seed, rast_binmodel **out);
 int rast_binmodel_destroy(rast_binmodel *m);
 int rast_binmodel_num_features(void);
